@@ -3,12 +3,17 @@
 // fine -> coarse L2 projection that builds its training data, and the glue that turns a
 // coarse model's state into MLP inputs and the MLP outputs into a tendency correction.
 //
-// GEMMs: C[M,N] = op(A) op(B) over FP32 with FP32 accumulation, 64x64 output tiles staged
-// through LDS (16-wide k slabs), 256 work-items computing 4x4 outputs each.  The reductions
-// over the batch dimension (weight gradients) are split over blocks and summed in a fixed
-// order by a second kernel, so training is deterministic.
+// Networks whose hidden layers are at most 256 wide (and whose row tile fits 64 KiB of LDS) run
+// on two FP32 matrix-core kernels: k_mlp_rows takes 16 rows of the batch through the whole
+// network, forward and, for training, backward, with the activations in LDS and the weights
+// read from L2; k_mlp_weight_grad forms all weight and bias gradients (A^T D over the batch) in
+// one launch, split over the rows, and k_sum_splits adds the splits in a fixed order, so
+// training is deterministic.  Larger networks take layer-by-layer GEMMs: C[M,N] = op(A) op(B)
+// with 64x64 output tiles staged through LDS (16-wide k slabs), 256 work-items computing 4x4
+// outputs each, the reductions over the batch split and summed in the same way.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "closure.hpp"
@@ -20,9 +25,46 @@ namespace {
 
 constexpr int TM = 64, TN = 64, TK = 16;
 
-__device__ __forceinline__ float gelu_f(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
+// h = gelu(z) = z Phi(z) and d = gelu'(z) = Phi(z) + z phi(z), without branches (a call of erff
+// runs both of its branches over a wavefront).  With x = z / sqrt 2: Phi = (1 + erf x) / 2 below
+// |x| = 1, erf x = x + x Q(x^2); beyond, from erfc |x| = exp(-x^2) t P(t), t = 1 / (1 + 0.4 |x|)
+// (the form of Hastings, Approximations for Digital Computers, 1955), with the exponential that
+// phi needs too.  Q and P (degree 6) are least-squares fits, weighted towards the smallest
+// maximum: relative errors 1.6e-9 of erf and 2.4e-8 of erfc.  In FP32 against 64 bits over
+// |z| <= 8: h within 9.8e-8 (|z| + 0.1), rms 3.5e-8 for normal z; d within 1.4e-7, rms 2.6e-8 (the
+// formulas with a correctly rounded erff: 9.9e-8, 3.7e-8, 1.3e-7, 2.6e-8).
+__device__ __forceinline__ void gelu_pair(float z, float &h, float &d) {
+  const float x = z * 0.70710678118654752f, x2 = x * x, ax = fabsf(x);
+  float q = 7.72090352e-05f;
+  q = fmaf(q, x2, -0.000797249028f);
+  q = fmaf(q, x2, 0.00518434215f);
+  q = fmaf(q, x2, -0.0268518832f);
+  q = fmaf(q, x2, 0.11283543f);
+  q = fmaf(q, x2, -0.37612623f);
+  q = fmaf(q, x2, 0.128379166f);
+  const float lo = fmaf(0.5f, fmaf(x, q, x), 0.5f);
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.4f, ax, 1.f));
+  float p = -0.117370792f;
+  p = fmaf(p, t, 0.246633857f);
+  p = fmaf(p, t, 0.00491613708f);
+  p = fmaf(p, t, 0.214964211f);
+  p = fmaf(p, t, 0.198186055f);
+  p = fmaf(p, t, 0.226788446f);
+  p = fmaf(p, t, 0.225620806f);
+  const float e = expf(-0.5f * z * z), half = 0.5f * (p * t) * e;
+  const float phi = ax < 1.f ? lo : (z >= 0.f ? 1.f - half : half);
+  h = z * phi;
+  d = fmaf(z * e, 0.39894228040143268f, phi);
+}
+__device__ __forceinline__ float gelu_f(float z) {
+  float h, d;
+  gelu_pair(z, h, d);
+  return h;
+}
 __device__ __forceinline__ float gelu_grad_f(float z) {
-  return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * expf(-0.5f * z * z) * 0.39894228040143268f;
+  float h, d;
+  gelu_pair(z, h, d);
+  return d;
 }
 
 // C = op(A) * op(B) (+ bias[col]); op(A) is M x K, op(B) is K x N; lda/ldb are the row
@@ -93,6 +135,7 @@ __global__ void k_sum_splits(const float *__restrict__ parts, float *__restrict_
                              int accumulate) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     float s = 0.f;
+  #pragma unroll 8
     for (int k = 0; k < splits; k++) s += parts[(size_t)k * n + i];
     out[i] = accumulate ? out[i] + s : s;
   }
@@ -148,8 +191,9 @@ struct selfamd_mlp {
   float *params = nullptr, *grads = nullptr, *m1 = nullptr, *m2 = nullptr;  // packed W1 b1 W2 b2 W3 b3
   float *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Y = nullptr, *dY = nullptr;
   float *D2 = nullptr, *D1 = nullptr, *parts = nullptr, *lossParts = nullptr;
-  float *ones = nullptr;  // maxB ones: bias gradients are ones^T D through the split GEMM
+  float *ones = nullptr;  // maxB ones: bias gradients are ones^T D through the split GEMM (layer-by-layer path)
   int splitsMax = 64;
+  bool rows = false;  // the network runs on the row kernels (Z1, Z2 and ones are not allocated then)
   float *W1() { return params; }
   float *b1() { return params + (size_t)nIn * nH; }
   float *W2() { return b1() + nH; }
@@ -174,8 +218,500 @@ hipError_t gemm(const float *A, const float *B, float *C, float *Z, const float 
   return hipGetLastError();
 }
 
+// ------------------------------------------------------------------------------
+// Row kernels: 16 rows of the batch through the whole network on the FP32 matrix cores
+// ------------------------------------------------------------------------------
+constexpr int kRowTile = 16, kRowThreads = 512, kRowWaves = kRowThreads / 64;
+constexpr int kRowMaxHidden = 256, kRowMaxOut = 256, kRowLds = 56 * 1024;  // 64 KiB with the static arrays
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+// kRowsForward: Y = net(X).  kRowsLoss: forward, dY = 2 (Y - T) / count, backward.
+// kRowsBackward: forward, backward from the cotangent T.  kRowsClosure: features of the state,
+// forward, FP64 correction and its mass integral.
+enum RowsMode { kRowsForward, kRowsLoss, kRowsBackward, kRowsClosure };
+
+struct RowsArgs {
+  int nIn, nH, nO, B;
+  int ldX, ldH, ldO;  // LDS row strides
+  const float *W1, *b1, *W2, *b2, *W3, *b3;
+  const float *X, *T;
+  float *Y, *H1, *H2, *D1, *D2, *dY, *dX, *lossParts;
+  float count;
+  const double *S, *geom, *qW;
+  const float *inMean, *inScale, *outMean, *outScale;
+  double *corr, *massParts;
+  int P, nVar, massVar;
+};
+
+// Columns of an operand in LDS: a multiple of 64 (zero beyond the data), rows an odd multiple of
+// 4 floats apart, so that the 16 rows of a 16-byte read do not conflict in the banks.
+inline __host__ __device__ int pad16(int n) { return (n + 15) & ~15; }
+inline __host__ __device__ int pad64(int n) { return (n + 63) & ~63; }
+inline int rows_ld(int n) { return pad64(n) + 4; }
+inline size_t rows_lds(int nIn, int nH, int nO) {
+  return sizeof(float) * kRowTile * ((size_t)rows_ld(nIn) + 2 * rows_ld(nH) + rows_ld(nO));
+}
+inline bool rows_fit(int nIn, int nH, int nO) {
+  return nH <= kRowMaxHidden && nO <= kRowMaxOut && rows_lds(nIn, nH, nO) <= kRowLds;
+}
+
+// element `at` of a uniform base (scalar base, 32-bit vector offset: operands are below 4 GiB)
+template <class T>
+__device__ __forceinline__ T load_at(const float *base, unsigned at) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + 4u * at);
+}
+// The weight operand of one layer: weight (k, n), k < K, n < Nc, at W[k ldw + n], or with TRANS at
+// W[n ldw + k].  VEC: 16-byte reads along k (K a multiple of 4, rows 16-byte aligned).
+struct RowsOperand {
+  const float *W;
+  int ldw, K, Nc;
+};
+// 64 reduction indices of this lane's column n, as the matrix instruction takes them: in
+// instruction 4 t + q, index k0 + 16 t + 4 g + q (lane group g = lane / 16).  The row operand is
+// read with the same index order, so both come in pieces of four consecutive indices.  Indices
+// past K and columns past Nc read a weight in range instead, without a select that would wait
+// for the load: past K the rows are zero in LDS, past Nc the column is discarded.
+template <bool TRANS, bool VEC>
+__device__ __forceinline__ void rows_load(const RowsOperand &o, int n, int g, int k0, float (&b)[16]) {
+  const unsigned nn = min(n, o.Nc - 1), k = k0 + 4 * g;
+  // 32-bit element offsets from the uniform base: one addition and one minimum per load
+  const unsigned at = TRANS ? nn * o.ldw + k : k * o.ldw + nn, step = TRANS ? 1 : o.ldw;
+  const unsigned last = TRANS ? nn * o.ldw + o.K - 1 : (o.K - 1) * o.ldw + nn;
+  if constexpr (TRANS && VEC) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const f32x4 v = load_at<f32x4>(o.W, min(at + 16 * t, last - 3));
+#pragma unroll
+      for (int q = 0; q < 4; q++) b[4 * t + q] = v[q];
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) b[4 * t + q] = load_at<float>(o.W, min(at + (16 * t + q) * step, last));
+  }
+}
+__device__ __forceinline__ f32x4 rows_mul(const float *rows, const float (&b)[16], f32x4 acc) {
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const f32x4 a = *reinterpret_cast<const f32x4 *>(rows + 16 * t);
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], b[4 * t + q], acc, 0, 0, 0);
+  }
+  return acc;
+}
+// One 16 x 16 tile of rows(LDS) * weights: `b` holds the tile's first 64 reduction indices on
+// entry, and the next 64 are loaded while the current ones are multiplied; during the last ones
+// the first 64 indices of whatever this wavefront multiplies next are loaded into `next`, which
+// stay in flight through the epilogue and the barrier.
+template <bool TRANS, bool VEC, class Prefetch>
+__device__ __forceinline__ f32x4 rows_tile(const float *rows, int ld, const RowsOperand &o, int n, int lane,
+                                           float (&b)[16], Prefetch prefetch) {
+  const float *mine = rows + (lane & 15) * ld + 4 * (lane >> 4);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int k0 = 0;
+  for (; k0 + 64 < o.K; k0 += 64) {
+    float t[16];
+    rows_load<TRANS, VEC>(o, n, lane >> 4, k0 + 64, t);
+    acc = rows_mul(mine + k0, b, acc);
+#pragma unroll
+    for (int q = 0; q < 16; q++) b[q] = t[q];
+  }
+  prefetch();
+  return rows_mul(mine + k0, b, acc);
+}
+
+// What bounds it: latency.  The configured closure (51 -> 128 -> 128 -> 48) on 4096 rows is 0.24
+// GFLOP, 1.6 us at the matrix cores' FP32 rate; a block has its 16 rows' layers in a chain of
+// barriers, and 4096 rows are one block per CU.  So a wavefront keeps the weights of its columns
+// in registers one piece ahead, across the layers, and one launch does the whole network: TILES
+// 16-column tiles of the hidden layers per wavefront (1 up to 128 hidden units, 2 up to 256).
+// Element (row, column) of a tile: lane group g holds rows 4 g .. 4 g + 3 of column lane % 16, the
+// same in the forward and backward passes, so gelu'(z) stays in registers.
+// Measured at that size, per launch: closure evaluation 9.5 us (32.8 us with 32 rows per block,
+// FMA lanes and the weights loaded inside the reduction loop), forward + loss + backward
+// 16.7 us and all weight gradients 7.9 us (with k_sum_splits, 4 us, about 29 us per training
+// step where layer-by-layer GEMMs took 26 launches and 390 us).
+template <int MODE, int TILES, bool VEC>
+__global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
+  extern __shared__ __align__(16) float rowsLds[];
+  __shared__ double sRed[kRowTile];
+  // closure: output scale and mean, element J, and w_i w_j per node of the mass variable (0 for the
+  // other outputs)
+  __shared__ float sScale[MODE == kRowsClosure ? kRowMaxOut : 1], sMean[MODE == kRowsClosure ? kRowMaxOut : 1];
+  __shared__ double sWeight[MODE == kRowsClosure ? kRowMaxOut : 1], sJ[MODE == kRowsClosure ? kRowTile : 1];
+  float *sX = rowsLds, *sH1 = sX + kRowTile * a.ldX, *sH2 = sH1 + kRowTile * a.ldH, *sO = sH2 + kRowTile * a.ldH;
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches on it
+  const int row0 = blockIdx.x * kRowTile;
+  constexpr bool BACK = MODE == kRowsLoss || MODE == kRowsBackward;
+  const RowsOperand w1{a.W1, a.nH, a.nIn, a.nH}, w2{a.W2, a.nH, a.nH, a.nH}, w3{a.W3, a.nO, a.nH, a.nO};
+  const RowsOperand t3{a.W3, a.nO, a.nO, a.nH}, t2{a.W2, a.nH, a.nH, a.nH}, t1{a.W1, a.nH, a.nH, a.nIn};
+  const int n0 = wave * 16 + r;  // this lane's column of the wavefront's first tile of a layer
+  float b[2][16];                // the weights in flight; a layer's first piece is in b[0]
+  rows_load<false, VEC>(w1, n0, g, 0, b[0]);
+  float bias1[TILES], bias2[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; t++) {
+    const int n = min(n0 + 128 * t, a.nH - 1);
+    bias1[t] = a.b1[n];
+    bias2[t] = a.b2[n];
+  }
+  const float bias3 = a.b3[min(n0, a.nO - 1)];
+  const int H16 = pad16(a.nH), O16 = pad16(a.nO);
+  // input rows and the zero columns of the other operands: 32 work-items per row
+  {
+    const int row = tid >> 5, c = tid & 31, KX = pad64(a.nIn), KH = pad64(a.nH), KO = pad64(a.nO);
+    const bool ok = row0 + row < a.B;
+    const size_t e = (size_t)(ok ? row0 + row : 0);
+    if constexpr (MODE == kRowsClosure) {
+      for (int k = tid; k < a.nO; k += kRowThreads) {
+        sScale[k] = a.outScale[k];
+        sMean[k] = a.outMean[k];
+        const int node = k - a.massVar * a.P * a.P;
+        sWeight[k] = node >= 0 && node < a.P * a.P ? a.qW[node % a.P] * a.qW[node / a.P] : 0.0;
+      }
+      if (c == 0) sJ[row] = ok ? a.geom[e * kGeomStride + 4] : 0.0;
+    }
+    // two values at a time, loaded before either is used: the launch starts with these loads'
+    // round trips to memory (positions past the row read one in it)
+    const int nS = a.nVar * a.P * a.P;
+    for (int k = c; k < KX; k += 64) {
+      double raw[2];
+      float mu[2], sd[2], x[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int kk = min(k + 32 * j, a.nIn - 1);
+        if constexpr (MODE == kRowsClosure) {
+          const double *gr = a.geom + e * kGeomStride;
+          raw[j] = *(kk < nS ? a.S + e * nS + kk : kk == nS ? gr + 4 : kk == nS + 1 ? gr : gr + 3);
+          mu[j] = a.inMean[kk];
+          sd[j] = a.inScale[kk];
+        } else {
+          x[j] = a.X[e * a.nIn + kk];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        if constexpr (MODE == kRowsClosure) x[j] = (float)((raw[j] - (double)mu[j]) / (double)sd[j]);
+        sX[row * a.ldX + k + 32 * j] = ok && k + 32 * j < a.nIn ? x[j] : 0.f;
+      }
+    }
+    for (int k = H16 + c; k < KH; k += 32) sH1[row * a.ldH + k] = sH2[row * a.ldH + k] = 0.f;
+    for (int k = O16 + c; k < KO; k += 32) sO[row * a.ldO + k] = 0.f;
+  }
+  __syncthreads();
+
+  float gp1[TILES][4], gp2[TILES][4];
+  // the tiles of one hidden-width layer of this wavefront, b[0] holding the first one's first
+  // piece: epilogue(t, n, acc) takes each tile; `after` loads the next layer's first piece
+  auto layer = [&](auto trans, const float *in, int ld, const RowsOperand &o, auto epilogue, auto after) {
+    constexpr bool TR = decltype(trans)::value;
+    if (wave * 16 >= H16) {
+      after(b[0]);
+      return;
+    }
+    const bool two = TILES > 1 && (wave + kRowWaves) * 16 < H16;
+    if (!two) {
+      const f32x4 acc = rows_tile<TR, VEC>(in, ld, o, n0, lane, b[0], [&] { after(b[1]); });
+      epilogue(std::integral_constant<int, 0>{}, n0, acc);
+    } else {
+      const f32x4 acc = rows_tile<TR, VEC>(in, ld, o, n0, lane, b[0], [&] { rows_load<TR, VEC>(o, n0 + 128, g, 0, b[1]); });
+      epilogue(std::integral_constant<int, 0>{}, n0, acc);
+      float cur[16];
+#pragma unroll
+      for (int q = 0; q < 16; q++) cur[q] = b[1][q];
+      const f32x4 acc1 = rows_tile<TR, VEC>(in, ld, o, n0 + 128, lane, cur, [&] { after(b[1]); });
+      epilogue(std::integral_constant<int, TILES - 1>{}, n0 + 128, acc1);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) b[0][q] = b[1][q];
+  };
+  // out = gelu(in W + bias), gelu' kept, the activations also to memory for the weight gradients
+  auto hidden = [&](const float *in, int ld, const RowsOperand &o, const float (&bias)[TILES], float *out, float *mem,
+                    float (&gp)[TILES][4], auto after) {
+    layer(std::false_type{}, in, ld, o, [&](auto t, int n, f32x4 acc) {
+      const bool ok = n < a.nH;
+      const float bn = bias[decltype(t)::value];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float z = acc[i] + bn;
+        float h, d;
+        gelu_pair(z, h, d);
+        out[(4 * g + i) * a.ldH + n] = h = ok ? h : 0.f;
+        if constexpr (BACK) {
+          gp[decltype(t)::value][i] = d;
+          if (ok && row0 + 4 * g + i < a.B) mem[(size_t)(row0 + 4 * g + i) * a.nH + n] = h;
+        }
+      }
+    }, after);
+  };
+  hidden(sX, a.ldX, w1, bias1, sH1, a.H1, gp1, [&](float (&x)[16]) { rows_load<false, VEC>(w2, n0, g, 0, x); });
+  __syncthreads();
+  hidden(sH1, a.ldH, w2, bias2, sH2, a.H2, gp2, [&](float (&x)[16]) {
+    if constexpr (MODE == kRowsBackward) rows_load<true, VEC>(t3, n0, g, 0, x);
+    else rows_load<false, VEC>(w3, n0, g, 0, x);
+  });
+  if constexpr (MODE != kRowsBackward) __syncthreads();
+
+  // output layer
+  float loss = 0.f;
+  if constexpr (MODE == kRowsBackward) {
+    // the cotangent is given: the output itself is not needed
+    const int row = tid >> 5;
+    const bool ok = row0 + row < a.B;
+    for (int k = tid & 31; k < O16; k += 32)
+      sO[row * a.ldO + k] = ok && k < a.nO ? a.T[(size_t)(row0 + row) * a.nO + k] : 0.f;
+  } else {
+    for (int ct = wave; ct * 16 < O16; ct += kRowWaves) {
+      const int n = ct * 16 + r;
+      const bool nok = n < a.nO;
+      float tv[4];
+      if constexpr (MODE == kRowsLoss) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) tv[i] = a.T[(size_t)min(row0 + 4 * g + i, a.B - 1) * a.nO + (nok ? n : 0)];
+      }
+      if (ct != wave) rows_load<false, VEC>(w3, n, g, 0, b[0]);
+      const f32x4 acc = rows_tile<false, VEC>(sH2, a.ldH, w3, n, lane, b[0], [] {});
+      const float bn = ct == wave ? bias3 : a.b3[nok ? n : 0];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = row0 + 4 * g + i;
+        const bool ok = nok && row < a.B;
+        float y = nok ? acc[i] + bn : 0.f;
+        if constexpr (MODE == kRowsForward) {
+          if (ok) a.Y[(size_t)row * a.nO + n] = y;
+        } else {
+          if constexpr (MODE == kRowsLoss) {
+            const float d = ok ? y - tv[i] : 0.f;
+            loss += d * d;
+            y = 2.f * d / a.count;
+            if (ok) a.dY[(size_t)row * a.nO + n] = y;
+          }
+          sO[(4 * g + i) * a.ldO + n] = y;
+        }
+      }
+    }
+    if constexpr (MODE == kRowsLoss) rows_load<true, VEC>(t3, n0, g, 0, b[0]);
+  }
+  if constexpr (MODE == kRowsForward) return;
+  if constexpr (MODE == kRowsClosure) {
+    __syncthreads();
+    const int row = tid >> 5;
+    const size_t e = (size_t)row0 + row;
+    double m = 0.0;
+    for (int k = tid & 31; k < a.nO; k += 32) {
+      const double c = (double)sO[row * a.ldO + k] * (double)sScale[k] + (double)sMean[k];
+      if (e < (size_t)a.B) a.corr[e * a.nO + k] = c;
+      m += sWeight[k] * c;
+    }
+    for (int off = 16; off > 0; off >>= 1) m += __shfl_xor(m, off, 32);
+    if ((tid & 31) == 0) sRed[row] = sJ[row] * m;
+    __syncthreads();
+    if (wave == 0) {
+      double s = sRed[lane & 15];
+      for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
+      if (tid == 0) a.massParts[blockIdx.x] = s;
+    }
+  }
+  if constexpr (BACK) {
+    // D2 = (dY W3^T) gelu'(z2), D1 = (D2 W2^T) gelu'(z1), dX = D1 W1^T
+    if constexpr (MODE == kRowsLoss) {
+      for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+      if (lane == 0) sRed[wave] = loss;
+    }
+    __syncthreads();
+    if constexpr (MODE == kRowsLoss) {
+      if (tid == 0) {
+        double s = 0.0;
+        for (int k = 0; k < kRowWaves; k++) s += sRed[k];
+        a.lossParts[blockIdx.x] = (float)s;
+      }
+    }
+    auto back = [&](const float *in, int ld, const RowsOperand &o, float *out, float *mem, const float (&gp)[TILES][4],
+                    auto after) {
+      layer(std::true_type{}, in, ld, o, [&](auto t, int n, f32x4 acc) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float d = n < a.nH ? acc[i] * gp[decltype(t)::value][i] : 0.f;
+          out[(4 * g + i) * a.ldH + n] = d;
+          if (n < a.nH && row0 + 4 * g + i < a.B) mem[(size_t)(row0 + 4 * g + i) * a.nH + n] = d;
+        }
+      }, after);
+    };
+    back(sO, a.ldO, t3, sH2, a.D2, gp2, [&](float (&x)[16]) { rows_load<true, VEC>(t2, n0, g, 0, x); });
+    __syncthreads();
+    back(sH2, a.ldH, t2, sH1, a.D1, gp1, [&](float (&x)[16]) {
+      if constexpr (MODE == kRowsBackward) rows_load<true, VEC>(t1, n0, g, 0, x);
+    });
+    if (MODE == kRowsLoss || !a.dX) return;
+    __syncthreads();
+    for (int ct = wave; ct * 16 < a.nIn; ct += kRowWaves) {
+      const int n = ct * 16 + r;
+      if (ct != wave) rows_load<true, VEC>(t1, n, g, 0, b[0]);
+      const f32x4 acc = rows_tile<true, VEC>(sH1, a.ldH, t1, n, lane, b[0], [] {});
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (n < a.nIn && row0 + 4 * g + i < a.B) a.dX[(size_t)(row0 + 4 * g + i) * a.nIn + n] = acc[i];
+    }
+  }
+}
+
+// All weight and bias gradients of one split of the rows: gW = A^T D and gb = column sums of D for
+// (A, D) = (X, D1), (H1, D2), (H2, dY), packed like the parameters at parts + split * nParams.  A
+// wavefront forms a 32 x 32 tile of one gW, reading both operands straight from L2 (16
+// consecutive floats per row and lane group); the tiles of the first 32 rows of a gW also sum D.
+struct GradArgs {
+  const float *A[3], *D[3];
+  int M[3], N[3];
+  size_t off[3];      // of the weights in the packed gradients; the bias follows them
+  int tilesN[3], first[4];  // column tiles of each product; its first tile, and the total
+  float *parts;
+  size_t nParams;
+  int B, rowsPerSplit;
+};
+__global__ void __launch_bounds__(256) k_mlp_weight_grad(const GradArgs a) {
+  const int tile = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (tile >= a.first[3]) return;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int p = tile >= a.first[2] ? 2 : tile >= a.first[1] ? 1 : 0;
+  const float *__restrict__ A = a.A[p], *__restrict__ D = a.D[p];
+  const int M = a.M[p], N = a.N[p], local = tile - a.first[p];
+  const int tm = local / a.tilesN[p], m0 = tm * 32, n0 = (local - tm * a.tilesN[p]) * 32;
+  const int k0 = blockIdx.x * a.rowsPerSplit, k1 = min(a.B, k0 + a.rowsPerSplit);
+  // columns past M and N read the last one; what they give is not stored
+  const bool nok[2] = {n0 + r < N, n0 + 16 + r < N};
+  const unsigned mi[2] = {(unsigned)min(m0 + r, M - 1), (unsigned)min(m0 + 16 + r, M - 1)};
+  const unsigned ni[2] = {(unsigned)min(n0 + r, N - 1), (unsigned)min(n0 + 16 + r, N - 1)};
+  // this split's rows; rows past its end read its last one
+  const float *As = A + (size_t)k0 * M, *Ds = D + (size_t)k0 * N;
+  const unsigned rows = k1 - k0;
+  f32x4 acc[2][2] = {};
+  float bias[2] = {0.f, 0.f};
+  constexpr int U = 16;
+  auto load = [&](int k, float (&av)[U][2], float (&dv)[U][2]) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const unsigned row = min((unsigned)(k - k0 + 4 * u + g), rows - 1);
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        av[u][q] = load_at<float>(As, row * M + mi[q]);
+        dv[u][q] = load_at<float>(Ds, row * N + ni[q]);
+      }
+    }
+  };
+  auto multiply = [&](int k, bool tail, float (&av)[U][2], float (&dv)[U][2]) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        if (tail && k + 4 * u + g >= k1) dv[u][q] = av[u][q] = 0.f;
+        bias[q] += dv[u][q];
+      }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) acc[s][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u][s], dv[u][q], acc[s][q], 0, 0, 0);
+  };
+  // 64 rows at a time, the next 64 in flight while the current ones are multiplied
+  float av[U][2], dv[U][2];
+  load(k0, av, dv);
+  int k = k0;
+  for (; k + 4 * U < k1; k += 4 * U) {
+    float an[U][2], dn[U][2];
+    load(k + 4 * U, an, dn);
+    multiply(k, false, av, dv);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) { av[u][q] = an[u][q]; dv[u][q] = dn[u][q]; }
+  }
+  multiply(k, true, av, dv);
+  float *out = a.parts + (size_t)blockIdx.x * a.nParams + a.off[p];
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int m = m0 + 16 * s + 4 * g + i;
+        if (m < M && nok[q]) out[(size_t)m * N + ni[q]] = acc[s][q][i];
+      }
+  if (tm == 0) {
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      float s = bias[q];
+      s += __shfl_xor(s, 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      if (g == 0 && nok[q]) out[(size_t)M * N + ni[q]] = s;
+    }
+  }
+}
+
+RowsArgs rows_args(selfamd_mlp *m, const float *X, int B) {
+  RowsArgs a{};
+  a.nIn = m->nIn; a.nH = m->nH; a.nO = m->nOut; a.B = B;
+  a.ldX = rows_ld(a.nIn); a.ldH = rows_ld(a.nH); a.ldO = rows_ld(a.nO);
+  a.W1 = m->W1(); a.b1 = m->b1(); a.W2 = m->W2(); a.b2 = m->b2(); a.W3 = m->W3(); a.b3 = m->b3();
+  a.X = X;
+  a.H1 = m->H1; a.H2 = m->H2; a.D1 = m->D1; a.D2 = m->D2;
+  return a;
+}
+
+template <int MODE>
+hipError_t launch_rows(const RowsArgs &a, hipStream_t st) {
+  const unsigned blocks = (unsigned)((a.B + kRowTile - 1) / kRowTile);
+  const size_t lds = rows_lds(a.nIn, a.nH, a.nO);
+  // the transposed weights of the backward pass are read 16 bytes at a time where every row of
+  // W1, W2 and W3 is 16-byte aligned
+  const bool back = MODE == kRowsLoss || MODE == kRowsBackward;
+  const bool vec = back && a.nH % 4 == 0 && a.nO % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(a.W1) | reinterpret_cast<uintptr_t>(a.W2) |
+                     reinterpret_cast<uintptr_t>(a.W3)) & 15) == 0;
+  const bool one = a.nH <= 16 * kRowWaves;
+  if (one && !vec) hipLaunchKernelGGL((k_mlp_rows<MODE, 1, false>), blocks, kRowThreads, lds, st, a);
+  else if (!vec) hipLaunchKernelGGL((k_mlp_rows<MODE, 2, false>), blocks, kRowThreads, lds, st, a);
+  else if constexpr (MODE == kRowsLoss || MODE == kRowsBackward) {
+    if (one) hipLaunchKernelGGL((k_mlp_rows<MODE, 1, true>), blocks, kRowThreads, lds, st, a);
+    else hipLaunchKernelGGL((k_mlp_rows<MODE, 2, true>), blocks, kRowThreads, lds, st, a);
+  }
+  return hipGetLastError();
+}
+
+// Parameter gradients from the activations and cotangents that k_mlp_rows left in memory.  At
+// most 64 splits of at least 128 rows: all of a split's loads are then in flight at once, and
+// with 64 rows the sum over twice the splits costs more than it saves (9.5 + 4.7 us against
+// 7.9 + 3.6 us at 4096 rows).
+hipError_t weight_grads_rows(selfamd_mlp *m, const float *X, const float *dY, int B, int accumulate, hipStream_t st) {
+  GradArgs a{};
+  const float *A[3] = {X, m->H1, m->H2}, *D[3] = {m->D1, m->D2, dY};
+  const int M[3] = {m->nIn, m->nH, m->nH}, N[3] = {m->nH, m->nH, m->nOut};
+  const size_t off[3] = {0, m->off_W2(), m->off_W3()};
+  for (int p = 0; p < 3; p++) {
+    a.A[p] = A[p]; a.D[p] = D[p]; a.M[p] = M[p]; a.N[p] = N[p]; a.off[p] = off[p];
+    a.tilesN[p] = (N[p] + 31) / 32;
+    a.first[p + 1] = a.first[p] + a.tilesN[p] * ((M[p] + 31) / 32);
+  }
+  a.parts = m->parts; a.nParams = m->nParams; a.B = B;
+  const int perSplit = (B + m->splitsMax - 1) / m->splitsMax;
+  a.rowsPerSplit = std::max(128, (perSplit + 31) / 32 * 32);
+  const int splits = (B + a.rowsPerSplit - 1) / a.rowsPerSplit, n = (int)m->nParams;
+  hipLaunchKernelGGL(k_mlp_weight_grad, dim3(splits, (a.first[3] + 3) / 4), 256, 0, st, a);
+  hipError_t e = hipGetLastError();
+  if (e) return e;
+  hipLaunchKernelGGL(k_sum_splits, (n + 255) / 256, 256, 0, st, m->parts, m->grads, n, splits, accumulate);
+  return hipGetLastError();
+}
+
 hipError_t forward_impl(selfamd_mlp *m, const float *X, float *Y, int B, hipStream_t st) {
   hipError_t e;
+  if (m->rows) {
+    RowsArgs a = rows_args(m, X, B);
+    a.Y = Y;
+    return launch_rows<kRowsForward>(a, st);
+  }
   if ((e = gemm<false, false, 2>(X, m->W1(), m->H1, m->Z1, m->b1(), B, m->nH, m->nIn, m->nIn, m->nH, 1, st))) return e;
   if ((e = gemm<false, false, 2>(m->H1, m->W2(), m->H2, m->Z2, m->b2(), B, m->nH, m->nH, m->nH, m->nH, 1, st))) return e;
   return gemm<false, false, 1>(m->H2, m->W3(), Y, nullptr, m->b3(), B, m->nOut, m->nH, m->nH, m->nOut, 1, st);
@@ -194,10 +730,11 @@ hipError_t weight_grad(selfamd_mlp *m, const float *A, const float *D, float *gW
   return hipGetLastError();
 }
 
-// Backward pass from the output cotangent dY (overwritten) through the activations that the
-// last forward_impl of the same rows left in Z1, H1, Z2, H2: parameter gradients written to (or,
-// with accumulate, added to) m->grads, and the input cotangent dX = D1 W1^T when dX is given.
-hipError_t backward_impl(selfamd_mlp *m, const float *X, float *dY, int B, int accumulate, float *dX,
+// Layer-by-layer backward pass from the output cotangent dY (overwritten) through the
+// activations that the last forward_impl of the same rows left in Z1, H1, Z2, H2: parameter
+// gradients written to (or, with accumulate, added to) m->grads, and the input cotangent
+// dX = D1 W1^T when dX is given.
+hipError_t backward_layers(selfamd_mlp *m, const float *X, float *dY, int B, int accumulate, float *dX,
                          hipStream_t st) {
   const int H = m->nH, nO = m->nOut;
   float *g = m->grads;
@@ -221,6 +758,22 @@ hipError_t backward_impl(selfamd_mlp *m, const float *X, float *dY, int B, int a
   return hipGetLastError();
 }
 
+// Forward pass of X and backward pass from the output cotangent dY: parameter gradients written
+// to (or, with accumulate, added to) m->grads, and the input cotangent when dX is given.
+hipError_t backward_impl(selfamd_mlp *m, const float *X, const float *dY, int B, int accumulate, float *dX,
+                         hipStream_t st) {
+  hipError_t e;
+  if (m->rows) {
+    RowsArgs a = rows_args(m, X, B);
+    a.T = dY; a.dX = dX;
+    if ((e = launch_rows<kRowsBackward>(a, st))) return e;
+    return weight_grads_rows(m, X, dY, B, accumulate, st);
+  }
+  if ((e = forward_impl(m, X, m->Y, B, st))) return e;
+  if ((e = hipMemcpyAsync(m->dY, dY, sizeof(float) * (size_t)B * m->nOut, hipMemcpyDeviceToDevice, st))) return e;
+  return backward_layers(m, X, m->dY, B, accumulate, dX, st);
+}
+
 }  // namespace
 
 extern "C" {
@@ -232,20 +785,24 @@ int selfamd_mlp_create(selfamd_mlp **out, int nIn, int nHidden, int nOut, int ma
   m->nIn = nIn; m->nH = nHidden; m->nOut = nOut; m->maxB = maxBatch;
   m->nParams = (size_t)nIn * nHidden + nHidden + (size_t)nHidden * nHidden + nHidden + (size_t)nHidden * nOut + nOut;
   const size_t B = maxBatch, H = nHidden;
-  const size_t maxW = std::max({(size_t)nIn * H, H * H, H * (size_t)nOut});
+  m->rows = rows_fit(nIn, nHidden, nOut);
+  const size_t lossBlocks = std::max<size_t>(1024, (B + kRowTile - 1) / kRowTile);
   float **bufs[] = {&m->params, &m->grads, &m->m1, &m->m2};
   bool ok = true;
   for (float **b : bufs) ok = ok && hipMalloc(b, 4 * m->nParams) == hipSuccess;
-  ok = ok && hipMalloc(&m->Z1, 4 * B * H) == hipSuccess && hipMalloc(&m->H1, 4 * B * H) == hipSuccess &&
-       hipMalloc(&m->Z2, 4 * B * H) == hipSuccess && hipMalloc(&m->H2, 4 * B * H) == hipSuccess &&
+  ok = ok && hipMalloc(&m->H1, 4 * B * H) == hipSuccess && hipMalloc(&m->H2, 4 * B * H) == hipSuccess &&
        hipMalloc(&m->Y, 4 * B * nOut) == hipSuccess && hipMalloc(&m->dY, 4 * B * nOut) == hipSuccess &&
        hipMalloc(&m->D2, 4 * B * H) == hipSuccess && hipMalloc(&m->D1, 4 * B * H) == hipSuccess &&
-       hipMalloc(&m->parts, 4 * maxW * m->splitsMax) == hipSuccess &&
-       hipMalloc(&m->lossParts, 4 * 1024) == hipSuccess && hipMalloc(&m->ones, 4 * B) == hipSuccess;
+       hipMalloc(&m->parts, 4 * m->nParams * m->splitsMax) == hipSuccess &&
+       hipMalloc(&m->lossParts, 4 * lossBlocks) == hipSuccess;
+  if (!m->rows)
+    ok = ok && hipMalloc(&m->Z1, 4 * B * H) == hipSuccess && hipMalloc(&m->Z2, 4 * B * H) == hipSuccess &&
+         hipMalloc(&m->ones, 4 * B) == hipSuccess;
   if (ok) ok = hipMemset(m->m1, 0, 4 * m->nParams) == hipSuccess && hipMemset(m->m2, 0, 4 * m->nParams) == hipSuccess &&
                hipMemset(m->params, 0, 4 * m->nParams) == hipSuccess;
   if (ok) {
-    hipLaunchKernelGGL(k_fill, (unsigned)std::min<size_t>((B + 255) / 256, 4096), 256, 0, nullptr, m->ones, 1.0f, B);
+    if (m->ones)
+      hipLaunchKernelGGL(k_fill, (unsigned)std::min<size_t>((B + 255) / 256, 4096), 256, 0, nullptr, m->ones, 1.0f, B);
     ok = hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess;
   }
   if (!ok) {
@@ -305,14 +862,21 @@ int selfamd_mlp_forward(selfamd_mlp *m, const float *X, float *Y, int B, void *s
 int selfamd_mlp_loss_grad(selfamd_mlp *m, const float *X, const float *T, int B, float *loss, void *stream) {
   SELFAMD_REQUIRE(m && X && T && B >= 1 && B <= m->maxB, "mlp_loss_grad: bad arguments");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int H = m->nH, nO = m->nOut;
-  SELFAMD_HIP(forward_impl(m, X, m->Y, B, st));
-  const size_t n = (size_t)B * nO;
-  int blocks = (int)std::min<size_t>((n + 255) / 256, 1024);
-  hipLaunchKernelGGL(k_mse, blocks, 256, 0, st, m->Y, T, m->dY, m->lossParts, n);
-  SELFAMD_HIP(hipGetLastError());
-  (void)H;
-  SELFAMD_HIP(backward_impl(m, X, m->dY, B, 0, nullptr, st));
+  const size_t n = (size_t)B * m->nOut;
+  int blocks;
+  if (m->rows) {
+    RowsArgs a = rows_args(m, X, B);
+    a.T = T; a.dY = m->dY; a.lossParts = m->lossParts; a.count = (float)n;
+    blocks = (B + kRowTile - 1) / kRowTile;
+    SELFAMD_HIP(launch_rows<kRowsLoss>(a, st));
+    SELFAMD_HIP(weight_grads_rows(m, X, m->dY, B, 0, st));
+  } else {
+    SELFAMD_HIP(forward_impl(m, X, m->Y, B, st));
+    blocks = (int)std::min<size_t>((n + 255) / 256, 1024);
+    hipLaunchKernelGGL(k_mse, blocks, 256, 0, st, m->Y, T, m->dY, m->lossParts, n);
+    SELFAMD_HIP(hipGetLastError());
+    SELFAMD_HIP(backward_layers(m, X, m->dY, B, 0, nullptr, st));
+  }
   if (loss) {
     std::vector<float> parts(blocks);
     SELFAMD_HIP(hipMemcpyAsync(parts.data(), m->lossParts, 4 * blocks, hipMemcpyDeviceToHost, st));
@@ -329,9 +893,7 @@ int selfamd_mlp_backward(selfamd_mlp *m, const float *X, const float *dY, int B,
   SELFAMD_REQUIRE(m && X && dY && B >= 1 && B <= m->maxB, "mlp_backward: bad arguments (B=%d, max %d)", B,
                   m ? m->maxB : 0);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  SELFAMD_HIP(forward_impl(m, X, m->Y, B, st));
-  SELFAMD_HIP(hipMemcpyAsync(m->dY, dY, sizeof(float) * (size_t)B * m->nOut, hipMemcpyDeviceToDevice, st));
-  SELFAMD_HIP(backward_impl(m, X, m->dY, B, accumulate, dX, st));
+  SELFAMD_HIP(backward_impl(m, X, dY, B, accumulate, dX, st));
   return kOk;
 }
 
@@ -455,111 +1017,6 @@ __global__ void __launch_bounds__(256) k_closure_shift(const double *__restrict_
   if (threadIdx.x == 0) shift[0] = red[0] * invArea;
 }
 
-// The whole closure for a tile of 32 elements in one block: features -> 3 layers -> FP64
-// correction and per-element mass integrals.  Accumulation orders and epilogues are those of
-// k_gemm / k_closure_features / k_closure_correct (each output sums k = 0..K-1 with fmaf
-// in order), so the result is bit-identical to the unfused sequence.
-constexpr int kCR = 32;  // elements per block
-template <int NIN, int NH, int NOUT>
-__global__ void __launch_bounds__(256) k_closure_fused(const double *__restrict__ S, const double *__restrict__ geom,
-                                                       const float *__restrict__ mu, const float *__restrict__ sd,
-                                                       const float *__restrict__ W1, const float *__restrict__ b1,
-                                                       const float *__restrict__ W2, const float *__restrict__ b2,
-                                                       const float *__restrict__ W3, const float *__restrict__ b3,
-                                                       const float *__restrict__ muOut, const float *__restrict__ sdOut,
-                                                       const double *__restrict__ qW, double *__restrict__ corr,
-                                                       double *__restrict__ elemMass, int N, int nVar, int massVar,
-                                                       int nEl) {
-  __shared__ float sX[kCR][NIN + 1];
-  __shared__ float sH1[kCR][NH + 4];
-  __shared__ float sH2[kCR][NH + 4];
-  __shared__ float sY[kCR][NOUT + 1];
-  const int t = threadIdx.x;
-  const int e0 = blockIdx.x * kCR;
-  const int NN = (N + 1) * (N + 1);
-  // features
-  for (int q = t; q < kCR * NIN; q += 256) {
-    const int r = q / NIN, k = q % NIN;
-    const int e = e0 + r;
-    float x = 0.f;
-    if (e < nEl) {
-      double raw;
-      if (k < nVar * NN) {
-        raw = S[(size_t)e * nVar * NN + k];
-      } else {
-        const double *g = geom + (size_t)e * kGeomStride;
-        raw = k == nVar * NN ? g[4] : (k == nVar * NN + 1 ? g[0] : g[3]);
-      }
-      x = (float)((raw - (double)mu[k]) / (double)sd[k]);
-    }
-    sX[r][k] = x;
-  }
-  __syncthreads();
-  // hidden layers: thread -> 4 rows x 4 columns
-  const int tr = t / 32, tc = t % 32;
-  auto hidden = [&](const float *A, int lda, int K, const float *W, const float *b, float *H, int ldh) {
-    float acc[4][4] = {{0}};
-    for (int k = 0; k < K; k++) {
-      float a[4], w[4];
-#pragma unroll
-      for (int p = 0; p < 4; p++) a[p] = A[(tr * 4 + p) * lda + k];
-#pragma unroll
-      for (int q = 0; q < 4; q++) w[q] = W[(size_t)k * NH + tc * 4 + q];
-#pragma unroll
-      for (int p = 0; p < 4; p++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) acc[p][q] = fmaf(a[p], w[q], acc[p][q]);
-    }
-#pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) H[(tr * 4 + p) * ldh + tc * 4 + q] = gelu_f(acc[p][q] + b[tc * 4 + q]);
-  };
-  hidden(&sX[0][0], NIN + 1, NIN, W1, b1, &sH1[0][0], NH + 4);
-  __syncthreads();
-  hidden(&sH1[0][0], NH + 4, NH, W2, b2, &sH2[0][0], NH + 4);
-  __syncthreads();
-  // output layer: thread -> 2 rows x 3 columns (NOUT = 48)
-  {
-    const int orow = t / 16, ocol = t % 16;
-    constexpr int OC = NOUT / 16;
-    float acc[2][OC] = {{0}};
-    for (int k = 0; k < NH; k++) {
-      float a0 = sH2[orow * 2][k], a1 = sH2[orow * 2 + 1][k];
-#pragma unroll
-      for (int q = 0; q < OC; q++) {
-        const float w = W3[(size_t)k * NOUT + ocol * OC + q];
-        acc[0][q] = fmaf(a0, w, acc[0][q]);
-        acc[1][q] = fmaf(a1, w, acc[1][q]);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < OC; q++) {
-      sY[orow * 2][ocol * OC + q] = acc[0][q] + b3[ocol * OC + q];
-      sY[orow * 2 + 1][ocol * OC + q] = acc[1][q] + b3[ocol * OC + q];
-    }
-  }
-  __syncthreads();
-  // correction, one wavefront per element (as k_closure_correct)
-  const int P = N + 1, lane = t & 63, wv = t >> 6;
-  for (int r = wv; r < kCR; r += 4) {
-    const size_t e = (size_t)e0 + r;
-    if (e >= (size_t)nEl) break;
-    double m = 0.0;
-    if (lane < NN) {
-      const int i = lane % P, j = lane / P;
-      for (int v = 0; v < nVar; v++) {
-        const int k = v * NN + lane;
-        const double c = (double)sY[r][k] * (double)sdOut[k] + (double)muOut[k];
-        corr[e * (size_t)nVar * NN + k] = c;
-        if (v == massVar) m = qW[i] * qW[j] * c;
-      }
-    }
-    for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off, 64);
-    if (lane == 0) elemMass[e] = geom[e * kGeomStride + 4] * m;
-  }
-}
-
 double lagrange_basis(const double *x, int n, int i, double s) {
   double l = 1.0;
   for (int k = 0; k <= n; k++)
@@ -594,14 +1051,15 @@ hipError_t closure_features(const double *S, const double *geom, const float *in
 hipError_t closure_evaluate(const ClosureBuffers &c, const double *S, const double *geom, const double *qW, int N,
                             int nVar, int massVar, int nEl, hipStream_t st) {
   hipError_t e;
-  const selfamd_mlp *m = c.mlp;
-  if (N == 3 && nVar == 3 && m->nIn == 51 && m->nH == 128 && m->nOut == 48) {
-    // the configured closure shape: one fused launch per 32 elements
-    selfamd_mlp *mm = c.mlp;
-    hipLaunchKernelGGL((k_closure_fused<51, 128, 48>), (nEl + kCR - 1) / kCR, 256, 0, st, S, geom, c.inMean,
-                       c.inScale, mm->W1(), mm->b1(), mm->W2(), mm->b2(), mm->W3(), mm->b3(), c.outMean, c.outScale,
-                       qW, c.corr, c.elemMass, N, nVar, massVar, nEl);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+  int nMass = nEl;  // partial mass integrals: one per element, or one per row tile
+  if (c.mlp->rows) {
+    RowsArgs a = rows_args(c.mlp, nullptr, nEl);
+    a.S = S; a.geom = geom; a.qW = qW;
+    a.inMean = c.inMean; a.inScale = c.inScale; a.outMean = c.outMean; a.outScale = c.outScale;
+    a.corr = c.corr; a.massParts = c.elemMass;
+    a.P = N + 1; a.nVar = nVar; a.massVar = massVar;
+    nMass = (nEl + kRowTile - 1) / kRowTile;
+    if ((e = launch_rows<kRowsClosure>(a, st)) != hipSuccess) return e;
   } else {
     if ((e = closure_features(S, geom, c.inMean, c.inScale, c.X, N, nVar, nEl, st)) != hipSuccess) return e;
     if ((e = forward_impl(c.mlp, c.X, c.Y, nEl, st)) != hipSuccess) return e;
@@ -609,7 +1067,7 @@ hipError_t closure_evaluate(const ClosureBuffers &c, const double *S, const doub
                        c.elemMass, N, nVar, massVar, nEl);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_closure_shift, 1, 256, 0, st, c.elemMass, c.shift, c.invArea, nEl);
+  hipLaunchKernelGGL(k_closure_shift, 1, 256, 0, st, c.elemMass, c.shift, c.invArea, nMass);
   return hipGetLastError();
 }
 
@@ -698,7 +1156,6 @@ hipError_t closure_vjp(const ClosureBuffers &c, const double *S, const double *g
   hipLaunchKernelGGL(k_vjp_dY, blocks, 256, 0, st, lam, c.vjpPartial + nb, c.outScale, geom, qW, c.dY, N, nVar, massVar,
                      c.invArea, n);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if ((e = forward_impl(c.mlp, c.X, c.mlp->Y, nEl, st)) != hipSuccess) return e;
   if ((e = backward_impl(c.mlp, c.X, c.dY, nEl, 1, c.dX, st)) != hipSuccess) return e;
   hipLaunchKernelGGL(k_vjp_mu, blocks, 256, 0, st, c.dX, c.inScale, mu, c.nIn, c.nOut, n);
   return hipGetLastError();
