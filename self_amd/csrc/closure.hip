@@ -1017,6 +1017,8 @@ __global__ void __launch_bounds__(256) k_closure_shift(const double *__restrict_
   if (threadIdx.x == 0) shift[0] = red[0] * invArea;
 }
 
+constexpr int kShiftParts = 512;
+
 double lagrange_basis(const double *x, int n, int i, double s) {
   double l = 1.0;
   for (int k = 0; k <= n; k++)
@@ -1048,7 +1050,7 @@ hipError_t closure_features(const double *S, const double *geom, const float *in
   return hipGetLastError();
 }
 
-hipError_t closure_evaluate(const ClosureBuffers &c, const double *S, const double *geom, const double *qW, int N,
+hipError_t closure_evaluate(ClosureBuffers &c, const double *S, const double *geom, const double *qW, int N,
                             int nVar, int massVar, int nEl, hipStream_t st) {
   hipError_t e;
   int nMass = nEl;  // partial mass integrals: one per element, or one per row tile
@@ -1067,7 +1069,13 @@ hipError_t closure_evaluate(const ClosureBuffers &c, const double *S, const doub
                        c.elemMass, N, nVar, massVar, nEl);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_closure_shift, 1, 256, 0, st, c.elemMass, c.shift, c.invArea, nMass);
+  // A few hundred partial integrals are added by the stage kernel itself; its wavefronts each
+  // read all of them, so more are reduced to their sum here first (one block, about 4.5 us).
+  c.shiftParts = c.elemMass; c.nShift = nMass; c.shiftScale = c.invArea;
+  if (nMass > kShiftParts) {
+    hipLaunchKernelGGL(k_closure_shift, 1, 256, 0, st, c.elemMass, c.shift, c.invArea, nMass);
+    c.shiftParts = c.shift; c.nShift = 1; c.shiftScale = 1.0;
+  }
   return hipGetLastError();
 }
 

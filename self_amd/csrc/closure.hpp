@@ -14,8 +14,12 @@ struct ClosureBuffers {
   float *X = nullptr, *Y = nullptr;          // MLP input / output, one row per element
   float *inMean = nullptr, *inScale = nullptr, *outMean = nullptr, *outScale = nullptr;
   double *corr = nullptr;                    // correction in the interior layout (0:N,0:N,nVar,nEl)
-  double *elemMass = nullptr;                // per-element integral of the mass-variable correction
+  double *elemMass = nullptr;                // integrals of the mass-variable correction, per element or per row tile
   double *shift = nullptr;                   // one double: global mean of the mass correction
+  // where closure_evaluate left that mean: shiftScale times the sum of nShift doubles
+  const double *shiftParts = nullptr;
+  int nShift = 0;
+  double shiftScale = 0.0;
   double invArea = 0.0;                      // 1 / (sum over elements of the element area in xi-space times J)
   // adjoint (closure_vjp) work space
   float *dY = nullptr, *dX = nullptr;        // output / input cotangents, one row per element
@@ -27,8 +31,8 @@ struct ClosureBuffers {
 hipError_t closure_features(const double *S, const double *geom, const float *inMean, const float *inScale, float *X,
                             int N, int nVar, int nEl, hipStream_t st);
 
-// features -> MLP -> correction (+ per-element mass integrals and the global mean shift)
-hipError_t closure_evaluate(const ClosureBuffers &c, const double *S, const double *geom, const double *qW, int N,
+// features -> MLP -> correction and its mass integrals; sets where their mean is to be read
+hipError_t closure_evaluate(ClosureBuffers &c, const double *S, const double *geom, const double *qW, int N,
                             int nVar, int massVar, int nEl, hipStream_t st);
 
 // Adjoint of the correction that closure_evaluate adds to dS/dt at state S: for the cotangent
