@@ -13,6 +13,7 @@
 // outputs each, the reductions over the batch split and summed in the same way.
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -931,8 +932,100 @@ int selfamd_mlp_adam_step(selfamd_mlp *m, float lr, int step, void *stream) {
 // Nc + Nf <= 2 Nf + 1), and mass-conserving: sum_ij w_i w_j u_c = r^-2 sum_ab sum_pq w_p w_q u_f.
 namespace {
 
-__global__ void k_project(const double *__restrict__ Sf, double *__restrict__ Sc, const double *__restrict__ Px, int Nf,
-                          int Nc, int nxc, int nyc, int r, int nVar) {
+// One block per coarse element.  The fine rows of elements are read as the contiguous runs they
+// are (r nVar Pf^2 doubles per sub-row b), `rowsB` sub-rows at a time, into LDS; then
+// row[b][v][q][i] = sum_a,p Px[a][i][p] u, and u_c += sum_b,q Px[b][j][q] row.  Bound by reading
+// the fine state: 104 MB (256^2 N = 7, three variables) in 38 us (2.7 TB/s: a block's loads and
+// sums do not overlap, five blocks per CU do), where one work-item per coarse value, each reading
+// r^2 Pf^2 doubles with its neighbours 64 bytes or whole elements away, took 276 us.  Chunks of
+// half the size, for twice the blocks per CU, run at the same 38 us, a quarter at 60 us.  LDS rows of Pf doubles are padded by one: four of five rows would share banks at
+// Pf = 8.
+constexpr int kProjectArgs = 448, kProjectLds = 6144, kProjectChunk = 3072;  // doubles
+struct ProjectArgs {
+  const double *fine;
+  double *coarse;
+  int Pf, Pc, nxc, r, nVar, rowsB;
+  unsigned invPf, invRun;      // k / Pf = (k invPf) >> 20 and k / run = high word of k invRun, k < kProjectLds
+  double px[kProjectArgs];     // Px[a][i][p]
+};
+static_assert(sizeof(ProjectArgs) <= 4096, "kernel arguments exceed the 4 KiB kernarg segment");
+
+// PC = Pc with the sums of one LDS row for all i in one work-item (the factors are uniform and
+// come in scalar registers), where one sum per work-item reads every u Pc times; PC = 0: one sum
+// per work-item, for other degrees.
+template <int PC>
+__global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
+  extern __shared__ double projectLds[];
+  const int tid = threadIdx.x, Pf = a.Pf, Pc = a.Pc, r = a.r, nVar = a.nVar, nPx = r * Pc * Pf, ld = Pf + 1;
+  const int run = r * nVar * Pf * Pf, rows = r * nVar * Pf, nOut = nVar * Pc * Pc, perB = nVar * Pf * Pc;
+  double *sPx = projectLds, *sU = sPx + nPx, *sRow = sU + a.rowsB * rows * ld, *sOut = sRow + a.rowsB * perB;
+  const int I = blockIdx.x % a.nxc, J = blockIdx.x / a.nxc;
+  const size_t nxf = (size_t)a.nxc * r;
+  for (int k = tid; k < nPx; k += 256) sPx[k] = a.px[k];
+  for (int k = tid; k < nOut; k += 256) sOut[k] = 0.0;
+  for (int b0 = 0; b0 < r; b0 += a.rowsB) {
+    const int nb = min(a.rowsB, r - b0);
+    // the whole chunk (up to 3,072 doubles) in flight at once: with one sub-row after another a
+    // block waits for memory rowsB times (43 us)
+    const double *src = a.fine + (size_t)nVar * Pf * Pf * ((size_t)I * r + nxf * ((size_t)J * r + b0));
+    const size_t subRow = (size_t)nVar * Pf * Pf * nxf;
+    const int total = nb * run;
+    for (int k0 = tid; k0 < total; k0 += kProjectChunk) {
+      constexpr int M = kProjectChunk / 256;
+      double v[M];
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        const unsigned k = min(k0 + 256 * m, total - 1), b = __umulhi(k, a.invRun);
+        v[m] = src[b * subRow + (k - b * run)];
+      }
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        const unsigned k = k0 + 256 * m;
+        if ((int)k < total) sU[k + (k * a.invPf >> 20)] = v[m];  // one pad per row of Pf
+      }
+    }
+    __syncthreads();
+    if constexpr (PC > 0) {
+      for (int t = tid; t < nb * nVar * Pf; t += 256) {
+        const int vq = t % (nVar * Pf), b = t / (nVar * Pf);
+        double row[PC] = {};
+        for (int aa = 0; aa < r; aa++) {
+          const double *u = sU + (b * rows + aa * nVar * Pf + vq) * ld, *px = a.px + aa * PC * Pf;
+          for (int p = 0; p < Pf; p++) {
+            const double x = u[p];
+#pragma unroll
+            for (int i = 0; i < PC; i++) row[i] += px[i * Pf + p] * x;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < PC; i++) sRow[t * PC + i] = row[i];
+      }
+    } else for (int t = tid; t < nb * perB; t += 256) {
+      const int i = t % Pc, vq = t / Pc % (nVar * Pf), b = t / perB;
+      double row = 0.0;
+      for (int aa = 0; aa < r; aa++) {
+        const double *u = sU + (b * rows + aa * nVar * Pf + vq) * ld, *px = sPx + (aa * Pc + i) * Pf;
+        for (int p = 0; p < Pf; p++) row += px[p] * u[p];
+      }
+      sRow[t] = row;
+    }
+    __syncthreads();
+    for (int t = tid; t < nOut; t += 256) {
+      const int i = t % Pc, j = t / Pc % Pc, v = t / (Pc * Pc);
+      double acc = sOut[t];
+      for (int b = 0; b < nb; b++)
+        for (int q = 0; q < Pf; q++) acc += sPx[((b0 + b) * Pc + j) * Pf + q] * sRow[b * perB + (v * Pf + q) * Pc + i];
+      sOut[t] = acc;
+    }
+    __syncthreads();
+  }
+  for (int t = tid; t < nOut; t += 256) a.coarse[(size_t)blockIdx.x * nOut + t] = sOut[t];
+}
+
+// The same, one work-item per coarse value, for coarsening factors and degrees whose factors or
+// runs are too long for the kernel arguments or LDS of k_project.
+__global__ void k_project_values(const double *__restrict__ Sf, double *__restrict__ Sc, const double *__restrict__ Px,
+                                 int Nf, int Nc, int nxc, int nyc, int r, int nVar) {
   const int Pf = Nf + 1, Pc = Nc + 1;
   const size_t total = (size_t)Pc * Pc * nVar * nxc * nyc;
   const int nxf = nxc * r;
@@ -1018,6 +1111,23 @@ __global__ void __launch_bounds__(256) k_closure_shift(const double *__restrict_
 }
 
 constexpr int kShiftParts = 512;
+
+// Gauss nodes and weights of degree N, computed once: the reference's Newton sweep runs all of
+// its 500 iterations for every negative node, about 0.1 ms per degree.
+struct GaussRule {
+  double x[kMaxN + 1], w[kMaxN + 1];
+  bool ok;
+};
+const GaussRule *gauss_rule(int N) {
+  static GaussRule rules[kMaxN + 1];
+  static std::once_flag once[kMaxN + 1];
+  GaussRule &g = rules[N];
+  std::call_once(once[N], [&g, N] {
+    double t[kMaxN + 1], bw[kMaxN + 1], m[3][(kMaxN + 1) * (kMaxN + 1)], bM[2 * (kMaxN + 1)];
+    g.ok = selfamd_lagrange_init(N, SELFAMD_GAUSS, N, SELFAMD_GAUSS, g.x, t, bw, g.w, m[0], m[1], m[2], bM) == kOk;
+  });
+  return g.ok ? &g : nullptr;
+}
 
 double lagrange_basis(const double *x, int n, int i, double s) {
   double l = 1.0;
@@ -1180,31 +1290,51 @@ int selfamd_project_l2_structured_2d(const double *fine, double *coarse, int Nf,
                   "project_l2_structured_2d: bad sizes (Nf=%d Nc=%d nxc=%d nyc=%d r=%d nVar=%d)", Nf, Nc, nxc, nyc, r,
                   nVar);
   SELFAMD_REQUIRE(Nc <= 2 * Nf + 1, "project_l2_structured_2d: fine quadrature too coarse for Nc=%d", Nc);
-  double xf[kMaxN + 1], tf[kMaxN + 1], bwf[kMaxN + 1], wf[kMaxN + 1];
-  double xc[kMaxN + 1], tc[kMaxN + 1], bwc[kMaxN + 1], wc[kMaxN + 1];
-  std::vector<double> iM((kMaxN + 1) * (kMaxN + 1)), dM(iM.size()), dgM(iM.size()), bM(2 * (kMaxN + 1));
-  int rc = selfamd_lagrange_init(Nf, SELFAMD_GAUSS, Nf, SELFAMD_GAUSS, xf, tf, bwf, wf, iM.data(), dM.data(),
-                                 dgM.data(), bM.data());
-  if (rc) return rc;
-  rc = selfamd_lagrange_init(Nc, SELFAMD_GAUSS, Nc, SELFAMD_GAUSS, xc, tc, bwc, wc, iM.data(), dM.data(), dgM.data(),
-                             bM.data());
-  if (rc) return rc;
+  const GaussRule *fineRule = gauss_rule(Nf), *coarseRule = gauss_rule(Nc);
+  SELFAMD_REQUIRE(fineRule && coarseRule, "project_l2_structured_2d: no quadrature for Nf=%d Nc=%d", Nf, Nc);
+  const double *xf = fineRule->x, *wf = fineRule->w, *xc = coarseRule->x, *wc = coarseRule->w;
   const int Pf = Nf + 1, Pc = Nc + 1;
-  std::vector<double> px((size_t)r * Pc * Pf);
+  const size_t nPx = (size_t)r * Pc * Pf, run = (size_t)r * nVar * Pf * Pf;
+  auto entry = [&](int a, int i, int p) {
+    const double xi = -1.0 + (2.0 * a + 1.0 + xf[p]) / r;
+    return wf[p] * lagrange_basis(xc, Nc, i, xi) / (r * wc[i]);
+  };
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (nPx <= (size_t)kProjectArgs && run <= (size_t)kProjectLds) {
+    ProjectArgs g;
+    g.fine = fine; g.coarse = coarse; g.Pf = Pf; g.Pc = Pc; g.nxc = nxc; g.r = r; g.nVar = nVar;
+    g.rowsB = std::max(1, std::min(r, kProjectChunk / (int)run));
+    g.invPf = ((1u << 20) + Pf - 1) / Pf;
+    g.invRun = (unsigned)(((1ull << 32) + run - 1) / run);
+    for (int a = 0; a < r; a++)
+      for (int i = 0; i < Pc; i++)
+        for (int p = 0; p < Pf; p++) g.px[(a * Pc + i) * Pf + p] = entry(a, i, p);
+    const size_t lds = nPx + (size_t)g.rowsB * r * nVar * Pf * (Pf + 1) + (size_t)g.rowsB * nVar * Pf * Pc + (size_t)nVar * Pc * Pc;
+    if (sizeof(double) * lds <= 64 * 1024) {
+      const unsigned blocks = (unsigned)((size_t)nxc * nyc);
+      switch (Pc) {
+#define CASE(PC) \
+  case PC: hipLaunchKernelGGL(k_project<PC>, blocks, 256, sizeof(double) * lds, st, g); break;
+        CASE(2) CASE(3) CASE(4) CASE(5) CASE(6)
+#undef CASE
+        default: hipLaunchKernelGGL(k_project<0>, blocks, 256, sizeof(double) * lds, st, g);
+      }
+      SELFAMD_HIP(hipGetLastError());
+      SELFAMD_HIP(hipStreamSynchronize(st));
+      return kOk;
+    }
+  }
+  std::vector<double> px(nPx);
   for (int a = 0; a < r; a++)
     for (int i = 0; i < Pc; i++)
-      for (int p = 0; p < Pf; p++) {
-        const double xi = -1.0 + (2.0 * a + 1.0 + xf[p]) / r;
-        px[((size_t)a * Pc + i) * Pf + p] = wf[p] * lagrange_basis(xc, Nc, i, xi) / (r * wc[i]);
-      }
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+      for (int p = 0; p < Pf; p++) px[((size_t)a * Pc + i) * Pf + p] = entry(a, i, p);
   double *dPx = nullptr;
   SELFAMD_HIP(hipMalloc(&dPx, sizeof(double) * px.size()));
   hipError_t e = hipMemcpyAsync(dPx, px.data(), sizeof(double) * px.size(), hipMemcpyHostToDevice, st);
   const size_t total = (size_t)Pc * Pc * nVar * nxc * nyc;
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_project, (unsigned)std::min<size_t>((total + 255) / 256, 65535), 256, 0, st, fine, coarse, dPx,
-                       Nf, Nc, nxc, nyc, r, nVar);
+    hipLaunchKernelGGL(k_project_values, (unsigned)std::min<size_t>((total + 255) / 256, 65535), 256, 0, st, fine, coarse,
+                       dPx, Nf, Nc, nxc, nyc, r, nVar);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(st);
