@@ -8,6 +8,10 @@
 // output (the node index i) on the lane index so every load/store of a variable's P*P
 // block is coalesced.  Each work-item accumulates its contraction in registers and
 // writes once (the reference kernels accumulate into global memory inside the loop).
+// Index arithmetic: kernels are instantiated for P = 2 .. 8 with 32-bit indices, where / and %
+// by P are a few instructions; other sizes take the runtime P and 64-bit indices, whose divisions
+// cost more than the arithmetic of the contractions (kIndex32).
+// The boundary interpolation and the divergences read each value once, through LDS, for P <= 8.
 #include "selfamd_common.hpp"
 #include "../../include/self_amd.h"
 
@@ -42,6 +46,40 @@ __global__ void k_boundary_interp(const double *__restrict__ bM, const double *_
       acc += b[ii] * f[c + ncomp * node];
     }
     fb[t] = acc;
+  }
+}
+
+// The same for P <= 8: a block takes SPB (element, variable) slabs of P*P nodes through LDS, so
+// that every value is read once, coalesced (one work-item per output reads P values, for two
+// sides of four a row apart: 15.4 us for three variables on 128 x 96 N = 7; this kernel 7.5 us for
+// 28 MB).
+// Slabs are numbered v + nVar e; a slab's values are contiguous, its traces four runs of P.
+template <int P, int NC>
+__global__ void __launch_bounds__(256) k_boundary_interp_lds(const double *__restrict__ bM, const double *__restrict__ f,
+                                                             double *__restrict__ fb, int nVar, unsigned slabs) {
+  constexpr int PP = P * P, SPB = 256 / (4 * P * NC) > 0 ? 256 / (4 * P * NC) : 1, LD = PP * NC + (PP * NC % 2 ? 0 : 1);
+  __shared__ double sF[SPB * LD], sB[2 * P];
+  const int tid = threadIdx.x;
+  const unsigned s0 = blockIdx.x * SPB, n = min((unsigned)SPB, slabs - s0);
+  constexpr int LOADS = (SPB * PP * NC + 255) / 256;
+  double v[LOADS];
+#pragma unroll
+  for (int q = 0; q < LOADS; q++) v[q] = f[(size_t)s0 * PP * NC + min(tid + 256u * q, n * PP * NC - 1)];
+  if (tid < 2 * P) sB[tid] = bM[tid];
+#pragma unroll
+  for (int q = 0; q < LOADS; q++) {
+    const unsigned k = tid + 256 * q;
+    if (k < n * PP * NC) sF[k + (LD - PP * NC) * (k / (PP * NC))] = v[q];
+  }
+  __syncthreads();
+  for (unsigned t = tid; t < n * 4 * P * NC; t += 256) {
+    const unsigned c = t % NC, i = t / NC % P, s = t / (NC * P) % 4, slab = t / (4 * P * NC);
+    const double *b = sB + (s == 1 || s == 2 ? P : 0), *u = sF + slab * LD + c;
+    double acc = 0.0;
+#pragma unroll
+    for (int ii = 0; ii < P; ii++) acc += b[ii] * u[NC * (s == 0 || s == 2 ? i + P * ii : ii + P * i)];
+    const unsigned sv = s0 + slab, e = sv / nVar, var = sv - e * nVar;
+    fb[c + NC * (i + P * (var + (size_t)nVar * (s + 4 * (size_t)e)))] = acc;
   }
 }
 
@@ -115,6 +153,47 @@ __global__ void k_divergence(const double *__restrict__ dM, const double *__rest
   }
 }
 
+// The same for P <= 8: the flux of 256 / P^2 (element, variable) slabs through LDS, read once as
+// 16-byte pairs (one work-item per output with all reads from memory: 2P cached loads each and
+// 64-bit index divisions, 56 us for the weak form of three variables on 128 x 96 N = 7; this
+// kernel 18 us for 66 MB).  Matrix rows are transposed in LDS: lanes of a row read consecutive
+// entries.  The sums keep the order of the kernel above.
+template <int P, bool WEAK>
+__global__ void __launch_bounds__(256) k_divergence_lds(const double *__restrict__ dM, const double *__restrict__ bM,
+                                                        const double *__restrict__ qW, const double *__restrict__ f,
+                                                        const double *__restrict__ bF, double *__restrict__ dF, int nVar,
+                                                        unsigned slabs) {
+  constexpr int PP = P * P, SPB = 256 / PP;
+  __shared__ double sF1[SPB * PP], sF2[SPB * PP], sM[PP];
+  const int tid = threadIdx.x, slab = tid / PP, node = tid % PP, i = node % P, j = node / P;
+  const unsigned sv = blockIdx.x * SPB + slab;
+  const bool active = slab < SPB && sv < slabs;
+  const size_t at = (size_t)sv * PP + node;
+  double bE = 0.0, bW = 0.0, bN = 0.0, bS = 0.0, m1i = 0.0, m0i = 0.0, m1j = 0.0, m0j = 0.0, wi = 1.0, wj = 1.0;
+  if (active) {
+    const double x = f[2 * at], y = f[2 * at + 1];
+    if (WEAK) {
+      const unsigned e = sv / nVar, v = sv - e * nVar;
+      const double *b = bF + P * (v + (size_t)nVar * 4 * e);
+      const size_t side = (size_t)P * nVar;
+      bE = b[side + j]; bW = b[3 * side + j]; bN = b[2 * side + i]; bS = b[i];
+      m1i = bM[i + P]; m0i = bM[i]; m1j = bM[j + P]; m0j = bM[j];
+      wi = qW[i]; wj = qW[j];
+    }
+    sF1[tid] = x;
+    sF2[tid] = y;
+  }
+  for (int k = tid; k < PP; k += 256) sM[(k % P) * P + k / P] = dM[k];  // sM(i, ii) = dM(ii, i)
+  __syncthreads();
+  if (!active) return;
+  const double *f1 = sF1 + slab * PP + P * j, *f2 = sF2 + slab * PP + i;
+  double d = 0.0;
+#pragma unroll
+  for (int ii = 0; ii < P; ii++) d = d + sM[P * ii + i] * f1[ii] + sM[P * ii + j] * f2[P * ii];
+  if (WEAK) d = d + (m1i * bE + m0i * bW) / wi + (m1j * bN + m0j * bS) / wj;
+  dF[at] = d;
+}
+
 // Determinant_Tensor2D (src/SELF_Data.f90:1570-1607)
 __global__ void k_determinant(const double *__restrict__ tsr, double *__restrict__ det, size_t n) {
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
@@ -126,17 +205,18 @@ __global__ void k_determinant(const double *__restrict__ tsr, double *__restrict
 // ---------------------------------------------------------------------------------
 
 // SideExchange (src/SELF_MappedData.f90:834-917, 1870-1958): work-item = (c, i, v, s, e)
+template <int PT, class Idx>
 __global__ void k_side_exchange(const double *__restrict__ bnd, double *__restrict__ ext,
                                 const int32_t *__restrict__ si, int N, int nVar, int nEl, int ncomp) {
-  const size_t P = N + 1;
-  const size_t total = (size_t)ncomp * P * nVar * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    size_t r = t;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = (Idx)ncomp * P * nVar * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    Idx r = t;
     const int c = r % ncomp; r /= ncomp;
     const int i1 = r % P; r /= P;
     const int v = r % nVar; r /= nVar;
     const int s1 = r % 4;
-    const size_t e1 = r / 4;
+    const Idx e1 = r / 4;
     const int32_t *s = si + 5 * (s1 + 4 * e1);
     if (s[4] != 0) continue;
     const int s2 = s[3] / 10, flip = s[3] - 10 * s2;
@@ -148,20 +228,21 @@ __global__ void k_side_exchange(const double *__restrict__ bnd, double *__restri
 }
 
 // GradientSF_MappedScalar2D (src/SELF_MappedData.f90:1080-1149)
+template <int PT, class Idx>
 __global__ void k_gradient_sf(const double *__restrict__ dM, const double *__restrict__ dsdx,
                               const double *__restrict__ J, const double *__restrict__ f,
                               double *__restrict__ gradF, int N, int nVar, int nEl) {
-  const size_t P = N + 1;
-  const size_t total = P * P * nVar * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    size_t r = t;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * P * nVar * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    Idx r = t;
     const int i = r % P; r /= P;
     const int j = r % P; r /= P;
     const int v = r % nVar;
-    const size_t e = r / nVar;
+    const Idx e = r / nVar;
     double gx = 0.0, gy = 0.0;
     for (int ii = 0; ii <= N; ii++) {
-      const size_t g1 = 4 * (ii + P * (j + P * e)), g2 = 4 * (i + P * (ii + P * e));
+      const Idx g1 = 4 * (ii + P * (j + P * e)), g2 = 4 * (i + P * (ii + P * e));
       const double fa = f[sc_idx(ii, j, v, e, P, nVar)], fb = f[sc_idx(i, ii, v, e, P, nVar)];
       gx = gx + dM[ii + P * i] * (fa * dsdx[g1 + 0]) + dM[ii + P * j] * (fb * dsdx[g2 + 2]);
       gy = gy + dM[ii + P * i] * (fa * dsdx[g1 + 1]) + dM[ii + P * j] * (fb * dsdx[g2 + 3]);
@@ -173,22 +254,24 @@ __global__ void k_gradient_sf(const double *__restrict__ dM, const double *__res
 }
 
 // JacobianWeight (src/SELF_MappedData.f90:1235-1268)
+template <int PT, class Idx>
 __global__ void k_jacobian_weight(const double *__restrict__ J, double *__restrict__ f, int N, int nVar, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nVar * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / (PP * nVar);
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nVar * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / (PP * nVar);
     f[t] = f[t] / J[node + PP * e];
   }
 }
 
 // ContravariantProjection (src/SELF_MappedData.f90:2220-2269)
+template <int PT, class Idx>
 __global__ void k_contravariant_projection(const double *__restrict__ dsdx, double *__restrict__ f, int N, int nVar,
                                            int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nVar * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / (PP * nVar);
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nVar * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / (PP * nVar);
     const double *g = dsdx + 4 * (node + PP * e);
     const double Fx = f[2 * t], Fy = f[2 * t + 1];
     f[2 * t] = g[0] * Fx + g[1] * Fy;
@@ -196,20 +279,45 @@ __global__ void k_contravariant_projection(const double *__restrict__ dsdx, doub
   }
 }
 
+// The streaming updates take two values per work-item (16-byte accesses) where every array is
+// 16-byte aligned, one where not; an odd last value is taken alone.
+inline __host__ __device__ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // UpdateGRK_Model2D (src/SELF_Model2D.f90:710-752)
+template <bool PAIRS>
 __global__ void k_update_grk(double *__restrict__ G, double *__restrict__ S, const double *__restrict__ dSdt,
                              double a, double gdt, size_t n) {
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
-    const double g = a * G[t] + dSdt[t];
-    G[t] = g;
-    S[t] = S[t] + gdt * g;
+  constexpr int W = PAIRS ? 2 : 1;
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; W * t < n; t += (size_t)gridDim.x * blockDim.x) {
+    if (PAIRS && 2 * t + 1 < n) {
+      double2 g = reinterpret_cast<double2 *>(G)[t], s = reinterpret_cast<double2 *>(S)[t];
+      const double2 d = reinterpret_cast<const double2 *>(dSdt)[t];
+      g.x = a * g.x + d.x;
+      g.y = a * g.y + d.y;
+      s.x = s.x + gdt * g.x;
+      s.y = s.y + gdt * g.y;
+      reinterpret_cast<double2 *>(G)[t] = g;
+      reinterpret_cast<double2 *>(S)[t] = s;
+    } else {
+      const double g = a * G[W * t] + dSdt[W * t];
+      G[W * t] = g;
+      S[W * t] = S[W * t] + gdt * g;
+    }
   }
 }
 
 // dSdt = source - fluxDivergence (src/SELF_Model2D.f90:843-855)
+template <bool PAIRS>
 __global__ void k_dsdt(const double *__restrict__ fd, const double *__restrict__ src, double *__restrict__ d, size_t n) {
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
-    d[t] = src[t] - fd[t];
+  constexpr int W = PAIRS ? 2 : 1;
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; W * t < n; t += (size_t)gridDim.x * blockDim.x) {
+    if (PAIRS && 2 * t + 1 < n) {
+      const double2 x = reinterpret_cast<const double2 *>(src)[t], y = reinterpret_cast<const double2 *>(fd)[t];
+      reinterpret_cast<double2 *>(d)[t] = make_double2(x.x - y.x, x.y - y.y);
+    } else {
+      d[W * t] = src[W * t] - fd[W * t];
+    }
+  }
 }
 
 // Contravariant basis, outward normals and face scale (src/SELF_Geometry.f90:437-526):
@@ -249,19 +357,20 @@ __global__ void k_dsdx_from_dxds(const double *__restrict__ dxds, double *__rest
 // ---------------------------------------------------------------------------------
 
 // SW PreTendency velocity (src/models/SELF_ShallowWater.f90:206-235)
+template <int PT, class Idx>
 __global__ void k_sw_velocity(const double *__restrict__ sol, const double *__restrict__ solB, double *__restrict__ vel,
                               double *__restrict__ velB, int N, int nEl) {
-  const size_t P = N + 1, PP = P * P;
-  const size_t nInt = PP * nEl, nBnd = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < nInt + nBnd; t += (size_t)gridDim.x * blockDim.x) {
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx nInt = PP * nEl, nBnd = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < nInt + nBnd; t += (Idx)gridDim.x * blockDim.x) {
     if (t < nInt) {
-      const size_t node = t % PP, e = t / PP;
+      const Idx node = t % PP, e = t / PP;
       const double H = sol[node + PP * (2 + 3 * e)];
       vel[2 * t] = sol[node + PP * (3 * e)] / H;
       vel[2 * t + 1] = sol[node + PP * (1 + 3 * e)] / H;
     } else {
-      const size_t b = t - nInt;
-      const size_t i = b % P, se = b / P;  // se = s + 4e
+      const Idx b = t - nInt;
+      const Idx i = b % P, se = b / P;  // se = s + 4e
       const double H = solB[i + P * (2 + 3 * se)];
       velB[2 * b] = solB[i + P * (3 * se)] / H;
       velB[2 * b + 1] = solB[i + P * (1 + 3 * se)] / H;
@@ -272,16 +381,17 @@ __global__ void k_sw_velocity(const double *__restrict__ sol, const double *__re
 // Boundary conditions on physical sides (e2 == 0), work-item = (i, s, e).
 // kind: 1 LSW (src/models/SELF_LinearShallowWater.f90:298-355), 2 SW (quirk: radiation
 // sets the external thickness to the topography trace, SELF_ShallowWater.f90:284-343).
+template <int PT, class Idx>
 __global__ void k_sw_bc(const double *__restrict__ solB, double *__restrict__ solE, const double *__restrict__ topoB,
                         const double *__restrict__ nHat, const int32_t *__restrict__ si, int N, int nEl, int kind) {
-  const size_t P = N + 1;
-  const size_t total = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t i = t % P, se = t / P;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx i = t % P, se = t / P;
     const int32_t *s = si + 5 * se;
     if (s[2] != 0) continue;
     const double nx = nHat[2 * t], ny = nHat[2 * t + 1];
-    const size_t o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
+    const Idx o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
     if (s[4] == SELFAMD_BC_NONORMALFLOW) {
       const double u = solB[o0], v = solB[o1];
       solE[o0] = (ny * ny - nx * nx) * u - 2.0 * nx * ny * v;
@@ -296,13 +406,14 @@ __global__ void k_sw_bc(const double *__restrict__ solB, double *__restrict__ so
 }
 
 // SW source (src/models/SELF_ShallowWater.f90:345-384)
+template <int PT, class Idx>
 __global__ void k_sw_source(double *__restrict__ src, const double *__restrict__ sol, const double *__restrict__ gradH,
                             double g, double f, int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
     src[o0] = -f * sol[o1] + g * sol[o2] * gradH[2 * t];
     src[o1] = f * sol[o0] + g * sol[o2] * gradH[2 * t + 1];
     src[o2] = 0.0;
@@ -310,13 +421,14 @@ __global__ void k_sw_source(double *__restrict__ src, const double *__restrict__
 }
 
 // SW flux (src/models/SELF_ShallowWater.f90:386-449)
+template <int PT, class Idx>
 __global__ void k_sw_flux(double *__restrict__ flux, const double *__restrict__ sol, const double *__restrict__ vel,
                           double g, int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
     const double u = vel[2 * t], v = vel[2 * t + 1], Hu = sol[o0], Hv = sol[o1], H = sol[o2];
     flux[2 * o0] = u * Hu + 0.5 * g * H * H;
     flux[2 * o0 + 1] = v * Hu;
@@ -328,18 +440,19 @@ __global__ void k_sw_flux(double *__restrict__ flux, const double *__restrict__ 
 }
 
 // SW Rusanov flux (src/models/SELF_ShallowWater.f90:451-529)
+template <int PT, class Idx>
 __global__ void k_sw_riemann(double *__restrict__ fbn, const double *__restrict__ solB, const double *__restrict__ solE,
                              const double *__restrict__ velB, const double *__restrict__ velE,
                              const double *__restrict__ nHat, const double *__restrict__ nScale, double g, int N,
                              int nEl) {
-  const size_t P = N + 1;
-  const size_t total = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t i = t % P, se = t / P;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx i = t % P, se = t / P;
     const double nx = nHat[2 * t], ny = nHat[2 * t + 1], nmag = nScale[t];
     const double unL = velB[2 * t] * nx + velB[2 * t + 1] * ny;
     const double unR = velE[2 * t] * nx + velE[2 * t + 1] * ny;
-    const size_t o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
+    const Idx o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
     const double HuL = solB[o0], HuR = solE[o0], HvL = solB[o1], HvR = solE[o1], HL = solB[o2], HR = solE[o2];
     const double cL = sqrt(g * HL), cR = sqrt(g * HR);
     const double fL0 = HuL * unL + g * HL * HL * 0.5 * nx, fL1 = HvL * unL + g * HL * HL * 0.5 * ny;
@@ -354,13 +467,14 @@ __global__ void k_sw_riemann(double *__restrict__ fbn, const double *__restrict_
 }
 
 // LSW source (src/models/SELF_LinearShallowWater.f90:413-446)
+template <int PT, class Idx>
 __global__ void k_lsw_source(double *__restrict__ src, const double *__restrict__ sol, const double *__restrict__ fc,
                              int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
     src[o0] = fc[t] * sol[o1];
     src[o1] = -fc[t] * sol[o0];
     src[o2] = 0.0;
@@ -368,13 +482,14 @@ __global__ void k_lsw_source(double *__restrict__ src, const double *__restrict_
 }
 
 // LSW flux (src/models/SELF_LinearShallowWater.f90:448-498)
+template <int PT, class Idx>
 __global__ void k_lsw_flux(double *__restrict__ flux, const double *__restrict__ sol, const double *__restrict__ H,
                            double g, int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 3 * e, o1 = o0 + PP, o2 = o1 + PP;
     flux[2 * o0] = g * sol[o2];
     flux[2 * o0 + 1] = 0.0;
     flux[2 * o1] = 0.0;
@@ -385,16 +500,17 @@ __global__ void k_lsw_flux(double *__restrict__ flux, const double *__restrict__
 }
 
 // LSW characteristic upwind flux (src/models/SELF_LinearShallowWater.f90:500-557)
+template <int PT, class Idx>
 __global__ void k_lsw_riemann(double *__restrict__ fbn, const double *__restrict__ solB, const double *__restrict__ solE,
                               const double *__restrict__ Hb, const double *__restrict__ nHat,
                               const double *__restrict__ nScale, double g, int N, int nEl) {
-  const size_t P = N + 1;
-  const size_t total = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t i = t % P, se = t / P;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx i = t % P, se = t / P;
     const double nx = nHat[2 * t], ny = nHat[2 * t + 1], nmag = nScale[t];
     const double c = sqrt(g * Hb[t]);
-    const size_t o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
+    const Idx o0 = i + P * (3 * se), o1 = o0 + P, o2 = o0 + 2 * P;
     const double unL = solB[o0] * nx + solB[o1] * ny, unR = solE[o0] * nx + solE[o1] * ny;
     const double wL = 0.5 * (unL / g + solB[o2] / c), wR = 0.5 * (unR / g - solE[o2] / c);
     fbn[o0] = g * c * (wL - wR) * nx * nmag;
@@ -405,13 +521,14 @@ __global__ void k_lsw_riemann(double *__restrict__ fbn, const double *__restrict
 
 // Euler node-local diagnostics (src/models/SELF_CompressibleIdealGas2D.f90:984-1215).
 // what: 0 diagnostics (KE, rho*E+p, c, T), 1 primitive (u, v, rho, p), 2 entropy variables.
+template <int PT, class Idx>
 __global__ void k_euler_nodal(const double *__restrict__ sol, double *__restrict__ out, double gam, double R, int N,
                               int nEl, int what) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
     const double rhoU = sol[o0], rhoV = sol[o1], rho = sol[o2], rhoE = sol[o3];
     const double u = rhoU / rho, v = rhoV / rho;
     const double ke = 0.5 * (rhoU * u + rhoV * v);
@@ -434,18 +551,19 @@ __global__ void k_euler_nodal(const double *__restrict__ sol, double *__restrict
 }
 
 // Euler boundary conditions (src/models/SELF_CompressibleIdealGas2D.f90:1217-1323)
+template <int PT, class Idx>
 __global__ void k_euler_bc(const double *__restrict__ solB, double *__restrict__ solE, const double *__restrict__ pSolB,
                            const double *__restrict__ primB, double *__restrict__ primE,
                            const double *__restrict__ pPrimB, const double *__restrict__ diagB,
                            double *__restrict__ diagE, const double *__restrict__ pDiagB,
                            const double *__restrict__ nHat, const int32_t *__restrict__ si, int N, int nEl) {
-  const size_t P = N + 1;
-  const size_t total = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t i = t % P, se = t / P;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx i = t % P, se = t / P;
     const int32_t *s = si + 5 * se;
     if (s[2] != 0) continue;
-    const size_t o[4] = {i + P * (4 * se), i + P * (1 + 4 * se), i + P * (2 + 4 * se), i + P * (3 + 4 * se)};
+    const Idx o[4] = {i + P * (4 * se), i + P * (1 + 4 * se), i + P * (2 + 4 * se), i + P * (3 + 4 * se)};
     if (s[4] == SELFAMD_BC_NONORMALFLOW) {
       const double nx = nHat[2 * t], ny = nHat[2 * t + 1];
       double u = solB[o[0]], v = solB[o[1]];
@@ -471,13 +589,14 @@ __global__ void k_euler_bc(const double *__restrict__ solB, double *__restrict__
 
 // Euler source, drag included (src/models/SELF_CompressibleIdealGas2D.f90:1325-1366;
 // quirk: the energy source is -rhou*gx - rhou*gy).
+template <int PT, class Idx>
 __global__ void k_euler_source(double *__restrict__ src, const double *__restrict__ sol, const double *__restrict__ env,
                                const double *__restrict__ envGrad, int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
     const double rhou = sol[o0], rhov = sol[o1], rho = sol[o2];
     const double gx = envGrad[2 * (node + PP * 2 * e)], gy = envGrad[2 * (node + PP * 2 * e) + 1];
     const double Cd = env[node + PP * (1 + 2 * e)];
@@ -489,13 +608,14 @@ __global__ void k_euler_source(double *__restrict__ src, const double *__restric
 }
 
 // Euler flux (src/models/SELF_CompressibleIdealGas2D.f90:1368-1440)
+template <int PT, class Idx>
 __global__ void k_euler_flux(double *__restrict__ flux, const double *__restrict__ sol, const double *__restrict__ prim,
                              const double *__restrict__ diag, int N, int nEl) {
-  const size_t PP = (size_t)(N + 1) * (N + 1);
-  const size_t total = PP * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t node = t % PP, e = t / PP;
-    const size_t o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
+  const Idx P = PT ? PT : N + 1, PP = P * P;
+  const Idx total = PP * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx node = t % PP, e = t / PP;
+    const Idx o0 = node + PP * 4 * e, o1 = o0 + PP, o2 = o1 + PP, o3 = o2 + PP;
     const double u = prim[o0], v = prim[o1], p = prim[o3], Hn = diag[o1];
     flux[2 * o0] = u * sol[o0] + p;
     flux[2 * o0 + 1] = v * sol[o0];
@@ -509,17 +629,18 @@ __global__ void k_euler_flux(double *__restrict__ flux, const double *__restrict
 }
 
 // Euler naive local Lax-Friedrichs flux (src/models/SELF_CompressibleIdealGas2D.f90:1455-1542)
+template <int PT, class Idx>
 __global__ void k_euler_riemann(double *__restrict__ fbn, const double *__restrict__ solB,
                                 const double *__restrict__ solE, const double *__restrict__ primB,
                                 const double *__restrict__ primE, const double *__restrict__ diagB,
                                 const double *__restrict__ diagE, const double *__restrict__ nHat,
                                 const double *__restrict__ nScale, int N, int nEl) {
-  const size_t P = N + 1;
-  const size_t total = P * 4 * nEl;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const size_t i = t % P, se = t / P;
+  const Idx P = PT ? PT : N + 1;
+  const Idx total = P * 4 * nEl;
+  for (Idx t = blockIdx.x * (Idx)blockDim.x + threadIdx.x; t < total; t += (Idx)gridDim.x * blockDim.x) {
+    const Idx i = t % P, se = t / P;
     const double nx = nHat[2 * t], ny = nHat[2 * t + 1], nmag = nScale[t];
-    const size_t o[4] = {i + P * (4 * se), i + P * (1 + 4 * se), i + P * (2 + 4 * se), i + P * (3 + 4 * se)};
+    const Idx o[4] = {i + P * (4 * se), i + P * (1 + 4 * se), i + P * (2 + 4 * se), i + P * (3 + 4 * se)};
     const double unL = primB[o[0]] * nx + primB[o[1]] * ny, unR = primE[o[0]] * nx + primE[o[1]] * ny;
     double fL[4], fR[4];
     fL[0] = unL * solB[o[0]] + primB[o[3]] * nx;
@@ -570,6 +691,69 @@ inline unsigned blocks_for(size_t n) {
 
 inline hipStream_t S(void *s) { return reinterpret_cast<hipStream_t>(s); }
 
+// Instance of a kernel<PT, Idx>: P = 2 .. 8 with 32-bit indices while every index (at most 8 per
+// work-item: a vector of four variables) stays below 2^32; else the runtime P and 64-bit indices.
+constexpr size_t kIndex32 = size_t(1) << 28;
+// one block per `perBlock` slabs: the grid's work-items must stay below 2^32
+inline bool slab_grid(size_t slabs, int perBlock) { return slabs <= (size_t)perBlock << 23; }
+#define LAUNCH_P(KERNEL, N, n, stream, ...)                                                             \
+  do {                                                                                                  \
+    const size_t n_ = (n);                                                                              \
+    switch (n_ < kIndex32 ? (N) + 1 : 0) {                                                              \
+      LAUNCH_P_CASE(KERNEL, 2, n_, stream, __VA_ARGS__) LAUNCH_P_CASE(KERNEL, 3, n_, stream, __VA_ARGS__) \
+      LAUNCH_P_CASE(KERNEL, 4, n_, stream, __VA_ARGS__) LAUNCH_P_CASE(KERNEL, 5, n_, stream, __VA_ARGS__) \
+      LAUNCH_P_CASE(KERNEL, 6, n_, stream, __VA_ARGS__) LAUNCH_P_CASE(KERNEL, 7, n_, stream, __VA_ARGS__) \
+      LAUNCH_P_CASE(KERNEL, 8, n_, stream, __VA_ARGS__)                                                 \
+      default:                                                                                          \
+        hipLaunchKernelGGL((KERNEL<0, size_t>), blocks_for(n_), kBlock, 0, S(stream), __VA_ARGS__);     \
+    }                                                                                                   \
+  } while (0)
+#define LAUNCH_P_CASE(KERNEL, PT, n, stream, ...) \
+  case PT: hipLaunchKernelGGL((KERNEL<PT, unsigned>), blocks_for(n), kBlock, 0, S(stream), __VA_ARGS__); break;
+
+template <int P, int NC>
+bool launch_interp_lds(const double *bM, const double *f, double *fb, int nVar, size_t slabs, hipStream_t st) {
+  constexpr int SPB = 256 / (4 * P * NC) > 0 ? 256 / (4 * P * NC) : 1;
+  if (!slab_grid(slabs, SPB)) return false;
+  hipLaunchKernelGGL((k_boundary_interp_lds<P, NC>), (unsigned)((slabs + SPB - 1) / SPB), 256, 0, st, bM, f, fb, nVar,
+                     (unsigned)slabs);
+  return true;
+}
+void launch_interp(const double *bM, const double *f, double *fb, int N, int nVar, int nEl, int ncomp, hipStream_t st) {
+  const size_t slabs = (size_t)nVar * nEl;
+  bool done = false;
+  switch (16 * (N + 1) + ncomp) {
+#define CASE(P)                                                                                   \
+  case 16 * P + 1: done = launch_interp_lds<P, 1>(bM, f, fb, nVar, slabs, st); break;             \
+  case 16 * P + 2: done = launch_interp_lds<P, 2>(bM, f, fb, nVar, slabs, st); break;             \
+  case 16 * P + 4: done = launch_interp_lds<P, 4>(bM, f, fb, nVar, slabs, st); break;
+    CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+  }
+  if (done) return;
+  const size_t n = (size_t)ncomp * (N + 1) * nVar * 4 * nEl;
+  hipLaunchKernelGGL(k_boundary_interp, blocks_for(n), kBlock, 0, st, bM, f, fb, N, nVar, nEl, ncomp);
+}
+template <bool WEAK>
+void launch_divergence(const double *dM, const double *bM, const double *qW, const double *f, const double *bF, double *dF,
+                       int N, int nVar, int nEl, hipStream_t st) {
+  const size_t slabs = (size_t)nVar * nEl;
+  switch (N + 1) {
+#define CASE(P)                                                                                                     \
+  case P: {                                                                                                         \
+    constexpr int SPB = 256 / (P * P);                                                                              \
+    if (!slab_grid(slabs, SPB)) break;                                                                              \
+    hipLaunchKernelGGL((k_divergence_lds<P, WEAK>), (unsigned)((slabs + SPB - 1) / SPB), 256, 0, st, dM, bM, qW, f, \
+                       bF, dF, nVar, (unsigned)slabs);                                                              \
+    return;                                                                                                         \
+  }
+    CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+  }
+  hipLaunchKernelGGL(k_divergence<WEAK>, blocks_for((size_t)(N + 1) * (N + 1) * slabs), kBlock, 0, st, dM, bM, qW, f, bF,
+                     dF, N, nVar, nEl);
+}
+
 #define CHECK_DIMS(N, nVar, nEl)                                                                  \
   SELFAMD_REQUIRE((N) >= 1 && (N) <= kMaxN && (nVar) >= 1 && (nEl) >= 1,                          \
                   "%s: bad sizes N=%d nVar=%d nEl=%d", __func__, (int)(N), (int)(nVar), (int)(nEl))
@@ -580,22 +764,19 @@ extern "C" {
 
 int selfamd_scalar_boundary_interp_2d(const double *bM, const double *f, double *fb, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
-  const size_t n = (size_t)(N + 1) * nVar * 4 * nEl;
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(n), kBlock, 0, S(s), bM, f, fb, N, nVar, nEl, 1);
+  launch_interp(bM, f, fb, N, nVar, nEl, 1, S(s));
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_vector_boundary_interp_2d(const double *bM, const double *f, double *fb, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
-  const size_t n = (size_t)2 * (N + 1) * nVar * 4 * nEl;
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(n), kBlock, 0, S(s), bM, f, fb, N, nVar, nEl, 2);
+  launch_interp(bM, f, fb, N, nVar, nEl, 2, S(s));
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_tensor_boundary_interp_2d(const double *bM, const double *f, double *fb, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
-  const size_t n = (size_t)4 * (N + 1) * nVar * 4 * nEl;
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(n), kBlock, 0, S(s), bM, f, fb, N, nVar, nEl, 4);
+  launch_interp(bM, f, fb, N, nVar, nEl, 4, S(s));
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -626,17 +807,14 @@ int selfamd_vector_gradient_2d(const double *dM, const double *f, double *g, int
 }
 int selfamd_vector_divergence_2d(const double *dM, const double *f, double *dF, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
-  const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_divergence<false>, blocks_for(n), kBlock, 0, S(s), dM, nullptr, nullptr, f, nullptr, dF, N,
-                     nVar, nEl);
+  launch_divergence<false>(dM, nullptr, nullptr, f, nullptr, dF, N, nVar, nEl, S(s));
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_vector_dg_divergence_2d(const double *dgM, const double *bM, const double *qW, const double *f,
                                     const double *bF, double *dF, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
-  const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_divergence<true>, blocks_for(n), kBlock, 0, S(s), dgM, bM, qW, f, bF, dF, N, nVar, nEl);
+  launch_divergence<true>(dgM, bM, qW, f, bF, dF, N, nVar, nEl, S(s));
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -651,7 +829,7 @@ int selfamd_side_exchange_scalar_2d(const double *b, double *ext, const int32_t 
                                     void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * nVar * 4 * nEl;
-  hipLaunchKernelGGL(k_side_exchange, blocks_for(n), kBlock, 0, S(s), b, ext, si, N, nVar, nEl, 1);
+  LAUNCH_P(k_side_exchange, N, n, s, b, ext, si, N, nVar, nEl, 1);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -659,7 +837,7 @@ int selfamd_side_exchange_vector_2d(const double *b, double *ext, const int32_t 
                                     void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)2 * (N + 1) * nVar * 4 * nEl;
-  hipLaunchKernelGGL(k_side_exchange, blocks_for(n), kBlock, 0, S(s), b, ext, si, N, nVar, nEl, 2);
+  LAUNCH_P(k_side_exchange, N, n, s, b, ext, si, N, nVar, nEl, 2);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -667,21 +845,21 @@ int selfamd_gradient_sf_2d(const double *dM, const double *dsdx, const double *J
                            int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_gradient_sf, blocks_for(n), kBlock, 0, S(s), dM, dsdx, J, f, gradF, N, nVar, nEl);
+  LAUNCH_P(k_gradient_sf, N, n, s, dM, dsdx, J, f, gradF, N, nVar, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_jacobian_weight_2d(const double *J, double *f, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_jacobian_weight, blocks_for(n), kBlock, 0, S(s), J, f, N, nVar, nEl);
+  LAUNCH_P(k_jacobian_weight, N, n, s, J, f, N, nVar, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_contravariant_projection_2d(const double *dsdx, double *f, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_contravariant_projection, blocks_for(n), kBlock, 0, S(s), dsdx, f, N, nVar, nEl);
+  LAUNCH_P(k_contravariant_projection, N, n, s, dsdx, f, N, nVar, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -689,7 +867,10 @@ int selfamd_update_grk(double *G, double *Sv, const double *dSdt, double a, doub
                        int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_update_grk, blocks_for(n), kBlock, 0, S(s), G, Sv, dSdt, a, g * dt, n);
+  if (aligned16(G) && aligned16(Sv) && aligned16(dSdt))
+    hipLaunchKernelGGL(k_update_grk<true>, blocks_for((n + 1) / 2), kBlock, 0, S(s), G, Sv, dSdt, a, g * dt, n);
+  else
+    hipLaunchKernelGGL(k_update_grk<false>, blocks_for(n), kBlock, 0, S(s), G, Sv, dSdt, a, g * dt, n);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -707,7 +888,10 @@ int selfamd_copy_f64(const double *src, double *dst, size_t n, void *s) {
 int selfamd_calculate_dsdt(const double *fd, const double *src, double *d, int N, int nVar, int nEl, void *s) {
   CHECK_DIMS(N, nVar, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nVar * nEl;
-  hipLaunchKernelGGL(k_dsdt, blocks_for(n), kBlock, 0, S(s), fd, src, d, n);
+  if (aligned16(fd) && aligned16(src) && aligned16(d))
+    hipLaunchKernelGGL(k_dsdt<true>, blocks_for((n + 1) / 2), kBlock, 0, S(s), fd, src, d, n);
+  else
+    hipLaunchKernelGGL(k_dsdt<false>, blocks_for(n), kBlock, 0, S(s), fd, src, d, n);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -736,13 +920,13 @@ int selfamd_semquad_generate(int N, int ctrl, int nGeo, int nEl, const double *n
   SELFAMD_HIP(hipMemcpyAsync(d_bM, mbM, sizeof(double) * 2 * P, hipMemcpyHostToDevice, st));
   const size_t nn = (size_t)P * P * nEl, nb = (size_t)P * 4 * nEl;
   hipLaunchKernelGGL(k_grid_interp, blocks_for(2 * nn), kBlock, 0, st, d_iM, nodeCoords, x, nGeo, N, 1, nEl, 2);
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(2 * nb), kBlock, 0, st, d_bM, x, xb, N, 1, nEl, 2);
+  launch_interp(d_bM, x, xb, N, 1, nEl, 2, st);
   hipLaunchKernelGGL(k_vector_gradient, blocks_for(nn), kBlock, 0, st, d_dM, x, dxds, N, 1, nEl);
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(4 * nb), kBlock, 0, st, d_bM, dxds, dxdsb, N, 1, nEl, 4);
+  launch_interp(d_bM, dxds, dxdsb, N, 1, nEl, 4, st);
   hipLaunchKernelGGL(k_determinant, blocks_for(nn), kBlock, 0, st, dxds, J, nn);
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(nb), kBlock, 0, st, d_bM, J, Jb, N, 1, nEl, 1);
+  launch_interp(d_bM, J, Jb, N, 1, nEl, 1, st);
   hipLaunchKernelGGL(k_dsdx_from_dxds, blocks_for(nn), kBlock, 0, st, dxds, dsdx, nn);
-  hipLaunchKernelGGL(k_boundary_interp, blocks_for(4 * nb), kBlock, 0, st, d_bM, dsdx, dsdxb, N, 1, nEl, 4);
+  launch_interp(d_bM, dsdx, dsdxb, N, 1, nEl, 4, st);
   hipLaunchKernelGGL(k_geom_normals, blocks_for(nb), kBlock, 0, st, dsdxb, Jb, nHatb, nScaleb, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   SELFAMD_HIP(hipStreamSynchronize(st));
@@ -753,7 +937,7 @@ int selfamd_semquad_generate(int N, int ctrl, int nGeo, int nEl, const double *n
 int selfamd_sw2d_velocity(const double *sol, const double *solB, double *vel, double *velB, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl + (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_sw_velocity, blocks_for(n), kBlock, 0, S(s), sol, solB, vel, velB, N, nEl);
+  LAUNCH_P(k_sw_velocity, N, n, s, sol, solB, vel, velB, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -761,7 +945,7 @@ int selfamd_sw2d_set_boundary_condition(const double *solB, double *solE, const 
                                         const int32_t *si, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_sw_bc, blocks_for(n), kBlock, 0, S(s), solB, solE, topoB, nHat, si, N, nEl, 2);
+  LAUNCH_P(k_sw_bc, N, n, s, solB, solE, topoB, nHat, si, N, nEl, 2);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -769,14 +953,14 @@ int selfamd_sw2d_source(double *src, const double *sol, const double *gradH, dou
                         void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_sw_source, blocks_for(n), kBlock, 0, S(s), src, sol, gradH, g, f, N, nEl);
+  LAUNCH_P(k_sw_source, N, n, s, src, sol, gradH, g, f, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_sw2d_flux(double *flux, const double *sol, const double *vel, double g, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_sw_flux, blocks_for(n), kBlock, 0, S(s), flux, sol, vel, g, N, nEl);
+  LAUNCH_P(k_sw_flux, N, n, s, flux, sol, vel, g, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -784,7 +968,7 @@ int selfamd_sw2d_riemann(double *fbn, const double *solB, const double *solE, co
                          const double *nHat, const double *nScale, double g, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_sw_riemann, blocks_for(n), kBlock, 0, S(s), fbn, solB, solE, velB, velE, nHat, nScale, g, N,
+  LAUNCH_P(k_sw_riemann, N, n, s, fbn, solB, solE, velB, velE, nHat, nScale, g, N,
                      nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
@@ -793,21 +977,21 @@ int selfamd_lsw2d_set_boundary_condition(const double *solB, double *solE, const
                                          int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_sw_bc, blocks_for(n), kBlock, 0, S(s), solB, solE, nullptr, nHat, si, N, nEl, 1);
+  LAUNCH_P(k_sw_bc, N, n, s, solB, solE, nullptr, nHat, si, N, nEl, 1);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_lsw2d_source(double *src, const double *sol, const double *fc, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_lsw_source, blocks_for(n), kBlock, 0, S(s), src, sol, fc, N, nEl);
+  LAUNCH_P(k_lsw_source, N, n, s, src, sol, fc, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_lsw2d_flux(double *flux, const double *sol, const double *H, double g, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_lsw_flux, blocks_for(n), kBlock, 0, S(s), flux, sol, H, g, N, nEl);
+  LAUNCH_P(k_lsw_flux, N, n, s, flux, sol, H, g, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -815,28 +999,28 @@ int selfamd_lsw2d_riemann(double *fbn, const double *solB, const double *solE, c
                           const double *nScale, double g, int N, int nEl, void *s) {
   CHECK_DIMS(N, 3, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_lsw_riemann, blocks_for(n), kBlock, 0, S(s), fbn, solB, solE, Hb, nHat, nScale, g, N, nEl);
+  LAUNCH_P(k_lsw_riemann, N, n, s, fbn, solB, solE, Hb, nHat, nScale, g, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_euler2d_diagnostics(const double *sol, double *diag, double gam, double R, int N, int nEl, void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_euler_nodal, blocks_for(n), kBlock, 0, S(s), sol, diag, gam, R, N, nEl, 0);
+  LAUNCH_P(k_euler_nodal, N, n, s, sol, diag, gam, R, N, nEl, 0);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_euler2d_primitive(const double *sol, double *prim, double gam, int N, int nEl, void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_euler_nodal, blocks_for(n), kBlock, 0, S(s), sol, prim, gam, 1.0, N, nEl, 1);
+  LAUNCH_P(k_euler_nodal, N, n, s, sol, prim, gam, 1.0, N, nEl, 1);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
 int selfamd_euler2d_entropy_vars(const double *sol, double *ent, double gam, int N, int nEl, void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_euler_nodal, blocks_for(n), kBlock, 0, S(s), sol, ent, gam, 1.0, N, nEl, 2);
+  LAUNCH_P(k_euler_nodal, N, n, s, sol, ent, gam, 1.0, N, nEl, 2);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -846,7 +1030,7 @@ int selfamd_euler2d_set_boundary_condition(const double *solB, double *solE, con
                                            void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_euler_bc, blocks_for(n), kBlock, 0, S(s), solB, solE, pSolB, primB, primE, pPrimB, diagB, diagE,
+  LAUNCH_P(k_euler_bc, N, n, s, solB, solE, pSolB, primB, primE, pPrimB, diagB, diagE,
                      pDiagB, nHat, si, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
@@ -855,7 +1039,7 @@ int selfamd_euler2d_source(double *src, const double *sol, const double *env, co
                            void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_euler_source, blocks_for(n), kBlock, 0, S(s), src, sol, env, envGrad, N, nEl);
+  LAUNCH_P(k_euler_source, N, n, s, src, sol, env, envGrad, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -863,7 +1047,7 @@ int selfamd_euler2d_flux(double *flux, const double *sol, const double *prim, co
                          void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * (N + 1) * nEl;
-  hipLaunchKernelGGL(k_euler_flux, blocks_for(n), kBlock, 0, S(s), flux, sol, prim, diag, N, nEl);
+  LAUNCH_P(k_euler_flux, N, n, s, flux, sol, prim, diag, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
 }
@@ -872,7 +1056,7 @@ int selfamd_euler2d_riemann(double *fbn, const double *solB, const double *solE,
                             const double *nScale, int N, int nEl, void *s) {
   CHECK_DIMS(N, 4, nEl);
   const size_t n = (size_t)(N + 1) * 4 * nEl;
-  hipLaunchKernelGGL(k_euler_riemann, blocks_for(n), kBlock, 0, S(s), fbn, solB, solE, primB, primE, diagB, diagE,
+  LAUNCH_P(k_euler_riemann, N, n, s, fbn, solB, solE, primB, primE, diagB, diagE,
                      nHat, nScale, N, nEl);
   SELFAMD_CHECK_LAUNCH();
   return kOk;
