@@ -64,7 +64,7 @@ int selfamd_device_count(int *count);
 int selfamd_device_name(int device, char *name, int len);
 int selfamd_malloc(void **ptr, size_t bytes);
 int selfamd_free(void *ptr);
-/* kind: 1 host->device, 2 device->host, 3 device->device (synchronous) */
+/* kind: 1 host->device, 2 device->host, 3 device->device (complete when it returns) */
 int selfamd_memcpy(void *dst, const void *src, size_t bytes, int kind);
 int selfamd_memset(void *ptr, int value, size_t bytes);
 int selfamd_device_synchronize(void);

@@ -837,6 +837,7 @@ int selfamd_mlp_set_params(selfamd_mlp *m, const float *host) {
   SELFAMD_HIP(hipMemcpy(m->params, host, 4 * m->nParams, hipMemcpyHostToDevice));
   SELFAMD_HIP(hipMemset(m->m1, 0, 4 * m->nParams));
   SELFAMD_HIP(hipMemset(m->m2, 0, 4 * m->nParams));
+  SELFAMD_HIP(hipStreamSynchronize(nullptr));  // the models' streams do not wait for the null stream
   return kOk;
 }
 

@@ -42,6 +42,10 @@ int selfamd_memcpy(void *dst, const void *src, size_t bytes, int kind) {
   SELFAMD_REQUIRE(dst && src, "memcpy: null pointer");
   const hipMemcpyKind k = kind == 1 ? hipMemcpyHostToDevice : kind == 2 ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
   SELFAMD_HIP(hipMemcpy(dst, src, bytes, k));
+  // The runtime may return from a copy whose target is device memory before the copy has landed.
+  // The models' streams do not wait for the null stream, so a copy that they make of dst next
+  // (set_solution, set_static) would read what the memory held before.
+  if (kind != 2) SELFAMD_HIP(hipStreamSynchronize(nullptr));
   return kOk;
 }
 
@@ -49,6 +53,7 @@ int selfamd_memset(void *ptr, int value, size_t bytes) {
   if (!bytes) return kOk;
   SELFAMD_REQUIRE(ptr, "memset: null pointer");
   SELFAMD_HIP(hipMemset(ptr, value, bytes));
+  SELFAMD_HIP(hipStreamSynchronize(nullptr));  // as in selfamd_memcpy
   return kOk;
 }
 

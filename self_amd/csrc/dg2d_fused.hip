@@ -1575,6 +1575,7 @@ int selfamd_model2d_create(selfamd_model2d **out, int kind, int N, int nEl, cons
       hipMemsetAsync(m->trace[1], 0, sizeof(double) * nT, m->stream) != hipSuccess ||
       (m->un[0] && hipMemsetAsync(m->un[0], 0, sizeof(double) * 2 * (size_t)P * 4 * nEl, m->stream) != hipSuccess) ||
       (m->un[1] && hipMemsetAsync(m->un[1], 0, sizeof(double) * 2 * (size_t)P * 4 * nEl, m->stream) != hipSuccess) ||
+      hipStreamSynchronize(nullptr) != hipSuccess ||  // copies into device memory may still be under way
       hipStreamSynchronize(m->stream) != hipSuccess) {
     set_error("model2d_create: device initialisation failed");
     return fail(kHipError);
@@ -1934,7 +1935,8 @@ int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const floa
   ok = ok && hipMemcpy(c->inMean, inMean, 4 * nIn, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(c->inScale, inScale, 4 * nIn, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(c->outMean, outMean, 4 * nOut, hipMemcpyHostToDevice) == hipSuccess &&
-       hipMemcpy(c->outScale, outScale, 4 * nOut, hipMemcpyHostToDevice) == hipSuccess;
+       hipMemcpy(c->outScale, outScale, 4 * nOut, hipMemcpyHostToDevice) == hipSuccess &&
+       hipStreamSynchronize(nullptr) == hipSuccess;
   if (!ok) {
     free_closure(c);
     set_error("model2d_set_closure: device allocation or copy failed");
@@ -2061,6 +2063,7 @@ int selfamd_model2d_set_bands(selfamd_model2d *m, int nBands) {
   for (int e = 0; e < nEl; e++) order[fill[bandOf[level[e]]]++] = e;  // by band, then element index
   SELFAMD_HIP(hipMalloc(&m->bandElems, sizeof(int32_t) * nEl));
   SELFAMD_HIP(hipMemcpy(m->bandElems, order.data(), sizeof(int32_t) * nEl, hipMemcpyHostToDevice));
+  SELFAMD_HIP(hipStreamSynchronize(nullptr));
   m->bandStart = start;
   m->nBands = nBands;
   return kOk;
@@ -2406,6 +2409,8 @@ int selfamd_batch_create(selfamd_batch **out, int nModels, selfamd_model2d *cons
       if (e) return fail("copy failed");
     }
   }
+  // copies into device memory may still be under way, and the batch's stream would not wait for them
+  if (hipStreamSynchronize(nullptr) != hipSuccess) return fail("copy failed");
   if (b->capture() != hipSuccess) return fail("stage graph capture failed");
   *out = b;
   return kOk;
