@@ -41,6 +41,10 @@ constexpr int kNbrOrphan = -0x40000000;
 // forward_step calls of at most this many steps with a step size other than the captured
 // graphs' are launched stage by stage instead of recapturing
 constexpr int kDirectSteps = 2;
+// Calls of at least kResidentSteps steps take a resident launch where the mesh allows it, single
+// steps from kResidentElements elements on: below, a cooperative launch of three stages costs what
+// it saves (N = 7: 28.8 against 28.3 us per call at 10^2 elements, 31.9 against 34.1 at 40^2).
+constexpr int kResidentSteps = 2, kResidentElements = 1024;
 
 // Williamson low-storage RK3 (src/SELF_Model.f90:25-27)
 constexpr double kRk3A[3] = {0.0, -5.0 / 9.0, -153.0 / 128.0};
@@ -1008,6 +1012,419 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 }
 
 // ------------------------------------------------------------------------------
+// Resident stepping: all RK stages of a call in one launch, for meshes that fit the device
+// ------------------------------------------------------------------------------
+// What bounds a small mesh is not the arithmetic but what comes once per stage: the launch (1.3 us,
+// with the write-back of the stage's dirty L2 lines up to 4 us), reloading state, metrics and
+// matrices (0.8 to 2 us before the first instruction that needs them), and interpolating own traces
+// that the previous stage had.  When every block can be resident at once, one cooperative launch
+// keeps the state, RK register, metrics, normals and the constant source gradient in registers and
+// exchanges only face traces:
+//   per stage  node lanes: volume flux -> LDS; face lanes: the neighbours' traces, boundary
+//              conditions, Riemann flux -> LDS; node lanes: divergence, update; face lanes: traces
+//              of the new state -> registers and the exchange ring.
+// The arithmetic and its order are the stage kernel's, so the results are the same bits.
+// Measured per stage (200-step and 24-step calls): linear SW 10^2 N = 7 4.1 -> 2.2 us, 45 x 37 N = 6
+// 8.6 -> 3.0 us, Euler 93 x 61 N = 4 19 -> 9 us.  Instances: WPE = 1 leaves the registers to the
+// compiler and unrolls the divergence; where the mesh needs more blocks than fit that way, 3 or 4
+// wavefronts per SIMD (twice the elements).
+//
+// Exchange: ring buffer m mod 3 takes stage m's traces (and lagged velocities).  Every value is its
+// own flag: a slot holds kEmpty, a signalling NaN that no arithmetic produces, until its owner
+// stores the value, with relaxed agent-scope atomics on both sides; the reader polls its own
+// values.  Face nodes are paired one to one: this lane reads the slots of lane L', and L' reads
+// this lane's.  At stage m, L' has stored its traces of stage m - 1, so it has read this lane's of
+// stage m - 2, and this lane empties those slots; the stores are complete (vmcnt 0) before this
+// lane stores its traces of stage m, which L' must have seen before it polls the emptied slots
+// again (for stage m + 1).  A call has a multiple of three stages and the last one stores to the
+// trace buffers instead, so the next call finds the slots of its stage -2 filled and empties them
+// first, and all others empty.
+//
+// All blocks must be resident: the launch is cooperative, which the runtime refuses if they
+// cannot be.  Every wait is bounded as well: a lane that has polled kPollBudget times in a call
+// stops waiting and raises `timedOut`, which the next synchronising call reports.
+constexpr unsigned long long kEmpty = 0x7FF0DEAD7FF0DEADull;
+constexpr int kPollBudget = 1 << 20;
+
+struct ResidentArgs {
+  unsigned long long *ring;  // 3 buffers (0:N, NX, 4, nEl)
+  int stages;                // 3 per step
+  double rkA[3], rkGdt[3];   // a_m, g_m dt
+  int *timedOut;             // host memory
+};
+
+template <class Phys, int N, bool NODAL>
+struct ResidentTile {
+  static constexpr int NP = N + 1, NN = NP * NP, NF = 4 * NP;
+  // one wavefront per block, so that no phase boundary is a block barrier, except at N = 5, where
+  // a wavefront would hold a single element on 36 of its lanes
+  static constexpr int T = N == 5 ? 128 : 64;
+  static constexpr int EPB = T / NN < T / NF ? T / NN : T / NF;
+  static constexpr bool WAVE = T == 64;
+  static constexpr bool SPLIT = N >= 6;  // the face sums of the stage kernel's tiles
+  static constexpr int NV = Phys::NV, NT = Phys::NT, NX = NT + (Phys::kLag ? (NODAL ? 2 : 1) : 0);
+  static constexpr int MRS = NP % 8 == 0 ? NP + 2 : NP, NNS = NP == 6 ? NN + 2 : NN;
+  static constexpr int even(int n) { return (n + 1) & ~1; }
+  // LDS in doubles; the static field and its metric products (prologue only) lie over BF and F1, F2
+  static constexpr int Q = 0, F1 = Q + even(NT * EPB * NNS), F2 = F1 + even(NV * EPB * NNS);
+  static constexpr int BF = F2 + even(NV * EPB * NNS), M = BF + even(NV * EPB * NF);
+  // affine metrics of the block's elements (scalar registers instead where a wavefront is one)
+  static constexpr int REC = M + even(2 * NP * MRS + 4 * NP), RECS = NODAL || NN == 64 ? 0 : 6 * EPB;
+  // The tile's packets, staged so that the ring is written in whole lines (at N = 7 every store is
+  // one; in runs of 8 (N + 1) bytes Euler 60^2 N = 1 took 11.7 us per stage, 4 us in lines): over F1
+  // and F2 where they fit and no other wavefront uses those
+  static constexpr bool STAGED = NP != 8;
+  static constexpr int PKS = STAGED ? EPB * NF * NX : 0, PKOVER = WAVE && PKS <= F2 + even(NV * EPB * NNS) - F1;
+  static constexpr int PK = PKOVER ? F1 : REC + RECS;
+  static constexpr int SIZE = REC + RECS + (PKOVER ? 0 : even(PKS));
+  static_assert(NNS <= NV * NF && F2 + even(NV * EPB * NNS) - F1 >= 4 * EPB * NNS, "prologue arrays do not fit");
+};
+
+__device__ inline unsigned long long ring_load(const unsigned long long *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void ring_store(unsigned long long *p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void k_ring_fill(unsigned long long *ring, size_t n) {
+  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
+    ring[t] = kEmpty;
+}
+
+template <class Phys, int N, bool NODAL, int WPE>
+__global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_resident(const FusedArgs a, const ResidentArgs ra) {
+  using L = ResidentTile<Phys, N, NODAL>;
+  constexpr int NP = L::NP, NN = L::NN, NF = L::NF, T = L::T, EPB = L::EPB, NV = L::NV, NT = L::NT, NX = L::NX;
+  constexpr int MRS = L::MRS, NNS = L::NNS;
+  constexpr bool SPLIT = L::SPLIT, WAVE = L::WAVE, SWZ = NP == 8;
+  constexpr bool USE_AUX = Phys::kAuxGrad || Phys::kAuxTrace, GRAD = Phys::kAuxGrad, GRADN = NODAL && GRAD;
+  __shared__ __align__(16) double lds[L::SIZE];
+  auto slot = [](int i_, int j_) { return SWZ ? NP * j_ + (i_ ^ (j_ & 6)) : i_ + NP * j_; };
+  auto sQ = reinterpret_cast<double (*)[EPB][NNS]>(lds + L::Q);
+  auto sF1 = reinterpret_cast<double (*)[EPB][NNS]>(lds + L::F1);
+  auto sF2 = reinterpret_cast<double (*)[EPB][NNS]>(lds + L::F2);
+  auto sBF = reinterpret_cast<double (*)[EPB][NF]>(lds + L::BF);
+  auto sAux = reinterpret_cast<double (*)[NNS]>(lds + L::BF);
+  auto sGb = reinterpret_cast<double (*)[EPB][NNS]>(lds + L::F1);
+  double *sM = lds + L::M;
+  const double *dgM = sM, *Dm = sM + NP * MRS, *bM0 = sM + 2 * NP * MRS, *bM1 = bM0 + NP, *qW = bM1 + NP;
+  const int tid = threadIdx.x;
+
+  // ---- lanes: nodes, and face nodes as in the stage kernel ----
+  const int el = tid / NN, node = tid % NN, i = node % NP, j = node / NP, nl = slot(i, j);
+  int e = blockIdx.x * EPB + el;
+  bool nodeActive = el < EPB && e < a.nEl;
+  if constexpr (NN == 64) {
+    e = __builtin_amdgcn_readfirstlane(e);
+    nodeActive = __builtin_amdgcn_readfirstlane((int)nodeActive) != 0;
+  }
+  const int fhalf = SPLIT ? tid >> 5 : 0, fslot = SPLIT ? tid & 31 : tid;
+  const int fel = fslot / NF, fslotN = fslot % NF;
+  const int side = SPLIT ? ((fslotN / NP) >> 1 | ((fslotN / NP) & 1) << 1) : fslotN / NP;
+  const int fi = fslotN % NP, fnode = side * NP + fi, fe = blockIdx.x * EPB + fel;
+  const bool faceActive = fel < EPB && fe < a.nEl && (!SPLIT || fslot < NF);
+  const bool faceOwner = faceActive && fhalf == 0;  // the lane of a pair that has the face node
+  const bool alongJ = side == 0 || side == 2;
+  constexpr int FH0 = NP / 2, FHN = NP - FH0;
+
+  for (int k = tid; k < 2 * NN + 4 * NP; k += T) {
+    const int r = k % NN;
+    sM[k < 2 * NN ? (k / NN) * NP * MRS + (r / NP) * MRS + r % NP : 2 * NP * MRS + k - 2 * NN] = a.mats[k];
+  }
+
+  // ---- prologue: everything that stays in registers ----
+  const size_t sBase = (size_t)e * NV * NN, nodeAt = nodeActive ? (size_t)e * NN + node : (size_t)node;
+  double s[NV], g[NV], auxVal = a.p.auxConst, statVal = a.p.stat2Const, dsdx[4] = {0, 0, 0, 0}, invJ = 1.0;
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    s[v] = a.S[(nodeActive ? sBase + node : (size_t)node) + (size_t)v * NN];
+    g[v] = 0.0;
+  }
+  if (USE_AUX && a.aux) auxVal = a.aux[nodeAt];
+  if (a.stat2) statVal = a.stat2[nodeAt];
+  if constexpr (NODAL) {
+    const double *gn = a.ndsdx + 4 * nodeAt;
+    dsdx[0] = gn[0]; dsdx[1] = gn[1]; dsdx[2] = gn[2]; dsdx[3] = gn[3];
+    invJ = 1.0 / a.nJ[nodeAt];
+  } else {
+    const double *gr = a.geom + (nodeActive ? (size_t)e : 0) * kGeomStride;
+    dsdx[0] = gr[0]; dsdx[1] = gr[1]; dsdx[2] = gr[2]; dsdx[3] = gr[3];
+    invJ = gr[6];
+  }
+  int code = kNbrOrphan;
+  double nx = 0.0, ny = 0.0, nmag = 0.0, unL = 0.0, unR = 0.0, qL[NT], qR[NT];
+  unsigned mine = 0, theirs = 0;  // slots of this lane and of the lane it reads, within a ring buffer
+  const unsigned ringLen = NP * NX * 4 * (unsigned)a.nEl;  // resident meshes are small
+  if (faceOwner) {
+    code = a.nbr[4 * (size_t)fe + side];
+    const size_t fb = (size_t)fi + NP * (side + 4 * (size_t)fe);
+    if constexpr (NODAL) {
+      nx = a.nnHat[2 * fb]; ny = a.nnHat[2 * fb + 1]; nmag = a.nnScale[fb];
+    } else {
+      const double *gr = a.geom + (size_t)fe * kGeomStride;
+      nx = gr[8 + side]; ny = gr[12 + side]; nmag = gr[16 + side];
+    }
+    mine = fi + NP * NX * (side + 4 * (unsigned)fe);
+    // stage 0 reads the previous launch's traces and lagged velocities
+    if (code >= 0) {
+      const int s2 = (code >> 1) & 3, fi2 = (code & 1) ? N - fi : fi;
+      const size_t e2 = (size_t)(code >> 3), nb = (size_t)fi2 + NP * (s2 + 4 * e2);
+      const double *tr = a.traceIn + (size_t)fi2 + NP * (size_t)NT * (s2 + 4 * e2);
+#pragma unroll
+      for (int k = 0; k < NT; k++) qR[k] = tr[(size_t)k * NP];
+      if (Phys::kLag) unR = lag_outer_raw<NODAL>(a.unIn, nb, nx, ny);
+      theirs = fi2 + NP * NX * (s2 + 4 * (unsigned)e2);
+    }
+    if (Phys::kLag) unL = lag_own<NODAL>(a.unIn, fb, nx, ny);
+  }
+  if (nodeActive) {
+    double q[NT];
+    phys_nodal<Phys>(s, a.p, q);
+#pragma unroll
+    for (int k = 0; k < NT; k++) sQ[k][el][nl] = q[k];
+    if (USE_AUX) sAux[el][nl] = auxVal;
+    if constexpr (GRADN) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) sGb[k][el][nl] = auxVal * dsdx[k];
+    }
+  }
+  __syncthreads();
+  // GradientSF of the static field (constant over the call) and its trace
+  double gx = 0.0, gy = 0.0;
+  if (GRAD && a.aux && nodeActive) {
+    double dxi = 0.0, deta = 0.0;
+    for (int ii = 0; ii < NP; ii++) {
+      const double di = Dm[ii + MRS * i], dj = Dm[ii + MRS * j];
+      if constexpr (GRADN) {
+        gx = gx + di * sGb[0][el][slot(ii, j)] + dj * sGb[2][el][slot(i, ii)];
+        gy = gy + di * sGb[1][el][slot(ii, j)] + dj * sGb[3][el][slot(i, ii)];
+      } else {
+        dxi = dxi + di * sAux[el][slot(ii, j)];
+        deta = deta + dj * sAux[el][slot(i, ii)];
+      }
+    }
+    if constexpr (!GRADN) {
+      gx = dsdx[0] * dxi + dsdx[2] * deta;
+      gy = dsdx[1] * dxi + dsdx[3] * deta;
+    }
+    gx = gx * invJ;
+    gy = gy * invJ;
+  }
+  // sums over this lane's face line (its half of it, added across the pair): out[k] += b(ii) at(k, node)
+  auto face_line = [&](auto count, auto at, double *out) {
+    constexpr int K = decltype(count)::value;
+    const double *bm = (side == 1 || side == 2) ? bM1 : bM0;
+#pragma unroll
+    for (int k = 0; k < K; k++) out[k] = 0.0;
+    if constexpr (SPLIT) {
+      const int lo = fhalf ? FH0 : 0;
+#pragma unroll
+      for (int t = 0; t < FHN; t++) {
+        const int ii = lo + t;
+        if (fhalf == 0 && t >= FH0) break;
+        const int nd = alongJ ? slot(fi, ii) : slot(ii, fi);
+#pragma unroll
+        for (int k = 0; k < K; k++) out[k] += bm[ii] * at(k, nd);
+      }
+#pragma unroll
+      for (int k = 0; k < K; k++) out[k] = pair_sum32(out[k]);
+    } else {
+#pragma unroll
+      for (int ii = 0; ii < NP; ii++) {
+        const int nd = alongJ ? slot(fi, ii) : slot(ii, fi);
+#pragma unroll
+        for (int k = 0; k < K; k++) out[k] += bm[ii] * at(k, nd);
+      }
+    }
+  };
+  using CountT = std::integral_constant<int, NT>;
+  using Count1 = std::integral_constant<int, 1>;
+  double auxB = a.p.auxConst;
+  if (faceActive) {
+    if (Phys::kAuxTrace && a.aux && (Phys::kAuxTraceInFlux || a.anyBoundary))
+      face_line(Count1{}, [&](int, int nd) { return sAux[fel][nd]; }, &auxB);
+    face_line(CountT{}, [&](int k, int nd) { return sQ[k][fel][nd]; }, qL);
+  }
+  __syncthreads();  // the prologue's arrays are overwritten from here on
+  // affine metrics come from LDS at each use rather than from 10 registers held throughout
+  double *rec = lds + L::REC + 6 * (el < EPB ? el : 0);
+  if constexpr (L::RECS > 0) {
+    if (nodeActive && node == 0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) rec[k] = dsdx[k];
+      rec[4] = invJ;
+    }
+    __syncthreads();
+  }
+
+  // ---- stages ----
+  const unsigned tileAt = blockIdx.x * (unsigned)(EPB * NF * NX);
+  const int tileSlots = min(EPB, a.nEl - (int)blockIdx.x * EPB) * NF * NX;
+  int budget = kPollBudget, fill = 0;  // fill: m mod 3
+#pragma unroll 1
+  for (int m = 0; m < ra.stages; m++) {
+    const bool last = m == ra.stages - 1;
+    const int before = fill == 0 ? 2 : fill - 1, empty = fill == 2 ? 0 : fill + 1;  // (m - 1), (m - 2) mod 3
+    if (nodeActive) {
+      double fx[NV], fy[NV], q[NT];
+      Phys::volume(s, auxVal, a.p, fx, fy, q);
+      if constexpr (L::RECS > 0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) dsdx[k] = rec[k];
+      }
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        sF1[v][el][nl] = dsdx[0] * fx[v] + dsdx[1] * fy[v];
+        sF2[v][el][nl] = dsdx[2] * fx[v] + dsdx[3] * fy[v];
+      }
+    }
+    double lag0 = 0.0, lag1 = 0.0;  // this stage's own face velocity, for the next one
+    if (faceOwner) {
+      if (code >= 0 && m > 0) {
+        const unsigned long long *p = ra.ring + (size_t)before * ringLen + theirs;
+        unsigned long long x[NX];
+        for (;;) {
+          bool ok = true;
+#pragma unroll
+          for (int k = 0; k < NX; k++) x[k] = ring_load(p + k * NP);
+#pragma unroll
+          for (int k = 0; k < NX; k++) ok = ok && x[k] != kEmpty;
+          if (ok || --budget < 0) break;
+        }
+#pragma unroll
+        for (int k = 0; k < NT; k++) qR[k] = __longlong_as_double((long long)x[k]);
+        if constexpr (Phys::kLag) {
+          const double u = __longlong_as_double((long long)x[NT]);
+          if constexpr (NODAL) unR = u * nx + __longlong_as_double((long long)x[NX - 1]) * ny;
+          else unR = u;
+        }
+      } else if (code < 0) {
+        if (code == kNbrOrphan) {
+#pragma unroll
+          for (int k = 0; k < NT; k++) qR[k] = 0.0;
+        } else {
+          const double *pres = a.presTrace ? a.presTrace + (size_t)fi + NP * (size_t)NT * (side + 4 * (size_t)fe) : nullptr;
+          double pv[NT];
+#pragma unroll
+          for (int k = 0; k < NT; k++) pv[k] = pres ? pres[(size_t)k * NP] : 0.0;
+          Phys::bc(qL, auxB, nx, ny, -code - 1, pv, pres != nullptr, qR);
+        }
+      }
+      if (!L::STAGED && code >= 0) {
+#pragma unroll
+        for (int k = 0; k < NX; k++) ring_store(ra.ring + (size_t)empty * ringLen + mine + k * NP, kEmpty);
+      }
+      if constexpr (Phys::kLag) {
+        const double invH = 1.0 / qL[2];
+        if constexpr (NODAL) {
+          lag0 = qL[0] * invH;
+          lag1 = qL[1] * invH;
+        } else {
+          lag0 = (qL[0] * invH) * nx + (qL[1] * invH) * ny;
+        }
+      }
+      double fstar[NV];
+      Phys::riemann(qL, qR, nx, ny, nmag, auxB, unL, outer_un<NODAL>(unR), a.p, fstar);
+#pragma unroll
+      for (int v = 0; v < NV; v++) sBF[v][fel][fnode] = fstar[v];
+    }
+    phase_sync<WAVE>();
+    if constexpr (L::STAGED)  // every lane of the tile has its neighbour's traces
+      for (int k = tid; k < tileSlots; k += T) ring_store(ra.ring + (size_t)empty * ringLen + tileAt + k, kEmpty);
+
+    if (nodeActive) {
+      double dxs[NV], des[NV];
+#pragma unroll
+      for (int v = 0; v < NV; v++) { dxs[v] = 0.0; des[v] = 0.0; }
+      auto line = [&](int ii) {
+        const double ai = dgM[ii + MRS * i], aj = dgM[ii + MRS * j];
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+          dxs[v] = dxs[v] + ai * sF1[v][el][slot(ii, j)];
+          des[v] = des[v] + aj * sF2[v][el][slot(i, ii)];
+        }
+      };
+      if constexpr (WPE == 1) {
+#pragma unroll
+        for (int ii = 0; ii < NP; ii++) line(ii);
+      } else {
+#pragma unroll 2
+        for (int ii = 0; ii < NP; ii++) line(ii);
+      }
+      double src[NV];
+      Phys::source(s, gx, gy, statVal, a.p, src);
+      const double rkA = ra.rkA[fill], gdt = ra.rkGdt[fill];
+      const double iwi = qW[NP + i], iwj = qW[NP + j];
+      const double bi1 = bM1[i], bi0 = bM0[i], bj1 = bM1[j], bj0 = bM0[j];
+      if constexpr (L::RECS > 0) invJ = rec[4];
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        double d = dxs[v] + des[v];
+        d = d + (bi1 * sBF[v][el][NP + j] + bi0 * sBF[v][el][3 * NP + j]) * iwi +
+            (bj1 * sBF[v][el][2 * NP + i] + bj0 * sBF[v][el][i]) * iwj;
+        d = d * invJ;
+        const double dsdt = src[v] - d;
+        g[v] = rkA * (fill == 0 ? 0.0 : g[v]) + dsdt;
+        s[v] = s[v] + gdt * g[v];
+        // the RK register that the last step's second stage leaves behind
+        if (m == ra.stages - 2) a.G[sBase + (size_t)v * NN + node] = g[v];
+      }
+      double q[NT];
+      phys_nodal<Phys>(s, a.p, q);
+#pragma unroll
+      for (int k = 0; k < NT; k++) sQ[k][el][nl] = q[k];
+    }
+    phase_sync<WAVE>();
+
+    if (faceActive) {
+      face_line(CountT{}, [&](int k, int nd) { return sQ[k][fel][nd]; }, qL);
+      if (fhalf == 0) {
+        if (!last) {
+          if constexpr (L::STAGED) {
+            double *p = lds + L::PK + fi + NP * NX * (side + 4 * fel);
+#pragma unroll
+            for (int k = 0; k < NT; k++) p[k * NP] = qL[k];
+            if constexpr (Phys::kLag) p[NT * NP] = lag0;
+            if constexpr (Phys::kLag && NODAL) p[(NX - 1) * NP] = lag1;
+          } else if (code >= 0) {
+            // the emptied slots before the new traces (see above)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            unsigned long long *p = ra.ring + (size_t)fill * ringLen + mine;
+#pragma unroll
+            for (int k = 0; k < NT; k++) ring_store(p + k * NP, (unsigned long long)__double_as_longlong(qL[k]));
+            if constexpr (Phys::kLag) ring_store(p + NT * NP, (unsigned long long)__double_as_longlong(lag0));
+            if constexpr (Phys::kLag && NODAL) ring_store(p + (NX - 1) * NP, (unsigned long long)__double_as_longlong(lag1));
+          }
+        } else {
+          const size_t fb = (size_t)fi + NP * (side + 4 * (size_t)fe);
+          double *tr = a.traceOut + (size_t)fi + NP * (size_t)NT * (side + 4 * (size_t)fe);
+#pragma unroll
+          for (int k = 0; k < NT; k++) tr[(size_t)k * NP] = qL[k];
+          if constexpr (Phys::kLag && NODAL) { a.unOut[2 * fb] = lag0; a.unOut[2 * fb + 1] = lag1; }
+          else if constexpr (Phys::kLag) a.unOut[fb] = lag0;
+        }
+        if constexpr (Phys::kLag) unL = NODAL ? lag0 * nx + lag1 * ny : lag0;
+      }
+    }
+    if constexpr (L::STAGED)
+      if (!last) {
+        phase_sync<WAVE>();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied slots before the new traces (see above)
+        for (int k = tid; k < tileSlots; k += T)
+          ring_store(ra.ring + (size_t)fill * ringLen + tileAt + k, (unsigned long long)__double_as_longlong(lds[L::PK + k]));
+        if constexpr (WAVE) phase_sync<WAVE>();
+      }
+    fill = empty;
+  }
+  if (nodeActive) {
+#pragma unroll
+    for (int v = 0; v < NV; v++) a.S[sBase + (size_t)v * NN + node] = s[v];
+  }
+  if (budget < 0) *ra.timedOut = 1;
+}
+
+// ------------------------------------------------------------------------------
 // Integrals of the state: CalculateEntropy and mass-type integrals
 // ------------------------------------------------------------------------------
 // One work-item per node forms w_i w_j J f(S) (the per-node J as SEMQuad stores it); blocks
@@ -1177,6 +1594,8 @@ inline bool tile_alternates(int kind, int N, int nEl) {
   return v < 0 || v >= 12 || (v & 2);
 }
 int g_tileEpoch = 0;
+// whether tile variant v of N = 5 splits the face sums between lane pairs (the 64-wide ones)
+inline bool tile_splits5(int v) { return v >= 0 && ((v < 12 && (v >> 2) == 0) || v == 12 || v == 13); }
 
 
 template <class Phys, int N>
@@ -1259,6 +1678,37 @@ hipError_t launch_un_init(int N, const double *tr, double *un, const double *geo
   }
 }
 
+struct ResidentKernel {
+  const void *fn = nullptr;
+  int threads = 0, elements = 0, values = 0;  // per block: work-items, elements; ring values per face node
+};
+template <class Phys, int N, bool NODAL>
+ResidentKernel resident_instance(int dense) {
+  using L = ResidentTile<Phys, N, NODAL>;
+  const void *fn = dense == 2   ? reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 4>)
+                   : dense == 1 ? reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 3>)
+                                : reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 1>);
+  return {fn, L::T, L::EPB, L::NX};
+}
+template <class Phys, bool NODAL>
+ResidentKernel resident_of(int N, int dense) {
+  switch (N) {
+#define CASE(NN_) case NN_: return resident_instance<Phys, NN_, NODAL>(dense);
+    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
+#undef CASE
+    default: return {};
+  }
+}
+// dense 1, 2: instances held to the registers of 3 and 4 wavefronts per SIMD, for more resident blocks
+constexpr int kResidentDense = 3;
+ResidentKernel resident_kernel(int kind, int N, bool nodal, int dense) {
+  switch (kind) {
+    case SELFAMD_MODEL_SW: return nodal ? resident_of<PhysSW, true>(N, dense) : resident_of<PhysSW, false>(N, dense);
+    case SELFAMD_MODEL_LSW: return nodal ? resident_of<PhysLSW, true>(N, dense) : resident_of<PhysLSW, false>(N, dense);
+    default: return nodal ? resident_of<PhysEuler, true>(N, dense) : resident_of<PhysEuler, false>(N, dense);
+  }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------------------
@@ -1308,9 +1758,38 @@ struct selfamd_model2d {
   std::vector<int> bandStart;     // nBands + 1 offsets into bandElems
   std::vector<int32_t> hnbr;      // host copy of the neighbour codes
 
+  // resident stepping: the exchange ring (allocated on first use), the blocks that can be
+  // resident at once (15 of 16 of the device's; -1: not asked yet; 0: not available), the
+  // host flag that a launch raises when a wait ran out
+  unsigned long long *ring = nullptr;
+  size_t ringLen = 0;
+  int ringValues = 0;  // values per face node of the slot layout the ring was emptied for
+  int residentBlocks[2][kResidentDense] = {{-1, -1, -1}, {-1, -1, -1}};  // [nodal][dense]
+  bool paired = false;  // every interior side's neighbour names that side as its own neighbour
+  int *timedOut = nullptr;
+
+  FusedArgs stage_args(int traceIn) const {
+    FusedArgs a{};
+    a.S = S; a.G = G;
+    a.traceIn = trace[traceIn];
+    a.traceOut = trace[traceIn ^ 1];
+    a.unIn = un[traceIn]; a.unOut = un[traceIn ^ 1];
+    a.aux = aux; a.stat2 = stat2; a.presTrace = presTrace;
+    a.geom = geom; a.nbr = nbr; a.mats = mats; a.nEl = nEl;
+    a.ndsdx = ndsdx; a.nJ = nJ; a.nnHat = nnHat; a.nnScale = nnScale;
+    a.anyBoundary = anyBoundary;
+    a.p = p;
+    return a;
+  }
+  // Whether a call of nSteps steps runs as one resident launch: the mesh's blocks are all resident
+  // at once with room to spare, and the stages saved pay for a cooperative launch.
+  // Sets the kernel to launch.
+  bool resident(int nSteps, ResidentKernel &k);
+  hipError_t launch_resident(const ResidentKernel &k, int nSteps, double dt);
+
   hipError_t launch_stage(int mode, int stage, double dt, int traceIn, double *dSdt, int band = -1,
                           double *fluxOut = nullptr, double *fluxDivOut = nullptr) {
-    FusedArgs a{};
+    FusedArgs a = stage_args(traceIn);
     a.fluxOut = fluxOut;
     a.fluxDivOut = fluxDivOut;
     if (closure) {
@@ -1322,17 +1801,11 @@ struct selfamd_model2d {
       a.nShift = closure->nShift;
       a.shiftScale = closure->shiftScale;
     }
-    a.S = S; a.G = G; a.dSdt = dSdt;
-    a.traceIn = trace[traceIn];
-    a.traceOut = trace[traceIn ^ 1];
-    a.unIn = un[traceIn]; a.unOut = un[traceIn ^ 1];
-    a.aux = aux; a.stat2 = stat2; a.presTrace = presTrace;
-    a.geom = geom; a.nbr = nbr; a.mats = mats; a.nEl = nEl;
+    a.dSdt = dSdt;
     if (band >= 0) {
       a.elems = bandElems + bandStart[band];
       a.nEl = bandStart[band + 1] - bandStart[band];
     }
-    a.ndsdx = ndsdx; a.nJ = nJ; a.nnHat = nnHat; a.nnScale = nnScale;
     a.rkA = kRk3A[stage];
     a.rkGdt = kRk3G[stage] * dt;
     a.rkG = kRk3G[stage];
@@ -1340,8 +1813,6 @@ struct selfamd_model2d {
     // element order alternates with the trace buffer parity, i.e. from stage to stage
     a.reverse = tile_alternates(kind, N, a.nEl) ? traceIn : 0;
     a.perElemDt = 0;
-    a.anyBoundary = anyBoundary;
-    a.p = p;
     switch (kind) {
       case SELFAMD_MODEL_SW: return Launcher<PhysSW>::stage(N, mode, nodal, a, stream);
       case SELFAMD_MODEL_LSW: return Launcher<PhysLSW>::stage(N, mode, nodal, a, stream);
@@ -1422,6 +1893,75 @@ struct selfamd_model2d {
 };
 
 using Model = selfamd_model2d;
+
+bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
+  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || closure || nBands > 0 || !paired || (timedOut && *timedOut)) return false;
+  // the 64-wide tile of nonlinear SW at N = 5 splits the face sums; the resident kernel does not
+  if (kind == SELFAMD_MODEL_SW && N == 5 && tile_splits5(tile_of(kind, 5))) return false;
+  bool fits = false;
+  for (int dense = 0; dense < kResidentDense && !fits; dense++) {
+    k = resident_kernel(kind, N, nodal, dense);
+    int &blocks = residentBlocks[nodal][dense];
+    if (blocks < 0) {
+      int cus = 0, perCU = 0, coop = 0;
+      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+          hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess ||
+          hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, k.fn, k.threads, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        perCU = 0;
+      }
+      blocks = coop ? cus * perCU * 15 / 16 : 0;
+    }
+    fits = (nEl + k.elements - 1) / k.elements <= blocks;
+  }
+  if (!fits) return false;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const size_t len = 3 * (size_t)(N + 1) * k.values * 4 * nEl;
+  if (ringLen < len) {
+    if (ring) (void)hipFree(ring);
+    ring = nullptr;
+    ringLen = 0;
+    if ((!timedOut && hipHostMalloc(&timedOut, sizeof(int), hipHostMallocDefault) != hipSuccess) ||
+        hipMalloc(&ring, sizeof(unsigned long long) * len) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    *timedOut = 0;
+    ringLen = len;
+    ringValues = 0;
+  }
+  if (ringValues != k.values) {  // first use, or the metric mode (and with it the slot layout) changed
+    hipLaunchKernelGGL(k_ring_fill, (unsigned)std::min<size_t>((ringLen + 255) / 256, 4096), 256, 0, stream, ring, ringLen);
+    if (hipGetLastError() != hipSuccess) return false;
+    ringValues = k.values;
+  }
+  return true;
+}
+
+hipError_t selfamd_model2d::launch_resident(const ResidentKernel &k, int nSteps, double dt) {
+  FusedArgs a = stage_args(cur);
+  const int end = cur ^ (nSteps & 1);  // the trace buffer after 3 nSteps stages
+  a.traceOut = trace[end];
+  a.unOut = un[end];
+  ResidentArgs ra{};
+  ra.ring = ring;
+  ra.stages = 3 * nSteps;
+  for (int q = 0; q < 3; q++) {
+    ra.rkA[q] = kRk3A[q];
+    ra.rkGdt[q] = kRk3G[q] * dt;
+  }
+  ra.timedOut = timedOut;
+  void *args[] = {&a, &ra};
+  const hipError_t e = hipLaunchCooperativeKernel(k.fn, dim3((nEl + k.elements - 1) / k.elements), dim3(k.threads), args, 0, stream);
+  if (e != hipSuccess) return e;
+  cur = end;
+  for (int q = 0; q < nSteps; q++) t += dt;
+  return hipSuccess;
+}
 
 namespace {
 void free_closure(ClosureBuffers *c) {
@@ -1521,6 +2061,12 @@ int selfamd_model2d_create(selfamd_model2d **out, int kind, int N, int nEl, cons
   Model *m = new Model();
   m->kind = kind; m->N = N; m->nEl = nEl;
   m->hnbr = nbr;
+  m->paired = nEl < (1 << 27);
+  for (int e = 0; e < nEl && m->paired; e++)
+    for (int sd = 0; sd < 4; sd++) {
+      const int c = nbr[4 * (size_t)e + sd];
+      if (c >= 0 && nbr[4 * (size_t)(c >> 3) + ((c >> 1) & 3)] != ((e << 3) | (sd << 1) | (c & 1))) m->paired = false;
+    }
   m->anyBoundary = std::any_of(nbr.begin(), nbr.end(), [](int32_t c) { return c < 0; });
   m->affine = affine;
   m->nodal = !affine;
@@ -1592,6 +2138,8 @@ int selfamd_model2d_destroy(selfamd_model2d *m) {
   double *bufs[] = {m->S,    m->G,    m->trace[0], m->trace[1], m->un[0], m->un[1], m->geom,  m->mats,
                     m->aux,  m->stat2, m->presTrace, m->ndsdx, m->nJ,    m->nnHat, m->nnScale};
   if (m->bandElems) (void)hipFree(m->bandElems);
+  if (m->ring) (void)hipFree(m->ring);
+  if (m->timedOut) (void)hipHostFree(m->timedOut);
   if (m->intScratch) (void)hipFree(m->intScratch);
   if (m->adjTrace) (void)hipFree(m->adjTrace);
   if (m->adjChi) (void)hipFree(m->adjChi);
@@ -1802,6 +2350,11 @@ int selfamd_model2d_flux_registers(selfamd_model2d *m, double *fluxDivergence, d
 }
 
 namespace {
+int resident_status(const selfamd_model2d *m) {
+  SELFAMD_REQUIRE(!m->timedOut || !*m->timedOut,
+                  "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
+  return kOk;
+}
 // a few steps of another size than the captured graphs' (e.g. ForwardStep's shorter last step
 // up to tn) are launched directly, so the graphs of the running step size survive
 bool direct_steps(const selfamd_model2d *m, int nSteps, double dt) {
@@ -1840,6 +2393,14 @@ hipError_t prepare_graphs(selfamd_model2d *m, int nSteps, double dt) {
 int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   SELFAMD_REQUIRE(m && nSteps >= 0 && dt > 0.0, "model2d_forward_step: bad arguments (nSteps=%d dt=%g)", nSteps, dt);
   if (nSteps == 0) return kOk;
+  ResidentKernel kernel;
+  if (m->resident(nSteps, kernel)) {
+    if (m->launch_resident(kernel, nSteps, dt) == hipSuccess) return kOk;
+    // not accepted by the runtime: step graphs from here on
+    (void)hipGetLastError();
+    for (auto &blocks : m->residentBlocks)
+      for (int &b : blocks) b = 0;
+  }
   if (direct_steps(m, nSteps, dt)) {
     SELFAMD_HIP(m->launch_steps(nSteps, dt));
     return kOk;
@@ -1867,7 +2428,7 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
 int selfamd_model2d_synchronize(selfamd_model2d *m) {
   SELFAMD_REQUIRE(m, "model2d_synchronize: null model");
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 int selfamd_model2d_stream(selfamd_model2d *m, void **stream) {
@@ -1880,7 +2441,8 @@ int selfamd_model2d_time_steps(selfamd_model2d *m, int nSteps, double dt, double
   SELFAMD_REQUIRE(m && elapsedMs && nSteps >= 0 && dt > 0.0, "model2d_time_steps: bad arguments");
   // graph capture is host work: done before the first event, so the GPU's idle time during it
   // is not timed
-  SELFAMD_HIP(prepare_graphs(m, nSteps, dt));
+  ResidentKernel kernel;
+  if (!m->resident(nSteps, kernel)) SELFAMD_HIP(prepare_graphs(m, nSteps, dt));
   hipEvent_t e0, e1;
   SELFAMD_HIP(hipEventCreate(&e0));
   SELFAMD_HIP(hipEventCreate(&e1));
