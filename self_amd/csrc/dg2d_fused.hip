@@ -1486,37 +1486,78 @@ __global__ void __launch_bounds__(kIntBlock) k_sum_partials(const double *partia
   block_sum_store(v, out);
 }
 
-// Traces of the nodal quantities of the current state (SetSolution's BoundaryInterp).
+// A state taken in (SetSolution) in one pass over it: copied to S, interpolated to the faces
+// (BoundaryInterp), and from the same registers the SW lagged velocities of the first stage and
+// the Euler prescribed traces.  What bounds it: memory on large meshes, the launch on small ones.
+// As copy, trace, velocity and trace copy launches one after another, with the call's
+// synchronisation: linear SW 10^2 N = 7 19.0 us, SW 256^2 N = 7 85, Euler 400^2 N = 7 432; in one
+// pass 15.5, 61 and 189.
+struct StateArgs {
+  const double *src;
+  double *S;      // or null: traces only
+  double *trace;
+  double *un;     // SW lagged velocities (nnHat: the nodal mode's vectors), or null
+  double *pres;   // Euler prescribed traces, or null; only sides on the physical boundary are read
+  const double *geom, *nnHat, *mats;
+  const int32_t *nbr;
+  Params p;
+  int nEl;
+};
 template <class Phys, int N>
-__global__ void __launch_bounds__(kThreads) k_traces(const double *S, double *traceOut, const double *mats, Params p,
-                                                     int nEl) {
+__global__ void __launch_bounds__(kThreads) k_state_in(const StateArgs a) {
   constexpr int NP = N + 1, NN = NP * NP, EPB = kThreads / NN, NF = 4 * NP;
   constexpr int NV = Phys::NV, NT = Phys::NT;
   __shared__ double sQ[NT][EPB][NN];
   const int tid = threadIdx.x;
   const int el = tid / NN, node = tid % NN;
   const int e = blockIdx.x * EPB + el;
-  if (el < EPB && e < nEl) {
+  if (el < EPB && e < a.nEl) {
+    const size_t at = (size_t)e * NV * NN + node;
     double s[NV], q[NT];
-    for (int v = 0; v < NV; v++) s[v] = S[(size_t)e * NV * NN + (size_t)v * NN + node];
-    phys_nodal<Phys>(s, p, q);
+#pragma unroll
+    for (int v = 0; v < NV; v++) s[v] = a.src[at + (size_t)v * NN];
+    if (a.S) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) a.S[at + (size_t)v * NN] = s[v];
+    }
+    phys_nodal<Phys>(s, a.p, q);
+#pragma unroll
     for (int k = 0; k < NT; k++) sQ[k][el][node] = q[k];
   }
   __syncthreads();
   for (int ft = tid; ft < EPB * NF; ft += kThreads) {
     const int fel = ft / NF, fnode = ft % NF, side = fnode / NP, fi = fnode % NP;
     const int fe = blockIdx.x * EPB + fel;
-    if (fe >= nEl) continue;
-    const double *bm = mats + 2 * NN + ((side == 1 || side == 2) ? NP : 0);
+    if (fe >= a.nEl) continue;
+    const double *bm = a.mats + 2 * NN + ((side == 1 || side == 2) ? NP : 0);
     const bool alongJ = (side == 0 || side == 2);
     double qn[NT];
+#pragma unroll
     for (int k = 0; k < NT; k++) qn[k] = 0.0;
+#pragma unroll
     for (int ii = 0; ii < NP; ii++) {
       const int nd = alongJ ? fi + NP * ii : ii + NP * fi;
+#pragma unroll
       for (int k = 0; k < NT; k++) qn[k] += bm[ii] * sQ[k][fel][nd];
     }
-    double *tr = traceOut + (size_t)fi + NP * (size_t)NT * (side + 4 * (size_t)fe);
-    for (int k = 0; k < NT; k++) tr[(size_t)k * NP] = qn[k];
+    const size_t first = (size_t)fi + NP * (size_t)NT * (side + 4 * (size_t)fe);
+#pragma unroll
+    for (int k = 0; k < NT; k++) a.trace[first + (size_t)k * NP] = qn[k];
+    if (a.pres && a.nbr[side + 4 * (size_t)fe] < 0) {
+#pragma unroll
+      for (int k = 0; k < NT; k++) a.pres[first + (size_t)k * NP] = qn[k];
+    }
+    if constexpr (Phys::kLag) {
+      const size_t fb = (size_t)fi + NP * (side + 4 * (size_t)fe);
+      if (a.un && a.nnHat) {
+        a.un[2 * fb] = qn[0] / qn[2];
+        a.un[2 * fb + 1] = qn[1] / qn[2];
+      } else if (a.un) {
+        const double *gr = a.geom + (size_t)fe * kGeomStride;
+        const double nx = gr[8 + side], ny = gr[12 + side];
+        a.un[fb] = (qn[0] / qn[2]) * nx + (qn[1] / qn[2]) * ny;
+      }
+    }
   }
 }
 
@@ -1649,13 +1690,12 @@ struct Launcher {
       default: return hipErrorInvalidValue;
     }
   }
-  static hipError_t traces(int N, const double *S, double *tr, const double *mats, const Params &p, int nEl,
-                           hipStream_t st) {
+  static hipError_t state_in(int N, const StateArgs &a, hipStream_t st) {
     switch (N) {
 #define CASE(NN_)                                                                                   \
   case NN_: {                                                                                       \
     constexpr int EPB = kThreads / ((NN_ + 1) * (NN_ + 1));                                         \
-    hipLaunchKernelGGL((k_traces<Phys, NN_>), dim3((nEl + EPB - 1) / EPB), kThreads, 0, st, S, tr, mats, p, nEl); \
+    hipLaunchKernelGGL((k_state_in<Phys, NN_>), dim3((a.nEl + EPB - 1) / EPB), kThreads, 0, st, a); \
     return hipGetLastError();                                                                       \
   }
       CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
@@ -1819,11 +1859,15 @@ struct selfamd_model2d {
       default: return Launcher<PhysEuler>::stage(N, mode, nodal, a, stream);
     }
   }
-  hipError_t launch_traces() {
+  // the state at `src` (S itself: already there) becomes the current one
+  hipError_t launch_state_in(const double *src) {
+    StateArgs a{};
+    a.src = src; a.S = src == S ? nullptr : S; a.trace = trace[cur]; a.un = un[cur]; a.pres = presTrace;
+    a.geom = geom; a.nnHat = nodal ? nnHat : nullptr; a.mats = mats; a.nbr = nbr; a.p = p; a.nEl = nEl;
     switch (kind) {
-      case SELFAMD_MODEL_SW: return Launcher<PhysSW>::traces(N, S, trace[cur], mats, p, nEl, stream);
-      case SELFAMD_MODEL_LSW: return Launcher<PhysLSW>::traces(N, S, trace[cur], mats, p, nEl, stream);
-      default: return Launcher<PhysEuler>::traces(N, S, trace[cur], mats, p, nEl, stream);
+      case SELFAMD_MODEL_SW: return Launcher<PhysSW>::state_in(N, a, stream);
+      case SELFAMD_MODEL_LSW: return Launcher<PhysLSW>::state_in(N, a, stream);
+      default: return Launcher<PhysEuler>::state_in(N, a, stream);
     }
   }
   void drop_graphs() {
@@ -2195,21 +2239,29 @@ int selfamd_model2d_set_field(selfamd_model2d *m, int which, const double *field
   return kOk;
 }
 
+// Whether a kernel on the model's device can read doubles at p in place of a copy call, which also
+// takes another device's memory, host memory and any alignment.
+static bool device_doubles(const selfamd_model2d *m, const void *p) {
+  hipPointerAttribute_t at{};
+  if (reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+    (void)hipGetLastError();  // memory that the runtime does not know
+    return false;
+  }
+  return at.type == hipMemoryTypeDevice && at.device == m->device;
+}
+
 int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   SELFAMD_REQUIRE(m && interior, "model2d_set_solution: null argument");
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
-  SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
-  SELFAMD_HIP(m->launch_traces());
-  if (m->kind == SELFAMD_MODEL_SW)
-    SELFAMD_HIP(launch_un_init(m->N, m->trace[m->cur], m->un[m->cur], m->geom, m->nodal ? m->nnHat : nullptr, m->nEl,
-                               m->stream));
-  if (m->kind == SELFAMD_MODEL_EULER) {
+  if (m->kind == SELFAMD_MODEL_EULER && !m->presTrace) {
     // prescribed boundary state := traces of this state (SetPrescribedSolutionFromSolution)
-    const size_t nT = (size_t)(m->N + 1) * 9 * 4 * m->nEl;
-    if (!m->presTrace) SELFAMD_HIP(hipMalloc(&m->presTrace, sizeof(double) * nT));
-    SELFAMD_HIP(hipMemcpyAsync(m->presTrace, m->trace[m->cur], sizeof(double) * nT, hipMemcpyDeviceToDevice, m->stream));
-    m->drop_graphs();
+    SELFAMD_HIP(hipMalloc(&m->presTrace, sizeof(double) * (size_t)(m->N + 1) * 9 * 4 * m->nEl));
+    m->drop_graphs();  // captured without it
   }
+  const bool direct = device_doubles(m, interior);
+  if (!direct) SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
+  SELFAMD_HIP(m->launch_state_in(direct ? interior : m->S));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
   return kOk;
 }
@@ -2535,8 +2587,13 @@ int selfamd_model2d_tendency_vjp(selfamd_model2d *m, const double *S, const doub
   // scratch: traces of S and of Sprev, neighbour-trace cotangents, lagged-velocity cotangents
   if (!m->adjTrace) SELFAMD_HIP(hipMalloc(&m->adjTrace, sizeof(double) * 2 * nTr));
   if (!m->adjChi) SELFAMD_HIP(hipMalloc(&m->adjChi, sizeof(double) * nTr * 5 / 3));
-  SELFAMD_HIP(Launcher<PhysSW>::traces(m->N, S, m->adjTrace, m->mats, m->p, m->nEl, m->stream));
-  if (Sprev) SELFAMD_HIP(Launcher<PhysSW>::traces(m->N, Sprev, m->adjTrace + nTr, m->mats, m->p, m->nEl, m->stream));
+  StateArgs tr{};  // traces only
+  tr.src = S; tr.trace = m->adjTrace; tr.mats = m->mats; tr.p = m->p; tr.nEl = m->nEl;
+  SELFAMD_HIP(Launcher<PhysSW>::state_in(m->N, tr, m->stream));
+  if (Sprev) {
+    tr.src = Sprev; tr.trace = m->adjTrace + nTr;
+    SELFAMD_HIP(Launcher<PhysSW>::state_in(m->N, tr, m->stream));
+  }
   SELFAMD_HIP(sw_tendency_vjp(m->N, m->nEl, S, m->adjTrace, un, m->aux, m->geom, m->nbr, m->mats, m->p.g, m->p.fCori,
                               m->p.auxConst, lambda, mu, m->adjChi, m->adjTrace + nTr, muPrev, m->adjChi + nTr,
                               m->stream));
