@@ -2754,7 +2754,7 @@ int selfamd_model2d_set_time(selfamd_model2d *m, double t) {
 // Models of one polynomial degree are concatenated into one virtual mesh (state, traces,
 // static fields, neighbour codes offset by each run's first element); each element record
 // carries its run's dt.  One fused launch per degree group and RK stage advances every run
-// of the group, and one hipGraph holds all groups' three stages of a step.  Per element the
+// of the group, and one hipGraph holds all groups' stages of one or more steps.  Per element the
 // arithmetic is that of the single-run engine, so a batched run is bit-identical to the same
 // run advanced alone.
 namespace {
@@ -2832,12 +2832,12 @@ struct selfamd_batch {
     a.p = p;
     return a;
   }
-  hipError_t launch_group(BatchGroup &g, int stage, int tin) {
+  hipError_t launch_group(const BatchGroup &g, int stage, int tin, hipStream_t st) {
     const FusedArgs a = group_args(g, stage, tin);
     switch (kind) {
-      case SELFAMD_MODEL_SW: return Launcher<PhysSW>::stage(g.N, 0, false, a, stream);
-      case SELFAMD_MODEL_LSW: return Launcher<PhysLSW>::stage(g.N, 0, false, a, stream);
-      default: return Launcher<PhysEuler>::stage(g.N, 0, false, a, stream);
+      case SELFAMD_MODEL_SW: return Launcher<PhysSW>::stage(g.N, 0, false, a, st);
+      case SELFAMD_MODEL_LSW: return Launcher<PhysLSW>::stage(g.N, 0, false, a, st);
+      default: return Launcher<PhysEuler>::stage(g.N, 0, false, a, st);
     }
   }
   // whether the persistent kernel covers this batch: nonlinear SW, every degree 3, 5 or 7, and
@@ -2867,26 +2867,80 @@ struct selfamd_batch {
     hipLaunchKernelGGL(k_batch_persistent<PhysSW>, dim3(persistentBlocks), 256, 0, stream, pa);
     return hipGetLastError();
   }
-  // graphs of one RK3 step for both starting trace buffers
-  // captures `steps` steps starting from trace buffer `start` (each step flips the buffer)
+  // Whether the groups of a graph of `steps` steps are branches of it: they are independent for the
+  // whole call, and a stage launch then fills what another group's last wave leaves idle and starts
+  // while that one ends.  10 steps of 48 shallow water runs of 8^2 to 64^2 elements (degrees 3, 5
+  // and 7) take 1,650 us as branches and 1,950 in turn, 12 runs up to 32^2 335 and 500.  It costs a
+  // fork and a join, 30 to 40 us per graph (one run each of degrees 3, 5 and 7, two steps: 304,000
+  // nodes 118 and 128 us, 135,000 115 and 101; 10 steps of 8,000 nodes still 399 and 418, but with
+  // two groups nothing).  And where the batch is larger than the Infinity Cache, a group's stages
+  // find their data there only in turn (degrees 5 and 7, 10 steps: 192 MiB 1,835 and 1,963 us,
+  // 264 MiB 2,567 and 2,544, 500 MiB 5,550 and 5,238).
+  bool branches_pay(int steps) const {
+    if (mode == SELFAMD_BATCH_PERSISTENT || groups.size() < 2) return false;
+    size_t nodes = 0, bytes = 0;
+    for (const auto &g : groups) {
+      const size_t P = g.N + 1, n = P * P * g.nEl, faces = P * 4 * g.nEl;
+      nodes += n;
+      bytes += 8 * (n * (2 * models[0]->nVar + (g.aux != nullptr) + (g.stat2 != nullptr)) +
+                    faces * (2 * models[0]->nT + (g.un[0] ? 2 : 0) + (g.presTrace ? models[0]->nT : 0)));
+    }
+    return bytes <= (size_t)256 << 20 && (nodes * steps >= (size_t)1 << 19 || (groups.size() > 2 && steps >= 8));
+  }
+  // Captures `steps` steps starting from trace buffer `start` (each step flips the buffer).
   hipError_t capture_steps(int start, int steps, hipGraphExec_t *out) {
+    const size_t branches = branches_pay(steps) ? groups.size() : 1;
+    struct Branches {  // a stream and the event of its end for each branch but the first
+      std::vector<hipStream_t> stream;
+      std::vector<hipEvent_t> end;
+      hipEvent_t fork = nullptr;
+      hipError_t create(size_t n) {
+        hipError_t e = n > 1 ? hipEventCreateWithFlags(&fork, hipEventDisableTiming) : hipSuccess;
+        for (size_t k = 1; k < n && e == hipSuccess; k++) {
+          hipStream_t s;
+          hipEvent_t v;
+          if ((e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) != hipSuccess) break;
+          stream.push_back(s);
+          if ((e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) == hipSuccess) end.push_back(v);
+        }
+        return e;
+      }
+      ~Branches() {
+        for (auto v : end) (void)hipEventDestroy(v);
+        for (auto s : stream) (void)hipStreamDestroy(s);
+        if (fork) (void)hipEventDestroy(fork);
+      }
+    } side;
+    hipError_t e = side.create(branches);
+    if (e != hipSuccess) return e;
     hipGraph_t gr;
-    hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
+    e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
     hipError_t le = hipSuccess;
-    for (int n = 0; n < steps && le == hipSuccess; n++) {
-      const int tin = start ^ (n & 1);
-      if (mode == SELFAMD_BATCH_PERSISTENT) {
-        for (int st = 0; st < 3 && le == hipSuccess; st++) le = launch_persistent(st, tin ^ (st & 1));
-      } else {
-        // The groups are independent, so each group's three stages run back to back (a stage
-        // then starts on the data its predecessor left in the Infinity Cache), and the group
-        // order reverses from step to step (with the buffer parity), so that a group's last
-        // stage of one step is followed by its first stage of the next.
-        const int ng = (int)groups.size();
-        for (int k = 0; k < ng; k++) {
-          BatchGroup &g = groups[tin == 0 ? k : ng - 1 - k];
-          for (int st = 0; st < 3 && le == hipSuccess; st++) le = launch_group(g, st, tin ^ (st & 1));
+    // the stages of step n (each one flips the buffer)
+    auto stages = [&](const BatchGroup &g, int n, hipStream_t st) {
+      for (int k = 0; k < 3 && le == hipSuccess; k++) le = launch_group(g, k, start ^ ((n + k) & 1), st);
+    };
+    if (branches > 1) {
+      le = hipEventRecord(side.fork, stream);
+      for (size_t k = 0; k < branches && le == hipSuccess; k++) {
+        const hipStream_t st = k ? side.stream[k - 1] : stream;
+        if (k) le = hipStreamWaitEvent(st, side.fork, 0);
+        for (int n = 0; n < steps; n++) stages(groups[k], n, st);
+        if (k && le == hipSuccess) le = hipEventRecord(side.end[k - 1], st);
+      }
+      for (size_t k = 1; k < branches && le == hipSuccess; k++) le = hipStreamWaitEvent(stream, side.end[k - 1], 0);
+    } else {
+      for (int n = 0; n < steps && le == hipSuccess; n++) {
+        const int tin = start ^ (n & 1), ng = (int)groups.size();
+        if (mode == SELFAMD_BATCH_PERSISTENT) {
+          for (int st = 0; st < 3 && le == hipSuccess; st++) le = launch_persistent(st, tin ^ (st & 1));
+        } else {
+          // Each group's three stages run back to back (a stage then starts on the data its
+          // predecessor left in the Infinity Cache), and the group order reverses from step to
+          // step (with the buffer parity), so that a group's last stage of one step is followed
+          // by its first stage of the next.
+          for (int k = 0; k < ng; k++) stages(groups[tin == 0 ? k : ng - 1 - k], n, stream);
         }
       }
     }
