@@ -44,6 +44,13 @@ hipError_t closure_vjp(const ClosureBuffers &c, const double *S, const double *g
 size_t closure_vjp_partials(int N, int nEl);
 
 hipError_t mlp_forward(selfamd_mlp *m, const float *X, float *Y, int B, hipStream_t st);
+// the network's parameters on the device (row-major W[in][out]); rows: it runs on the row kernels
+struct MlpWeights {
+  bool rows;
+  int nH;
+  const float *W1, *b1, *W2, *b2, *W3, *b3;
+};
+MlpWeights mlp_weights(const selfamd_mlp *m);
 int mlp_shape(const selfamd_mlp *m, int *nIn, int *nOut, int *maxB);
 
 }  // namespace selfamd

@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "closure.hpp"
+#include "mlp_rows.hpp"
 #include "sw_adjoint.hpp"
 #include "../../include/self_amd.h"
 
@@ -318,16 +319,10 @@ __device__ inline double pair_sum32(double x) {
   return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
 }
 
-// Sum of x over a wavefront, in every lane, by VALU lane exchanges: lanes l ^ 32, l ^ 16, then
-// rotations by 8, 4, 2 and 1 within each row of 16 lanes.
-__device__ inline double wave_sum(double x) {
-  x = pair_sum32(x);
-  {
-    const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
-    const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-    const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-    x = __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
-  }
+// Sums of x over 16, 32 or all 64 lanes, in every lane of them, by VALU lane exchanges: lanes l ^ 32,
+// l ^ 16, then rotations by 8, 4, 2 and 1 within each row of 16 lanes, which exchange what xors
+// would (the partial sums repeat with that period).
+__device__ inline double row_sum16(double x) {
   auto rotate = [](double v, auto n) {  // DPP row_ror:n
     constexpr int ctrl = 0x120 + decltype(n)::value;
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, false);
@@ -340,6 +335,13 @@ __device__ inline double wave_sum(double x) {
   x += rotate(x, std::integral_constant<int, 1>{});
   return x;
 }
+__device__ inline double half_sum32(double x) {
+  const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
+  const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return row_sum16(__hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]));
+}
+__device__ inline double wave_sum(double x) { return half_sum32(pair_sum32(x)); }
 
 // ------------------------------------------------------------------------------
 // The fused kernel
@@ -1040,6 +1042,15 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // trace buffers instead, so the next call finds the slots of its stage -2 filled and empties them
 // first, and all others empty.
 //
+// With a closure (NET) a block has 16 elements, a row tile of the network, and the stage starts with
+// features -> network -> correction in LDS.  The network's weights stay in registers (at 128 hidden
+// units 80 of them; 1 block per CU), so a stage reads nothing from memory but traces and the other
+// blocks' mass integrals, which every block sends to all others right after the network and needs
+// only at the update.  64 x 64 elements, N = 3, 51 -> 128 -> 128 -> 48, per stage: 16.2 us in two
+// launches (network 8.1 us of them), 6.7 us here: network 3.9, face and volume work 2.5.  With the
+// integrals in one copy that all blocks poll, sent after the face phase, the wait for them alone was
+// 3.3 us (9.5 us per stage).  A call of one step takes 78 us with set and get, 110 in launches.
+//
 // All blocks must be resident: the launch is cooperative, which the runtime refuses if they
 // cannot be.  Every wait is bounded as well: a lane that has polled kPollBudget times in a call
 // stops waiting and raises `timedOut`, which the next synchronising call reports.
@@ -1052,14 +1063,28 @@ struct ResidentArgs {
   double rkA[3], rkGdt[3];   // a_m, g_m dt
   int *timedOut;             // host memory
 };
+// With a closure attached (NET): the network and where the blocks exchange their mass integrals
+struct ResidentNetArgs {
+  MlpWeights w;
+  const float *inMean, *inScale, *outMean, *outScale;
+  double shiftScale;
+  unsigned long long *mass;  // 3 buffers, used like the trace ring, of kMassCopies times massStride values
+  int massStride;            // one value per block, rounded up to 4 KiB
+};
 
-template <class Phys, int N, bool NODAL>
+// The blocks' integrals go to every block: in as many copies as there are XCDs, so that not all
+// blocks read the same few lines.
+constexpr int kMassCopies = 8;
+
+template <class Phys, int N, bool NODAL, bool NET = false>
 struct ResidentTile {
   static constexpr int NP = N + 1, NN = NP * NP, NF = 4 * NP;
   // one wavefront per block, so that no phase boundary is a block barrier, except at N = 5, where
-  // a wavefront would hold a single element on 36 of its lanes
-  static constexpr int T = N == 5 ? 128 : 64;
-  static constexpr int EPB = T / NN < T / NF ? T / NN : T / NF;
+  // a wavefront would hold a single element on 36 of its lanes, and with a closure, whose network
+  // takes 16 elements through its layers with 8 wavefronts
+  static constexpr int T = NET ? kRowThreads : N == 5 ? 128 : 64;
+  static constexpr int EPB = NET ? kRowTile : T / NN < T / NF ? T / NN : T / NF;
+  static constexpr int FACE0 = NET ? T - EPB * NF : 0;  // first face lane
   static constexpr bool WAVE = T == 64;
   static constexpr bool SPLIT = N >= 6;  // the face sums of the stage kernel's tiles
   static constexpr int NV = Phys::NV, NT = Phys::NT, NX = NT + (Phys::kLag ? (NODAL ? 2 : 1) : 0);
@@ -1087,14 +1112,71 @@ __device__ inline void ring_store(unsigned long long *p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The closure's network in a resident block: wavefront w holds the weights of columns 16 w .. 16 w +
+// 15 of all three layers in registers for the whole call, pieces of 64 reduction indices each.
+constexpr int kResidentHidden = 128;  // one 16-column tile per wavefront
+template <int NIN, int NO>
+struct ResidentNet {
+  static constexpr int PIECES = pad64(NIN) / 64;
+  static constexpr int LDX = rows_ld(NIN), LDH = rows_ld(kResidentHidden), LDO = rows_ld(NO);
+  static constexpr int FLOATS = kRowTile * (LDX + 2 * LDH + LDO) + 2 * NO;
+  static_assert(NIN <= 128 && NO <= 128, "a wavefront holds one tile of the output layer");
+  float w1[PIECES][16], w2[2][16], w3[2][16], b1, b2, b3;
+  int nH, wave, lane;
+
+  __device__ void load(const ResidentNetArgs &n, int tid) {
+    nH = n.w.nH;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lane = tid & 63;
+    const int col = 16 * wave + (lane & 15), g = lane >> 4;
+    const RowsOperand o1{n.w.W1, nH, NIN, nH}, o2{n.w.W2, nH, nH, nH}, o3{n.w.W3, NO, nH, NO};
+#pragma unroll
+    for (int k = 0; k < PIECES; k++) rows_load<false, false>(o1, col, g, 64 * k, w1[k]);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      rows_load<false, false>(o2, col, g, 64 * k, w2[k]);
+      rows_load<false, false>(o3, col, g, 64 * k, w3[k]);
+    }
+    b1 = n.w.b1[min(col, nH - 1)];
+    b2 = n.w.b2[min(col, nH - 1)];
+    b3 = n.w.b3[min(col, NO - 1)];
+  }
+  // one layer of this wavefront's columns: out(rows, column) = act(in W + b), 0 past `width`
+  template <bool GELU, int K>
+  __device__ void layer(const float *in, int ldIn, const float (&w)[K][16], bool second, float bias, int width,
+                        float *out, int ldOut) const {
+    if (16 * wave >= pad16(width)) return;
+    const float *rows = in + (lane & 15) * ldIn + 4 * (lane >> 4);
+    f32x4 acc = rows_mul(rows, w[0], f32x4{0.f, 0.f, 0.f, 0.f});
+    if (K > 1 && second) acc = rows_mul(rows + 64, w[K - 1], acc);
+    const int col = 16 * wave + (lane & 15), g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float y = acc[i] + bias;
+      if constexpr (GELU) y = gelu_f(y);
+      out[(4 * g + i) * ldOut + col] = col < width ? y : 0.f;
+    }
+  }
+  // the network from the features in sX to the outputs in sO (not ended by a barrier)
+  __device__ void run(const float *sX, float *sH1, float *sH2, float *sO) const {
+    const bool second = nH > 64;
+    layer<true>(sX, LDX, w1, true, b1, nH, sH1, LDH);
+    __syncthreads();
+    layer<true>(sH1, LDH, w2, second, b2, nH, sH2, LDH);
+    __syncthreads();
+    layer<false>(sH2, LDH, w3, second, b3, NO, sO, LDO);
+  }
+};
+
 __global__ void k_ring_fill(unsigned long long *ring, size_t n) {
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
     ring[t] = kEmpty;
 }
 
-template <class Phys, int N, bool NODAL, int WPE>
-__global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_resident(const FusedArgs a, const ResidentArgs ra) {
-  using L = ResidentTile<Phys, N, NODAL>;
+template <class Phys, int N, bool NODAL, int WPE, bool NET = false>
+__global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL, NET>::T)) __attribute__((amdgpu_waves_per_eu(WPE, 8)))
+k_resident(const FusedArgs a, const ResidentArgs ra, const ResidentNetArgs na) {
+  using L = ResidentTile<Phys, N, NODAL, NET>;
   constexpr int NP = L::NP, NN = L::NN, NF = L::NF, T = L::T, EPB = L::EPB, NV = L::NV, NT = L::NT, NX = L::NX;
   constexpr int MRS = L::MRS, NNS = L::NNS;
   constexpr bool SPLIT = L::SPLIT, WAVE = L::WAVE, SWZ = NP == 8;
@@ -1119,11 +1201,11 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
     e = __builtin_amdgcn_readfirstlane(e);
     nodeActive = __builtin_amdgcn_readfirstlane((int)nodeActive) != 0;
   }
-  const int fhalf = SPLIT ? tid >> 5 : 0, fslot = SPLIT ? tid & 31 : tid;
+  const int fhalf = SPLIT ? tid >> 5 : 0, fslot = SPLIT ? tid & 31 : max(tid - L::FACE0, 0);
   const int fel = fslot / NF, fslotN = fslot % NF;
   const int side = SPLIT ? ((fslotN / NP) >> 1 | ((fslotN / NP) & 1) << 1) : fslotN / NP;
   const int fi = fslotN % NP, fnode = side * NP + fi, fe = blockIdx.x * EPB + fel;
-  const bool faceActive = fel < EPB && fe < a.nEl && (!SPLIT || fslot < NF);
+  const bool faceActive = tid >= L::FACE0 && fel < EPB && fe < a.nEl && (!SPLIT || fslot < NF);
   const bool faceOwner = faceActive && fhalf == 0;  // the lane of a pair that has the face node
   const bool alongJ = side == 0 || side == 2;
   constexpr int FH0 = NP / 2, FHN = NP - FH0;
@@ -1258,6 +1340,44 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
     __syncthreads();
   }
 
+  // the closure: network, features that stay (the element's metric terms), scales and weights
+  constexpr int NO = NV * NN, NIN = NO + 3;
+  using Net = ResidentNet<NET ? NIN : 1, NET ? NO : 1>;
+  __shared__ __align__(16) float netLds[NET ? Net::FLOATS : 4];
+  __shared__ double sWeight[NET ? NO : 1], sJ[NET ? EPB : 1], sRed[NET ? EPB : 1], sShift;
+  float *sX = netLds, *sH1 = sX + kRowTile * Net::LDX, *sH2 = sH1 + kRowTile * Net::LDH, *sO = sH2 + kRowTile * Net::LDH;
+  float *sScale = sO + kRowTile * Net::LDO, *sMean = sScale + NO;
+  [[maybe_unused]] Net net;
+  [[maybe_unused]] float inMean[NV], inScale[NV];
+  if constexpr (NET) {
+    net.load(na, tid);
+    for (int k = tid; k < Net::FLOATS - 2 * NO; k += T) netLds[k] = 0.f;  // rows and columns that stay empty
+    for (int k = tid; k < NO; k += T) {
+      sScale[k] = na.outScale[k];
+      sMean[k] = na.outMean[k];
+      const int nd = k - 2 * NN;  // variable 2 is H / eta / rho
+      sWeight[k] = nd >= 0 && nd < NN ? qW[nd % NP] * qW[nd / NP] : 0.0;
+    }
+    __syncthreads();
+    for (int k = tid; k < 3 * EPB; k += T) {
+      const int row = k / 3, c = k % 3;
+      const size_t re = (size_t)blockIdx.x * EPB + row;
+      if (re < (size_t)a.nEl) {
+        const double *gr = a.geom + re * kGeomStride;
+        const double raw = gr[c == 0 ? 4 : c == 1 ? 0 : 3];
+        sX[row * Net::LDX + NO + c] = (float)((raw - (double)na.inMean[NO + c]) / (double)na.inScale[NO + c]);
+        if (c == 0) sJ[row] = raw;
+      } else if (c == 0) {
+        sJ[row] = 0.0;
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      inMean[v] = na.inMean[v * NN + node];
+      inScale[v] = na.inScale[v * NN + node];
+    }
+  }
+
   // ---- stages ----
   const unsigned tileAt = blockIdx.x * (unsigned)(EPB * NF * NX);
   const int tileSlots = min(EPB, a.nEl - (int)blockIdx.x * EPB) * NF * NX;
@@ -1277,6 +1397,36 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
       for (int v = 0; v < NV; v++) {
         sF1[v][el][nl] = dsdx[0] * fx[v] + dsdx[1] * fy[v];
         sF2[v][el][nl] = dsdx[2] * fx[v] + dsdx[3] * fy[v];
+      }
+      if constexpr (NET) {
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+          sX[el * Net::LDX + v * NN + node] = (float)((s[v] - (double)inMean[v]) / (double)inScale[v]);
+      }
+    }
+    if constexpr (NET) {
+      // every block has read this one's integral of stage m - 2: their integrals of stage m - 1 are here
+      const size_t mine8 = (size_t)(net.lane & (kMassCopies - 1)) * na.massStride + blockIdx.x;
+      const bool publisher = net.wave == T / 64 - 1 && net.lane < kMassCopies;
+      if (publisher) ring_store(na.mass + (size_t)empty * kMassCopies * na.massStride + mine8, kEmpty);
+      __syncthreads();
+      net.run(sX, sH1, sH2, sO);
+      __syncthreads();
+      // integral of the mass variable's correction over each element: 32 work-items per element
+      const int row = tid >> 5;
+      double mass = 0.0;
+      for (int k = tid & 31; k < NO; k += 32) {
+        const double c = (double)sO[row * Net::LDO + k] * (double)sScale[k] + (double)sMean[k];
+        mass += sWeight[k] * c;
+      }
+      mass = half_sum32(mass);
+      if ((tid & 31) == 0) sRed[row] = sJ[row] * mass;
+      __syncthreads();
+      if (net.wave == T / 64 - 1) {  // as early as it can be: the face phase hides its way to the other blocks
+        const double own = row_sum16(sRed[net.lane & 15]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the emptied slots first (see above)
+        if (publisher)
+          ring_store(na.mass + (size_t)fill * kMassCopies * na.massStride + mine8, (unsigned long long)__double_as_longlong(own));
       }
     }
     double lag0 = 0.0, lag1 = 0.0;  // this stage's own face velocity, for the next one
@@ -1333,8 +1483,7 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
     if constexpr (L::STAGED)  // every lane of the tile has its neighbour's traces
       for (int k = tid; k < tileSlots; k += T) ring_store(ra.ring + (size_t)empty * ringLen + tileAt + k, kEmpty);
 
-    if (nodeActive) {
-      double dxs[NV], des[NV];
+    auto divergence = [&](double *dxs, double *des) {
 #pragma unroll
       for (int v = 0; v < NV; v++) { dxs[v] = 0.0; des[v] = 0.0; }
       auto line = [&](int ii) {
@@ -1345,13 +1494,15 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
           des[v] = des[v] + aj * sF2[v][el][slot(i, ii)];
         }
       };
-      if constexpr (WPE == 1) {
+      if constexpr (WPE <= 2) {
 #pragma unroll
         for (int ii = 0; ii < NP; ii++) line(ii);
       } else {
 #pragma unroll 2
         for (int ii = 0; ii < NP; ii++) line(ii);
       }
+    };
+    auto update = [&](const double *dxs, const double *des, double shift) {
       double src[NV];
       Phys::source(s, gx, gy, statVal, a.p, src);
       const double rkA = ra.rkA[fill], gdt = ra.rkGdt[fill];
@@ -1364,7 +1515,13 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
         d = d + (bi1 * sBF[v][el][NP + j] + bi0 * sBF[v][el][3 * NP + j]) * iwi +
             (bj1 * sBF[v][el][2 * NP + i] + bj0 * sBF[v][el][i]) * iwj;
         d = d * invJ;
-        const double dsdt = src[v] - d;
+        double dsdt = src[v] - d;
+        if constexpr (NET) {
+          const int k = v * NN + node;
+          double c = (double)sO[el * Net::LDO + k] * (double)sScale[k] + (double)sMean[k];
+          if (v == 2) c -= shift;
+          dsdt += c;
+        }
         g[v] = rkA * (fill == 0 ? 0.0 : g[v]) + dsdt;
         s[v] = s[v] + gdt * g[v];
         // the RK register that the last step's second stage leaves behind
@@ -1374,6 +1531,41 @@ __global__ void __launch_bounds__((ResidentTile<Phys, N, NODAL>::T)) __attribute
       phys_nodal<Phys>(s, a.p, q);
 #pragma unroll
       for (int k = 0; k < NT; k++) sQ[k][el][nl] = q[k];
+    };
+    if constexpr (NET) {
+      // the last wavefront, which has no nodes, adds up all blocks' integrals meanwhile, in the
+      // order of the stage kernel
+      static_assert(EPB * NN <= T - 64, "the last wavefront has nodes");
+      double dxs[NV], des[NV];
+      if (nodeActive) divergence(dxs, des);
+      if (net.wave == T / 64 - 1) {
+        double part = 0.0;
+        const unsigned long long *box =
+            na.mass + (size_t)(fill * kMassCopies + (int)(blockIdx.x & (kMassCopies - 1))) * na.massStride;
+        const int n = (int)gridDim.x;
+        for (int k = net.lane; k < n; k += 256) {
+          unsigned long long x[4];
+          for (;;) {
+            bool ok = true;
+#pragma unroll
+            for (int q = 0; q < 4; q++) x[q] = ring_load(box + min(k + 64 * q, n - 1));
+#pragma unroll
+            for (int q = 0; q < 4; q++) ok = ok && x[q] != kEmpty;
+            if (ok || --budget < 0) break;
+          }
+#pragma unroll
+          for (int q = 0; q < 4; q++) part += k + 64 * q < n ? __longlong_as_double((long long)x[q]) : 0.0;
+        }
+        part = wave_sum(part);
+        part *= na.shiftScale;
+        if (net.lane == 0) sShift = part;
+      }
+      __syncthreads();
+      if (nodeActive) update(dxs, des, sShift);
+    } else if (nodeActive) {
+      double dxs[NV], des[NV];
+      divergence(dxs, des);
+      update(dxs, des, 0.0);
     }
     phase_sync<WAVE>();
 
@@ -1739,6 +1931,27 @@ ResidentKernel resident_of(int N, int dense) {
     default: return {};
   }
 }
+// with a closure attached (affine metrics): degrees whose nodes leave a wavefront of the block free
+template <class Phys>
+ResidentKernel resident_net_of(int N) {
+  switch (N) {
+#define CASE(NN_)                                                                                   \
+  case NN_: {                                                                                       \
+    using L = ResidentTile<Phys, NN_, false, true>;                                                 \
+    return {reinterpret_cast<const void *>(&k_resident<Phys, NN_, false, 2, true>), L::T, L::EPB, L::NX}; \
+  }
+    CASE(1) CASE(2) CASE(3) CASE(4)
+#undef CASE
+    default: return {};
+  }
+}
+ResidentKernel resident_net_kernel(int kind, int N) {
+  switch (kind) {
+    case SELFAMD_MODEL_SW: return resident_net_of<PhysSW>(N);
+    case SELFAMD_MODEL_LSW: return resident_net_of<PhysLSW>(N);
+    default: return resident_net_of<PhysEuler>(N);
+  }
+}
 // dense 1, 2: instances held to the registers of 3 and 4 wavefronts per SIMD, for more resident blocks
 constexpr int kResidentDense = 3;
 ResidentKernel resident_kernel(int kind, int N, bool nodal, int dense) {
@@ -1805,6 +2018,7 @@ struct selfamd_model2d {
   size_t ringLen = 0;
   int ringValues = 0;  // values per face node of the slot layout the ring was emptied for
   int residentBlocks[2][kResidentDense] = {{-1, -1, -1}, {-1, -1, -1}};  // [nodal][dense]
+  int residentNetBlocks = -1;  // with a closure
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
   int *timedOut = nullptr;
 
@@ -1825,6 +2039,7 @@ struct selfamd_model2d {
   // at once with room to spare, and the stages saved pay for a cooperative launch.
   // Sets the kernel to launch.
   bool resident(int nSteps, ResidentKernel &k);
+  int mass_stride(const ResidentKernel &k) const { return ((nEl + k.elements - 1) / k.elements + 511) & ~511; }
   hipError_t launch_resident(const ResidentKernel &k, int nSteps, double dt);
 
   hipError_t launch_stage(int mode, int stage, double dt, int traceIn, double *dSdt, int band = -1,
@@ -1939,13 +2154,11 @@ struct selfamd_model2d {
 using Model = selfamd_model2d;
 
 bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
-  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || closure || nBands > 0 || !paired || (timedOut && *timedOut)) return false;
+  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || (timedOut && *timedOut)) return false;
   // the 64-wide tile of nonlinear SW at N = 5 splits the face sums; the resident kernel does not
   if (kind == SELFAMD_MODEL_SW && N == 5 && tile_splits5(tile_of(kind, 5))) return false;
-  bool fits = false;
-  for (int dense = 0; dense < kResidentDense && !fits; dense++) {
-    k = resident_kernel(kind, N, nodal, dense);
-    int &blocks = residentBlocks[nodal][dense];
+  // blocks of k that the device holds at once, `of` 16ths of them
+  auto capacity = [&](int &blocks, int of) {
     if (blocks < 0) {
       int cus = 0, perCU = 0, coop = 0;
       if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
@@ -1954,9 +2167,20 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
         (void)hipGetLastError();
         perCU = 0;
       }
-      blocks = coop ? cus * perCU * 15 / 16 : 0;
+      blocks = coop ? cus * perCU * of / 16 : 0;
     }
-    fits = (nEl + k.elements - 1) / k.elements <= blocks;
+    return (nEl + k.elements - 1) / k.elements <= blocks;
+  };
+  bool fits = false;
+  if (closure) {
+    k = resident_net_kernel(kind, N);
+    const MlpWeights w = mlp_weights(closure->mlp);
+    fits = k.fn && !nodal && w.rows && w.nH <= kResidentHidden && capacity(residentNetBlocks, 16);
+  } else {
+    for (int dense = 0; dense < kResidentDense && !fits; dense++) {
+      k = resident_kernel(kind, N, nodal, dense);
+      fits = capacity(residentBlocks[nodal][dense], 15);
+    }
   }
   if (!fits) return false;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -1964,7 +2188,7 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
     (void)hipGetLastError();
     return false;
   }
-  const size_t len = 3 * (size_t)(N + 1) * k.values * 4 * nEl;
+  const size_t len = 3 * ((size_t)(N + 1) * k.values * 4 * nEl + (closure ? (size_t)kMassCopies * mass_stride(k) : 0));
   if (ringLen < len) {
     if (ring) (void)hipFree(ring);
     ring = nullptr;
@@ -1999,7 +2223,16 @@ hipError_t selfamd_model2d::launch_resident(const ResidentKernel &k, int nSteps,
     ra.rkGdt[q] = kRk3G[q] * dt;
   }
   ra.timedOut = timedOut;
-  void *args[] = {&a, &ra};
+  ResidentNetArgs na{};
+  if (closure) {
+    na.w = mlp_weights(closure->mlp);
+    na.inMean = closure->inMean; na.inScale = closure->inScale;
+    na.outMean = closure->outMean; na.outScale = closure->outScale;
+    na.shiftScale = closure->invArea;
+    na.mass = ring + 3 * (size_t)(N + 1) * k.values * 4 * nEl;
+    na.massStride = mass_stride(k);
+  }
+  void *args[] = {&a, &ra, &na};
   const hipError_t e = hipLaunchCooperativeKernel(k.fn, dim3((nEl + k.elements - 1) / k.elements), dim3(k.threads), args, 0, stream);
   if (e != hipSuccess) return e;
   cur = end;
@@ -2452,6 +2685,7 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
     (void)hipGetLastError();
     for (auto &blocks : m->residentBlocks)
       for (int &b : blocks) b = 0;
+    m->residentNetBlocks = 0;
   }
   if (direct_steps(m, nSteps, dt)) {
     SELFAMD_HIP(m->launch_steps(nSteps, dt));
