@@ -1781,10 +1781,13 @@ __global__ void k_sw_un_init(const double *trace, double *un, const double *geom
 }
 
 // Block size (tile) per polynomial degree: one wavefront per element at N = 7, larger
-// blocks where an element covers only part of a wavefront.
+// blocks where an element covers only part of a wavefront.  N = 5 with nodal metrics: 7 elements
+// on 252 of 256 lanes against 3 on 108 of 128; per stage SW 121 x 87 20.2 against 21.2 us, 300 x
+// 200 81.7 and 86.2, Euler 121 x 87 25.3 and 27.0, linear SW 17.0 and 18.1 (with affine metrics
+// the tuned tiles' 128 lanes are the faster ones).
 template <int N>
-constexpr int tile_threads() {
-  return N == 7 ? 64 : N == 6 ? 64 : N == 5 ? 128 : N == 4 ? 128 : 256;
+constexpr int tile_threads(bool nodal = false) {
+  return N == 7 ? 64 : N == 6 ? 64 : N == 5 ? (nodal ? 256 : 128) : N == 4 ? 128 : 256;
 }
 
 // Tuned tiles: the stage kernel (affine metrics, RK update) of SW at N = 3, 5, 7 and of LSW
@@ -1865,12 +1868,12 @@ struct Launcher {
     switch (N) {
 #define CASE(NN_)                                                                                     \
   case NN_: {                                                                                         \
-    constexpr int T = tile_threads<NN_>();                                                            \
-    constexpr int EPB = T / ((NN_ + 1) * (NN_ + 1));                                                  \
+    constexpr int T = tile_threads<NN_>(), TNOD = tile_threads<NN_>(true);                            \
+    const int EPB = (nodal ? TNOD : T) / ((NN_ + 1) * (NN_ + 1));                                     \
     dim3 grid((a.nEl + EPB - 1) / EPB);                                                               \
     if (nodal) {                                                                                      \
-      if (mode == 0) hipLaunchKernelGGL((k_fused<Phys, NN_, 0, true, T>), grid, T, 0, st, a);         \
-      else hipLaunchKernelGGL((k_fused<Phys, NN_, 1, true, T>), grid, T, 0, st, a);                   \
+      if (mode == 0) hipLaunchKernelGGL((k_fused<Phys, NN_, 0, true, TNOD>), grid, TNOD, 0, st, a);   \
+      else hipLaunchKernelGGL((k_fused<Phys, NN_, 1, true, TNOD>), grid, TNOD, 0, st, a);             \
     } else {                                                                                          \
       if (mode == 0) hipLaunchKernelGGL((k_fused<Phys, NN_, 0, false, T>), grid, T, 0, st, a);        \
       else hipLaunchKernelGGL((k_fused<Phys, NN_, 1, false, T>), grid, T, 0, st, a);                  \
