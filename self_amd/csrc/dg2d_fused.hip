@@ -46,6 +46,9 @@ constexpr int kDirectSteps = 2;
 // steps from kResidentElements elements on: below, a cooperative launch of three stages costs what
 // it saves (N = 7: 28.8 against 28.3 us per call at 10^2 elements, 31.9 against 34.1 at 40^2).
 constexpr int kResidentSteps = 2, kResidentElements = 1024;
+// Longer calls are several resident launches (27 ms each at 10^2 elements of degree 7, against some
+// 10 us for a launch), so that other streams get the device in between.
+constexpr int kResidentLaunchSteps = 4096;
 
 // Williamson low-storage RK3 (src/SELF_Model.f90:25-27)
 constexpr double kRk3A[3] = {0.0, -5.0 / 9.0, -153.0 / 128.0};
@@ -1052,10 +1055,10 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // 3.3 us (9.5 us per stage).  A call of one step takes 78 us with set and get, 110 in launches.
 //
 // All blocks must be resident: the launch is cooperative, which the runtime refuses if they
-// cannot be.  Every wait is bounded as well: a lane that has polled kPollBudget times in a call
-// stops waiting and raises `timedOut`, which the next synchronising call reports.
+// cannot be.  Every wait is bounded as well: a lane that has polled kPollBudget times in one wait
+// (seconds) waits no more and raises `timedOut`, which the next synchronising call reports.
 constexpr unsigned long long kEmpty = 0x7FF0DEAD7FF0DEADull;
-constexpr int kPollBudget = 1 << 20;
+constexpr int kPollBudget = 1 << 22;
 
 struct ResidentArgs {
   unsigned long long *ring;  // 3 buffers (0:N, NX, 4, nEl)
@@ -1386,6 +1389,7 @@ k_resident(const FusedArgs a, const ResidentArgs ra, const ResidentNetArgs na) {
   for (int m = 0; m < ra.stages; m++) {
     const bool last = m == ra.stages - 1;
     const int before = fill == 0 ? 2 : fill - 1, empty = fill == 2 ? 0 : fill + 1;  // (m - 1), (m - 2) mod 3
+    if (budget >= 0) budget = kPollBudget;
     if (nodeActive) {
       double fx[NV], fy[NV], q[NT];
       Phys::volume(s, auxVal, a.p, fx, fy, q);
@@ -2158,6 +2162,8 @@ using Model = selfamd_model2d;
 
 bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
   if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || (timedOut && *timedOut)) return false;
+  int current = -1;  // the ring is allocated on the current device
+  if (hipGetDevice(&current) != hipSuccess || current != device) return false;
   // the 64-wide tile of nonlinear SW at N = 5 splits the face sums; the resident kernel does not
   if (kind == SELFAMD_MODEL_SW && N == 5 && tile_splits5(tile_of(kind, 5))) return false;
   // blocks of k that the device holds at once, `of` 16ths of them
@@ -2487,6 +2493,15 @@ static bool device_doubles(const selfamd_model2d *m, const void *p) {
   return at.type == hipMemoryTypeDevice && at.device == m->device;
 }
 
+namespace {
+// after the model's stream has been waited for
+int resident_status(const selfamd_model2d *m) {
+  SELFAMD_REQUIRE(!m->timedOut || !*m->timedOut,
+                  "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
+  return kOk;
+}
+}  // namespace
+
 int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   SELFAMD_REQUIRE(m && interior, "model2d_set_solution: null argument");
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
@@ -2499,6 +2514,10 @@ int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   if (!direct) SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(m->launch_state_in(direct ? interior : m->S));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  if (m->timedOut && *m->timedOut) {  // a valid state again; the exchange ring is emptied before its next use
+    *m->timedOut = 0;
+    m->ringValues = 0;
+  }
   return kOk;
 }
 
@@ -2507,7 +2526,7 @@ int selfamd_model2d_get_solution(selfamd_model2d *m, double *interior) {
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
   SELFAMD_HIP(hipMemcpyAsync(interior, m->S, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 // integral of the current state over the mesh (the integrand kind, and the variable for
@@ -2542,7 +2561,7 @@ static int model_integral(selfamd_model2d *m, int what, int var, double *value, 
   SELFAMD_CHECK_LAUNCH();
   SELFAMD_HIP(hipMemcpyAsync(value, m->intScratch + nBlocks, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 namespace {
@@ -2620,7 +2639,7 @@ int selfamd_model2d_tendency(selfamd_model2d *m, double *dSdt) {
                                hipMemcpyDeviceToDevice, m->stream));
   }
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 int selfamd_model2d_flux_registers(selfamd_model2d *m, double *fluxDivergence, double *flux) {
@@ -2634,15 +2653,10 @@ int selfamd_model2d_flux_registers(selfamd_model2d *m, double *fluxDivergence, d
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   (void)hipFree(scratch);
   SELFAMD_HIP(e);
-  return kOk;
+  return resident_status(m);
 }
 
 namespace {
-int resident_status(const selfamd_model2d *m) {
-  SELFAMD_REQUIRE(!m->timedOut || !*m->timedOut,
-                  "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
-  return kOk;
-}
 // a few steps of another size than the captured graphs' (e.g. ForwardStep's shorter last step
 // up to tn) are launched directly, so the graphs of the running step size survive
 bool direct_steps(const selfamd_model2d *m, int nSteps, double dt) {
@@ -2683,7 +2697,13 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   if (nSteps == 0) return kOk;
   ResidentKernel kernel;
   if (m->resident(nSteps, kernel)) {
-    if (m->launch_resident(kernel, nSteps, dt) == hipSuccess) return kOk;
+    hipError_t e = hipSuccess;
+    while (e == hipSuccess && nSteps > 0) {
+      const int n = std::min(nSteps, kResidentLaunchSteps);
+      e = m->launch_resident(kernel, n, dt);
+      if (e == hipSuccess) nSteps -= n;
+    }
+    if (nSteps == 0) return kOk;
     // not accepted by the runtime: step graphs from here on
     (void)hipGetLastError();
     for (auto &blocks : m->residentBlocks)
@@ -2745,7 +2765,7 @@ int selfamd_model2d_time_steps(selfamd_model2d *m, int nSteps, double dt, double
   *elapsedMs = ms;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  return kOk;
+  return resident_status(m);
 }
 
 int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const float *inMean, const float *inScale,
