@@ -185,8 +185,10 @@ constexpr int kRowMaxHidden = 256, kRowMaxOut = 256, kRowLds = 56 * 1024;  // 64
 
 // kRowsForward: Y = net(X).  kRowsLoss: forward, dY = 2 (Y - T) / count, backward.
 // kRowsBackward: forward, backward from the cotangent T.  kRowsClosure: features of the state,
-// forward, FP64 correction and its mass integral.
-enum RowsMode { kRowsForward, kRowsLoss, kRowsBackward, kRowsClosure };
+// forward, FP64 correction and its mass integral.  kRowsClosureVjp: features of the state (also to
+// Xout) and the output cotangent of the correction's cotangent lam (also to dY), forward, backward,
+// and the state cotangent added to mu.
+enum RowsMode { kRowsForward, kRowsLoss, kRowsBackward, kRowsClosure, kRowsClosureVjp };
 
 struct RowsArgs {
   int nIn, nH, nO, B;
@@ -199,6 +201,12 @@ struct RowsArgs {
   const float *inMean, *inScale, *outMean, *outScale;
   double *corr, *massParts;
   int P, nVar, massVar;
+  // kRowsClosureVjp: lamParts[nLamParts] add up to the sum of lam's mass variable over the mesh
+  const double *lam, *lamParts;
+  int nLamParts;
+  double invArea;
+  float *Xout;
+  double *mu;
 };
 
 inline size_t rows_lds(int nIn, int nH, int nO) {
@@ -252,7 +260,9 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches on it
   const int row0 = blockIdx.x * kRowTile;
-  constexpr bool BACK = MODE == kRowsLoss || MODE == kRowsBackward;
+  constexpr bool VJP = MODE == kRowsClosureVjp, STATE = MODE == kRowsClosure || VJP;  // rows of a model's state
+  constexpr bool GIVEN = MODE == kRowsBackward || VJP;                               // a given output cotangent
+  constexpr bool BACK = MODE == kRowsLoss || GIVEN;
   const RowsOperand w1{a.W1, a.nH, a.nIn, a.nH}, w2{a.W2, a.nH, a.nH, a.nH}, w3{a.W3, a.nO, a.nH, a.nO};
   const RowsOperand t3{a.W3, a.nO, a.nO, a.nH}, t2{a.W2, a.nH, a.nH, a.nH}, t1{a.W1, a.nH, a.nH, a.nIn};
   const int n0 = wave * 16 + r;  // this lane's column of the wavefront's first tile of a layer
@@ -290,7 +300,7 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const int kk = min(k + 32 * j, a.nIn - 1);
-        if constexpr (MODE == kRowsClosure) {
+        if constexpr (STATE) {
           const double *gr = a.geom + e * kGeomStride;
           raw[j] = *(kk < nS ? a.S + e * nS + kk : kk == nS ? gr + 4 : kk == nS + 1 ? gr : gr + 3);
           mu[j] = a.inMean[kk];
@@ -301,8 +311,35 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
       }
 #pragma unroll
       for (int j = 0; j < 2; j++) {
-        if constexpr (MODE == kRowsClosure) x[j] = (float)((raw[j] - (double)mu[j]) / (double)sd[j]);
+        if constexpr (STATE) x[j] = (float)((raw[j] - (double)mu[j]) / (double)sd[j]);
         sX[row * a.ldX + k + 32 * j] = ok && k + 32 * j < a.nIn ? x[j] : 0.f;
+        if constexpr (VJP)
+          if (ok && k + 32 * j < a.nIn) a.Xout[e * a.nIn + k + 32 * j] = x[j];
+      }
+    }
+    if constexpr (VJP) {
+      // every wavefront adds the partial sums itself, in flight beside its other loads
+      double total = 0.0;
+      for (int k = lane; k < a.nLamParts; k += 256) {
+        double t[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) t[j] = a.lamParts[min(k + 64 * j, a.nLamParts - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; j++) total += k + 64 * j < a.nLamParts ? t[j] : 0.0;
+      }
+      for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+      // Forward: corr_k = y_k outScale_k + outMean_k, and for the mass variable corr' = corr - invArea
+      // sum_n omega_n corr_n (omega = w_i w_j J); so dY_k = outScale_k (lam_k - omega_k invArea
+      // sum_n lam_n) on the mass variable, outScale_k lam_k elsewhere.
+      const double J = a.geom[e * kGeomStride + 4];
+      for (int k = c; k < O16; k += 32) {
+        const int kk = min(k, a.nO - 1), node = kk - a.massVar * a.P * a.P;
+        double l = a.lam[e * a.nO + kk];
+        if (node >= 0 && node < a.P * a.P) l -= a.qW[node % a.P] * a.qW[node / a.P] * J * a.invArea * total;
+        const float d = (float)(l * (double)a.outScale[kk]);
+        const bool in = ok && k < a.nO;
+        sO[row * a.ldO + k] = in ? d : 0.f;
+        if (in) a.dY[e * a.nO + k] = d;
       }
     }
     for (int k = H16 + c; k < KH; k += 32) sH1[row * a.ldH + k] = sH2[row * a.ldH + k] = 0.f;
@@ -357,10 +394,10 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
   hidden(sX, a.ldX, w1, bias1, sH1, a.H1, gp1, [&](float (&x)[16]) { rows_load<false, VEC>(w2, n0, g, 0, x); });
   __syncthreads();
   hidden(sH1, a.ldH, w2, bias2, sH2, a.H2, gp2, [&](float (&x)[16]) {
-    if constexpr (MODE == kRowsBackward) rows_load<true, VEC>(t3, n0, g, 0, x);
+    if constexpr (GIVEN) rows_load<true, VEC>(t3, n0, g, 0, x);
     else rows_load<false, VEC>(w3, n0, g, 0, x);
   });
-  if constexpr (MODE != kRowsBackward) __syncthreads();
+  if constexpr (!GIVEN) __syncthreads();
 
   // output layer
   float loss = 0.f;
@@ -370,7 +407,7 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
     const bool ok = row0 + row < a.B;
     for (int k = tid & 31; k < O16; k += 32)
       sO[row * a.ldO + k] = ok && k < a.nO ? a.T[(size_t)(row0 + row) * a.nO + k] : 0.f;
-  } else {
+  } else if constexpr (!VJP) {
     for (int ct = wave; ct * 16 < O16; ct += kRowWaves) {
       const int n = ct * 16 + r;
       const bool nok = n < a.nO;
@@ -450,17 +487,29 @@ __global__ void __launch_bounds__(kRowThreads) k_mlp_rows(const RowsArgs a) {
     back(sO, a.ldO, t3, sH2, a.D2, gp2, [&](float (&x)[16]) { rows_load<true, VEC>(t2, n0, g, 0, x); });
     __syncthreads();
     back(sH2, a.ldH, t2, sH1, a.D1, gp1, [&](float (&x)[16]) {
-      if constexpr (MODE == kRowsBackward) rows_load<true, VEC>(t1, n0, g, 0, x);
+      if constexpr (GIVEN) rows_load<true, VEC>(t1, n0, g, 0, x);
     });
-    if (MODE == kRowsLoss || !a.dX) return;
+    if (MODE == kRowsLoss || (!VJP && !a.dX)) return;
     __syncthreads();
-    for (int ct = wave; ct * 16 < a.nIn; ct += kRowWaves) {
+    // the metric inputs, past the nodal ones, do not depend on the state
+    const int nX = VJP ? a.nO : a.nIn;
+    for (int ct = wave; ct * 16 < nX; ct += kRowWaves) {
       const int n = ct * 16 + r;
+      double m[4], sd = 1.0;
+      if constexpr (VJP) {
+        const int nn = min(n, nX - 1);
+        sd = (double)a.inScale[nn];
+#pragma unroll
+        for (int i = 0; i < 4; i++) m[i] = a.mu[(size_t)min(row0 + 4 * g + i, a.B - 1) * nX + nn];
+      }
       if (ct != wave) rows_load<true, VEC>(t1, n, g, 0, b[0]);
       const f32x4 acc = rows_tile<true, VEC>(sH1, a.ldH, t1, n, lane, b[0], [] {});
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        if (n < a.nIn && row0 + 4 * g + i < a.B) a.dX[(size_t)(row0 + 4 * g + i) * a.nIn + n] = acc[i];
+        if (n < nX && row0 + 4 * g + i < a.B) {
+          if constexpr (VJP) a.mu[(size_t)(row0 + 4 * g + i) * nX + n] = m[i] + (double)acc[i] / sd;
+          else a.dX[(size_t)(row0 + 4 * g + i) * nX + n] = acc[i];
+        }
     }
   }
 }
@@ -574,14 +623,14 @@ hipError_t launch_rows(const RowsArgs &a, hipStream_t st) {
   const size_t lds = rows_lds(a.nIn, a.nH, a.nO);
   // the transposed weights of the backward pass are read 16 bytes at a time where every row of
   // W1, W2 and W3 is 16-byte aligned
-  const bool back = MODE == kRowsLoss || MODE == kRowsBackward;
+  constexpr bool back = MODE == kRowsLoss || MODE == kRowsBackward || MODE == kRowsClosureVjp;
   const bool vec = back && a.nH % 4 == 0 && a.nO % 4 == 0 &&
                    ((reinterpret_cast<uintptr_t>(a.W1) | reinterpret_cast<uintptr_t>(a.W2) |
                      reinterpret_cast<uintptr_t>(a.W3)) & 15) == 0;
   const bool one = a.nH <= 16 * kRowWaves;
   if (one && !vec) hipLaunchKernelGGL((k_mlp_rows<MODE, 1, false>), blocks, kRowThreads, lds, st, a);
   else if (!vec) hipLaunchKernelGGL((k_mlp_rows<MODE, 2, false>), blocks, kRowThreads, lds, st, a);
-  else if constexpr (MODE == kRowsLoss || MODE == kRowsBackward) {
+  else if constexpr (back) {
     if (one) hipLaunchKernelGGL((k_mlp_rows<MODE, 1, true>), blocks, kRowThreads, lds, st, a);
     else hipLaunchKernelGGL((k_mlp_rows<MODE, 2, true>), blocks, kRowThreads, lds, st, a);
   }
@@ -1176,12 +1225,29 @@ hipError_t closure_vjp(const ClosureBuffers &c, const double *S, const double *g
                        const double *lam, double *mu, int N, int nVar, int massVar, int nEl, hipStream_t st) {
   hipError_t e;
   const int NN = (N + 1) * (N + 1);
-  if ((e = closure_features(S, geom, c.inMean, c.inScale, c.X, N, nVar, nEl, st)) != hipSuccess) return e;
   const size_t nNodes = (size_t)NN * nEl, nb = (nNodes + kVjpBlock - 1) / kVjpBlock;
   hipLaunchKernelGGL(k_vjp_mass_partial, (unsigned)nb, kVjpBlock, 0, st, lam, c.vjpPartial, NN, nVar, massVar, nNodes);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_vjp_sum, 1, kVjpBlock, 0, st, c.vjpPartial, (int)nb);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  // As for the mean correction, a few hundred partial sums are added where they are used.
+  const bool sum = !c.mlp->rows || nb > (size_t)kShiftParts;
+  if (sum) {
+    hipLaunchKernelGGL(k_vjp_sum, 1, kVjpBlock, 0, st, c.vjpPartial, (int)nb);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (c.mlp->rows) {
+    // One launch for features, output cotangent, network and state cotangent.  64 x 64 elements of
+    // N = 3, 51 -> 128 -> 128 -> 48: 17.6 us where the network's launch took 15.3 and four more
+    // 12 us and a launch each; the adjoint of a stage with its reads 139 -> 125 us.
+    RowsArgs a = rows_args(c.mlp, nullptr, nEl);
+    a.S = S; a.geom = geom; a.qW = qW; a.lam = lam; a.mu = mu;
+    a.inMean = c.inMean; a.inScale = c.inScale; a.outScale = c.outScale;
+    a.P = N + 1; a.nVar = nVar; a.massVar = massVar; a.invArea = c.invArea;
+    a.lamParts = c.vjpPartial + (sum ? nb : 0); a.nLamParts = sum ? 1 : (int)nb;
+    a.Xout = c.X; a.dY = c.dY;
+    if ((e = launch_rows<kRowsClosureVjp>(a, st)) != hipSuccess) return e;
+    return weight_grads_rows(c.mlp, c.X, c.dY, nEl, 1, st);
+  }
+  if ((e = closure_features(S, geom, c.inMean, c.inScale, c.X, N, nVar, nEl, st)) != hipSuccess) return e;
   const size_t n = (size_t)c.nOut * nEl;
   const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 65535);
   hipLaunchKernelGGL(k_vjp_dY, blocks, 256, 0, st, lam, c.vjpPartial + nb, c.outScale, geom, qW, c.dY, N, nVar, massVar,
