@@ -148,6 +148,7 @@ __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float
 struct selfamd_mlp {
   int nIn = 0, nH = 0, nOut = 0, maxB = 0;
   size_t nParams = 0;
+  float *memory = nullptr;  // all arrays below
   float *params = nullptr, *grads = nullptr, *m1 = nullptr, *m2 = nullptr;  // packed W1 b1 W2 b2 W3 b3
   float *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Y = nullptr, *dY = nullptr;
   float *D2 = nullptr, *D1 = nullptr, *parts = nullptr, *lossParts = nullptr;
@@ -743,20 +744,27 @@ int selfamd_mlp_create(selfamd_mlp **out, int nIn, int nHidden, int nOut, int ma
   m->nParams = (size_t)nIn * nHidden + nHidden + (size_t)nHidden * nHidden + nHidden + (size_t)nHidden * nOut + nOut;
   const size_t B = maxBatch, H = nHidden;
   m->rows = rows_fit(nIn, nHidden, nOut);
+  // One allocation for all arrays (a call each takes longer than the kernels of a training step),
+  // each 256-byte aligned; the partial gradients are of at most 64 splits of at least 128 rows.
   const size_t lossBlocks = std::max<size_t>(1024, (B + kRowTile - 1) / kRowTile);
-  float **bufs[] = {&m->params, &m->grads, &m->m1, &m->m2};
-  bool ok = true;
-  for (float **b : bufs) ok = ok && hipMalloc(b, 4 * m->nParams) == hipSuccess;
-  ok = ok && hipMalloc(&m->H1, 4 * B * H) == hipSuccess && hipMalloc(&m->H2, 4 * B * H) == hipSuccess &&
-       hipMalloc(&m->Y, 4 * B * nOut) == hipSuccess && hipMalloc(&m->dY, 4 * B * nOut) == hipSuccess &&
-       hipMalloc(&m->D2, 4 * B * H) == hipSuccess && hipMalloc(&m->D1, 4 * B * H) == hipSuccess &&
-       hipMalloc(&m->parts, 4 * m->nParams * m->splitsMax) == hipSuccess &&
-       hipMalloc(&m->lossParts, 4 * lossBlocks) == hipSuccess;
-  if (!m->rows)
-    ok = ok && hipMalloc(&m->Z1, 4 * B * H) == hipSuccess && hipMalloc(&m->Z2, 4 * B * H) == hipSuccess &&
-         hipMalloc(&m->ones, 4 * B) == hipSuccess;
-  if (ok) ok = hipMemset(m->m1, 0, 4 * m->nParams) == hipSuccess && hipMemset(m->m2, 0, 4 * m->nParams) == hipSuccess &&
-               hipMemset(m->params, 0, 4 * m->nParams) == hipSuccess;
+  const size_t splits = std::min<size_t>(m->splitsMax, (B + 127) / 128), general = m->rows ? 0 : B;
+  const struct { float **at; size_t n; } arrays[] = {
+      {&m->params, m->nParams}, {&m->m1, m->nParams}, {&m->m2, m->nParams}, {&m->grads, m->nParams},
+      {&m->H1, B * H}, {&m->H2, B * H}, {&m->Y, B * nOut}, {&m->dY, B * nOut}, {&m->D2, B * H}, {&m->D1, B * H},
+      {&m->parts, m->nParams * splits}, {&m->lossParts, lossBlocks},
+      {&m->Z1, general * H}, {&m->Z2, general * H}, {&m->ones, general}};
+  auto padded = [](size_t n) { return (n + 63) & ~(size_t)63; };
+  size_t total = 0;
+  for (const auto &a : arrays) total += padded(a.n);
+  bool ok = hipMalloc(&m->memory, 4 * total) == hipSuccess;
+  if (ok) {
+    float *p = m->memory;
+    for (const auto &a : arrays) {
+      *a.at = a.n ? p : nullptr;
+      p += padded(a.n);
+    }
+    ok = hipMemset(m->params, 0, 4 * 3 * padded(m->nParams)) == hipSuccess;  // params, m1, m2
+  }
   if (ok) {
     if (m->ones)
       hipLaunchKernelGGL(k_fill, (unsigned)std::min<size_t>((B + 255) / 256, 4096), 256, 0, nullptr, m->ones, 1.0f, B);
@@ -773,10 +781,7 @@ int selfamd_mlp_create(selfamd_mlp **out, int nIn, int nHidden, int nOut, int ma
 
 int selfamd_mlp_destroy(selfamd_mlp *m) {
   if (!m) return kOk;
-  float *bufs[] = {m->params, m->grads, m->m1, m->m2, m->Z1, m->H1, m->Z2, m->H2, m->Y, m->dY, m->D2, m->D1,
-                   m->parts, m->lossParts, m->ones};
-  for (float *b : bufs)
-    if (b) (void)hipFree(b);
+  if (m->memory) (void)hipFree(m->memory);
   delete m;
   return kOk;
 }
