@@ -897,11 +897,10 @@ namespace {
 // One block per coarse element.  The fine rows of elements are read as the contiguous runs they
 // are (r nVar Pf^2 doubles per sub-row b), `rowsB` sub-rows at a time, into LDS; then
 // row[b][v][q][i] = sum_a,p Px[a][i][p] u, and u_c += sum_b,q Px[b][j][q] row.  Bound by reading
-// the fine state: 104 MB (256^2 N = 7, three variables) in 38 us (2.7 TB/s: a block's loads and
+// the fine state: 104 MB (256^2 N = 7, three variables) in 24 us (4.3 TB/s: a block's loads and
 // sums do not overlap, five blocks per CU do), where one work-item per coarse value, each reading
-// r^2 Pf^2 doubles with its neighbours 64 bytes or whole elements away, took 276 us.  Chunks of
-// half the size, for twice the blocks per CU, run at the same 38 us, a quarter at 60 us.  LDS rows of Pf doubles are padded by one: four of five rows would share banks at
-// Pf = 8.
+// r^2 Pf^2 doubles with its neighbours 64 bytes or whole elements away, took 276 us.  LDS rows of Pf
+// doubles are padded by one: four of five rows would share banks at Pf = 8.
 constexpr int kProjectArgs = 448, kProjectLds = 6144, kProjectChunk = 3072;  // doubles
 struct ProjectArgs {
   const double *fine;
@@ -914,11 +913,12 @@ static_assert(sizeof(ProjectArgs) <= 4096, "kernel arguments exceed the 4 KiB ke
 
 // PC = Pc with the sums of one LDS row for all i in one work-item (the factors are uniform and
 // come in scalar registers), where one sum per work-item reads every u Pc times; PC = 0: one sum
-// per work-item, for other degrees.
-template <int PC>
+// per work-item, for other degrees.  PF = Pf, so that the LDS reads of a row's sum are in flight at
+// once: with a loop over Pf (PF = 0, other degrees) every term waits for its own, 37 us.
+template <int PC, int PF>
 __global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
   extern __shared__ double projectLds[];
-  const int tid = threadIdx.x, Pf = a.Pf, Pc = a.Pc, r = a.r, nVar = a.nVar, nPx = r * Pc * Pf, ld = Pf + 1;
+  const int tid = threadIdx.x, Pf = PF > 0 ? PF : a.Pf, Pc = PC > 0 ? PC : a.Pc, r = a.r, nVar = a.nVar, nPx = r * Pc * Pf, ld = Pf + 1;
   const int run = r * nVar * Pf * Pf, rows = r * nVar * Pf, nOut = nVar * Pc * Pc, perB = nVar * Pf * Pc;
   double *sPx = projectLds, *sU = sPx + nPx, *sRow = sU + a.rowsB * rows * ld, *sOut = sRow + a.rowsB * perB;
   const int I = blockIdx.x % a.nxc, J = blockIdx.x / a.nxc;
@@ -953,6 +953,7 @@ __global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
         double row[PC] = {};
         for (int aa = 0; aa < r; aa++) {
           const double *u = sU + (b * rows + aa * nVar * Pf + vq) * ld, *px = a.px + aa * PC * Pf;
+#pragma unroll
           for (int p = 0; p < Pf; p++) {
             const double x = u[p];
 #pragma unroll
@@ -976,6 +977,7 @@ __global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
       const int i = t % Pc, j = t / Pc % Pc, v = t / (Pc * Pc);
       double acc = sOut[t];
       for (int b = 0; b < nb; b++)
+#pragma unroll
         for (int q = 0; q < Pf; q++) acc += sPx[((b0 + b) * Pc + j) * Pf + q] * sRow[b * perB + (v * Pf + q) * Pc + i];
       sOut[t] = acc;
     }
@@ -1296,13 +1298,21 @@ int selfamd_project_l2_structured_2d(const double *fine, double *coarse, int Nf,
     const size_t lds = nPx + (size_t)g.rowsB * r * nVar * Pf * (Pf + 1) + (size_t)g.rowsB * nVar * Pf * Pc + (size_t)nVar * Pc * Pc;
     if (sizeof(double) * lds <= 64 * 1024) {
       const unsigned blocks = (unsigned)((size_t)nxc * nyc);
+      auto run_as = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, 256, sizeof(double) * lds, st, g); };
+#define CASE_F(PC, PF) case PF: run_as(k_project<PC, PF>); break;
+#define CASE(PC)                                                                                        \
+  case PC:                                                                                              \
+    switch (Pf) {                                                                                       \
+      CASE_F(PC, 3) CASE_F(PC, 4) CASE_F(PC, 5) CASE_F(PC, 6) CASE_F(PC, 7) CASE_F(PC, 8)               \
+      default: run_as(k_project<PC, 0>);                                                                \
+    }                                                                                                   \
+    break;
       switch (Pc) {
-#define CASE(PC) \
-  case PC: hipLaunchKernelGGL(k_project<PC>, blocks, 256, sizeof(double) * lds, st, g); break;
         CASE(2) CASE(3) CASE(4) CASE(5) CASE(6)
-#undef CASE
-        default: hipLaunchKernelGGL(k_project<0>, blocks, 256, sizeof(double) * lds, st, g);
+        default: run_as(k_project<0, 0>);
       }
+#undef CASE
+#undef CASE_F
       SELFAMD_HIP(hipGetLastError());
       SELFAMD_HIP(hipStreamSynchronize(st));
       return kOk;
