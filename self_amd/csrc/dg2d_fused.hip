@@ -46,6 +46,9 @@ constexpr int kDirectSteps = 2;
 // steps from kResidentElements elements on: below, a cooperative launch of three stages costs what
 // it saves (N = 7: 28.8 against 28.3 us per call at 10^2 elements, 31.9 against 34.1 at 40^2).
 constexpr int kResidentSteps = 2, kResidentElements = 1024;
+// Instances whose registers spill pay for it once per call: from this many steps on (SW N = 3,
+// 18,400 elements: 60 against 49 us for one step, 10.2 against 11.3 us per stage).
+constexpr int kResidentSpillSteps = 5;
 // Longer calls are several resident launches (27 ms each at 10^2 elements of degree 7, against some
 // 10 us for a launch), so that other streams get the device in between.
 constexpr int kResidentLaunchSteps = 4096;
@@ -1031,8 +1034,8 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // The arithmetic and its order are the stage kernel's, so the results are the same bits.
 // Measured per stage (200-step and 24-step calls): linear SW 10^2 N = 7 4.1 -> 2.2 us, 45 x 37 N = 6
 // 8.6 -> 3.0 us, Euler 93 x 61 N = 4 19 -> 9 us.  Instances: WPE = 1 leaves the registers to the
-// compiler and unrolls the divergence; where the mesh needs more blocks than fit that way, 3 or 4
-// wavefronts per SIMD (twice the elements).
+// compiler and unrolls the divergence; where the mesh needs more blocks than fit that way, 3, 4 or 5
+// wavefronts per SIMD (twice the elements and more).
 //
 // Exchange: ring buffer m mod 3 takes stage m's traces (and lagged velocities).  Every value is its
 // own flag: a slot holds kEmpty, a signalling NaN that no arithmetic produces, until its owner
@@ -1921,12 +1924,25 @@ struct ResidentKernel {
   const void *fn = nullptr;
   int threads = 0, elements = 0, values = 0;  // per block: work-items, elements; ring values per face node
 };
+// dense 1, 2, 3: instances held to the registers of 3, 4 and 5 wavefronts per SIMD, for more resident
+// blocks.  Per stage of 20-step calls, stage launches against resident ones: 4 wavefronts, SW 64^2
+// N = 7 9.7 and 6.0 us, N = 5 6,000 elements 11.1 and 5.9, linear SW 128^2 N = 3 12.2 and 8.2; 5
+// wavefronts (4,096 to 5,120 blocks), SW N = 7 12.1 and 8.1, N = 3 11.3 and 10.2, linear SW N = 7 10.6
+// and 5.9, N = 2 13.7 and 10.2.  SW with 5 wavefronts loses at N = 1 (12.6 and 15.6) and gains
+// nothing at N = 2 on nodal metrics, linear SW at N = 1 neither; Euler needs more registers or LDS.
+constexpr int kResidentDense = 4;
 template <class Phys, int N, bool NODAL>
 ResidentKernel resident_instance(int dense) {
   using L = ResidentTile<Phys, N, NODAL>;
-  const void *fn = dense == 2   ? reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 4>)
-                   : dense == 1 ? reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 3>)
-                                : reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 1>);
+  constexpr bool FIVE = Phys::NV == 3 && (N >= 3 || (N == 2 && !Phys::kLag));
+  const void *fn = nullptr;
+  switch (dense) {
+    case 0: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 1>); break;
+    case 1: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 3>); break;
+    case 2: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 4>); break;
+    case 3:
+      if constexpr (FIVE) fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 5>);
+  }
   return {fn, L::T, L::EPB, L::NX};
 }
 template <class Phys, bool NODAL>
@@ -1959,8 +1975,6 @@ ResidentKernel resident_net_kernel(int kind, int N) {
     default: return resident_net_of<PhysEuler>(N);
   }
 }
-// dense 1, 2: instances held to the registers of 3 and 4 wavefronts per SIMD, for more resident blocks
-constexpr int kResidentDense = 3;
 ResidentKernel resident_kernel(int kind, int N, bool nodal, int dense) {
   switch (kind) {
     case SELFAMD_MODEL_SW: return nodal ? resident_of<PhysSW, true>(N, dense) : resident_of<PhysSW, false>(N, dense);
@@ -2019,13 +2033,14 @@ struct selfamd_model2d {
   std::vector<int32_t> hnbr;      // host copy of the neighbour codes
 
   // resident stepping: the exchange ring (allocated on first use), the blocks that can be
-  // resident at once (15 of 16 of the device's; -1: not asked yet; 0: not available), the
+  // resident at once (-1: not asked yet; 0: not available), the
   // host flag that a launch raises when a wait ran out
   unsigned long long *ring = nullptr;
   size_t ringLen = 0;
   int ringValues = 0;  // values per face node of the slot layout the ring was emptied for
-  int residentBlocks[2][kResidentDense] = {{-1, -1, -1}, {-1, -1, -1}};  // [nodal][dense]
-  int residentNetBlocks = -1;  // with a closure
+  int residentBlocks[2][kResidentDense] = {{-1, -1, -1, -1}, {-1, -1, -1, -1}};  // [nodal][dense]
+  bool residentSpills[2][kResidentDense] = {};  // whether those instances' registers spill
+  int residentNetBlocks = -1;                   // with a closure
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
   int *timedOut = nullptr;
 
@@ -2042,8 +2057,8 @@ struct selfamd_model2d {
     a.p = p;
     return a;
   }
-  // Whether a call of nSteps steps runs as one resident launch: the mesh's blocks are all resident
-  // at once with room to spare, and the stages saved pay for a cooperative launch.
+  // Whether a call of nSteps steps runs as resident launches: the mesh's blocks are all resident
+  // at once, and the stages saved pay for a cooperative launch.
   // Sets the kernel to launch.
   bool resident(int nSteps, ResidentKernel &k);
   int mass_stride(const ResidentKernel &k) const { return ((nEl + k.elements - 1) / k.elements + 511) & ~511; }
@@ -2166,8 +2181,8 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
   if (hipGetDevice(&current) != hipSuccess || current != device) return false;
   // the 64-wide tile of nonlinear SW at N = 5 splits the face sums; the resident kernel does not
   if (kind == SELFAMD_MODEL_SW && N == 5 && tile_splits5(tile_of(kind, 5))) return false;
-  // blocks of k that the device holds at once, `of` 16ths of them
-  auto capacity = [&](int &blocks, int of) {
+  // whether the device holds k's blocks at once; their number and whether k spills are asked once
+  auto capacity = [&](int &blocks, bool &spills) {
     if (blocks < 0) {
       int cus = 0, perCU = 0, coop = 0;
       if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
@@ -2176,19 +2191,30 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
         (void)hipGetLastError();
         perCU = 0;
       }
-      blocks = coop ? cus * perCU * of / 16 : 0;
+      hipFuncAttributes at{};
+      if (hipFuncGetAttributes(&at, k.fn) != hipSuccess) {
+        (void)hipGetLastError();
+        perCU = 0;
+      }
+      spills = at.localSizeBytes > 0;
+      blocks = coop ? cus * perCU : 0;
+      // Euler at N = 2 on a full device: 3,060 blocks 17.1 us per stage, in launches 15.9; 2,600 blocks
+      // 10.2 and 14.1
+      if (kind == SELFAMD_MODEL_EULER && N == 2) blocks -= blocks / 8;
     }
+    if (spills && !closure && nSteps < kResidentSpillSteps) return false;  // a closure's launch pays from one step on
     return (nEl + k.elements - 1) / k.elements <= blocks;
   };
   bool fits = false;
   if (closure) {
+    bool netSpills = false;
     k = resident_net_kernel(kind, N);
     const MlpWeights w = mlp_weights(closure->mlp);
-    fits = k.fn && !nodal && w.rows && w.nH <= kResidentHidden && capacity(residentNetBlocks, 16);
+    fits = k.fn && !nodal && w.rows && w.nH <= kResidentHidden && capacity(residentNetBlocks, netSpills);
   } else {
     for (int dense = 0; dense < kResidentDense && !fits; dense++) {
       k = resident_kernel(kind, N, nodal, dense);
-      fits = capacity(residentBlocks[nodal][dense], 15);
+      fits = k.fn && capacity(residentBlocks[nodal][dense], residentSpills[nodal][dense]);
     }
   }
   if (!fits) return false;
