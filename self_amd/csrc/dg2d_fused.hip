@@ -1033,7 +1033,7 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 //              of the new state -> registers and the exchange ring.
 // The arithmetic and its order are the stage kernel's, so the results are the same bits.
 // Measured per stage (200-step and 24-step calls): linear SW 10^2 N = 7 4.1 -> 2.2 us, 45 x 37 N = 6
-// 8.6 -> 3.0 us, Euler 93 x 61 N = 4 19 -> 9 us.  Instances: WPE = 1 leaves the registers to the
+// 8.6 -> 3.0 us, Euler 93 x 61 N = 4 19 -> 7 us.  Instances: WPE = 1 leaves the registers to the
 // compiler and unrolls the divergence; where the mesh needs more blocks than fit that way, 3, 4 or 5
 // wavefronts per SIMD (twice the elements and more).
 //
