@@ -319,7 +319,9 @@ int selfamd_model2d_integral(selfamd_model2d *model, int var, double *value);
 int selfamd_model2d_integral_noalloc(selfamd_model2d *model, int var, double *value_dev);
 /* nSteps full low-storage RK3 steps of size dt (ForwardStep with tn = t + nSteps*dt). */
 int selfamd_model2d_forward_step(selfamd_model2d *model, int nSteps, double dt);
-/* Blocks until the model's stream has drained. */
+/* Blocks until the model's stream has drained.  An error if a step launch gave up waiting for
+ * another block's traces (seconds on a device that others hold): the state is then not valid
+ * until it is set again. */
 int selfamd_model2d_synchronize(selfamd_model2d *model);
 /* The HIP stream (hipStream_t, as void*) that the model's kernels and graphs run on, so that
  * a caller can order its own work with the model's.  No reference counterpart (the reference
