@@ -410,8 +410,8 @@ int selfamd_mlp_loss_grad(selfamd_mlp *mlp, const float *X_dev, const float *T_d
 int selfamd_mlp_adam_step(selfamd_mlp *mlp, float lr, int step, void *stream);
 /* Backward pass from a given output cotangent dY[batch][nOut] (device): forward of X, then the
  * parameter gradients written to the gradient buffer (accumulate = 0) or added to it
- * (accumulate = 1), and the input cotangent dX[batch][nIn] (device, may be NULL).  For
- * training through a solver (the closure's a-posteriori training).  No reference counterpart. */
+ * (accumulate = 1), and the input cotangent dX[batch][nIn] (device, may be NULL; it may lie
+ * over X or dY, which are then overwritten).  For training through a solver (the closure's a-posteriori training).  No reference counterpart. */
 int selfamd_mlp_backward(selfamd_mlp *mlp, const float *X_dev, const float *dY_dev, int batch, int accumulate,
                          float *dX_dev, void *stream);
 /* Sets the gradient buffer to zero (before accumulating backward passes). */

@@ -717,15 +717,21 @@ hipError_t backward_layers(selfamd_mlp *m, const float *X, float *dY, int B, int
 }
 
 // Forward pass of X and backward pass from the output cotangent dY: parameter gradients written
-// to (or, with accumulate, added to) m->grads, and the input cotangent when dX is given.
+// to (or, with accumulate, added to) m->grads, and the input cotangent when dX is given; dX may lie
+// over X or dY.
 hipError_t backward_impl(selfamd_mlp *m, const float *X, const float *dY, int B, int accumulate, float *dX,
                          hipStream_t st) {
   hipError_t e;
   if (m->rows) {
+    // The weight gradients read X and dY after k_mlp_rows: where dX lies over one of them it is
+    // formed last, as a product of its own.
+    const size_t nX = sizeof(float) * (size_t)B * m->nIn, nY = sizeof(float) * (size_t)B * m->nOut;
+    const bool last = dX && (ranges_overlap(dX, nX, X, nX) || ranges_overlap(dX, nX, dY, nY));
     RowsArgs a = rows_args(m, X, B);
-    a.T = dY; a.dX = dX;
+    a.T = dY; a.dX = last ? nullptr : dX;
     if ((e = launch_rows<kRowsBackward>(a, st))) return e;
-    return weight_grads_rows(m, X, dY, B, accumulate, st);
+    if ((e = weight_grads_rows(m, X, dY, B, accumulate, st)) || !last) return e;
+    return gemm<false, true, 0>(m->D1, m->W1(), dX, nullptr, nullptr, B, m->nIn, m->nH, m->nH, m->nH, 1, st);
   }
   if ((e = forward_impl(m, X, m->Y, B, st))) return e;
   if ((e = hipMemcpyAsync(m->dY, dY, sizeof(float) * (size_t)B * m->nOut, hipMemcpyDeviceToDevice, st))) return e;

@@ -76,6 +76,12 @@ inline __host__ __device__ size_t scb_idx(int i, int v, int s, int e, int P, int
 //   dsdx(4) J(1) dt(1, batched runs) 1/J(1) pad(1) nHat_x(4 sides) nHat_y(4) nScale(4)
 constexpr int kGeomStride = 20;
 
+// Whether the na bytes at a and the nb bytes at b share a byte.
+inline bool ranges_overlap(const void *a, size_t na, const void *b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + nb && y < x + na;
+}
+
 inline unsigned grid1d(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace selfamd
