@@ -401,6 +401,7 @@ int selfamd_mlp_set_params(selfamd_mlp *mlp, const float *params);
 int selfamd_mlp_get_params(selfamd_mlp *mlp, float *params);
 /* Gradients of the last selfamd_mlp_loss_grad call, packed like the parameters (host). */
 int selfamd_mlp_get_grads(selfamd_mlp *mlp, float *grads);
+/* Y[batch][nOut] = net(X[batch][nIn]); Y may lie over X, which is then overwritten. */
 int selfamd_mlp_forward(selfamd_mlp *mlp, const float *X_dev, float *Y_dev, int batch, void *stream);
 /* Forward + backward of L = mean((Y - T)^2) over batch rows; *loss (host, may be null) is the
  * loss of this batch (synchronises the stream when requested). */

@@ -663,12 +663,17 @@ hipError_t weight_grads_rows(selfamd_mlp *m, const float *X, const float *dY, in
   return hipGetLastError();
 }
 
+// Y = net(X); Y may lie over X.
 hipError_t forward_impl(selfamd_mlp *m, const float *X, float *Y, int B, hipStream_t st) {
   hipError_t e;
   if (m->rows) {
+    // a block writes its rows of Y while others still read theirs of X
+    const size_t nY = sizeof(float) * (size_t)B * m->nOut;
+    const bool over = ranges_overlap(Y, nY, X, sizeof(float) * (size_t)B * m->nIn);
     RowsArgs a = rows_args(m, X, B);
-    a.Y = Y;
-    return launch_rows<kRowsForward>(a, st);
+    a.Y = over ? m->Y : Y;
+    if ((e = launch_rows<kRowsForward>(a, st)) || !over) return e;
+    return hipMemcpyAsync(Y, m->Y, nY, hipMemcpyDeviceToDevice, st);
   }
   if ((e = gemm<false, false, 2>(X, m->W1(), m->H1, m->Z1, m->b1(), B, m->nH, m->nIn, m->nIn, m->nH, 1, st))) return e;
   if ((e = gemm<false, false, 2>(m->H1, m->W2(), m->H2, m->Z2, m->b2(), B, m->nH, m->nH, m->nH, m->nH, 1, st))) return e;

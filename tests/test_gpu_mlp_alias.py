@@ -52,3 +52,20 @@ def test_backward_with_the_input_cotangent_over_an_operand(nIn, nH, nOut, rows, 
     # dX is a product of its own there: another order of nH FP32 terms
     dX = mem.to_host()[at:at + X.size].reshape(X.shape)
     assert np.max(np.abs(dX - want_dX)) <= 4 * U * (nH + 16) * np.max(np.abs(want_dX))
+
+
+# outputs narrower, as wide and wider than the inputs: rows of Y over rows of X that other blocks read
+@pytest.mark.parametrize("nIn,nH,nOut,rows", [(51, 128, 48, 4000), (20, 33, 20, 70), (17, 200, 60, 500), (12, 257, 9, 33)])
+@pytest.mark.parametrize("shift", [0, 3])
+def test_forward_over_its_input(nIn, nH, nOut, rows, shift):
+    import self_amd
+    net = _net(nIn, nH, nOut, rows)
+    X = np.random.default_rng(rows).standard_normal((rows, nIn)).astype(np.float32)
+    want = net.forward(X)
+    mem = self_amd.DeviceArray((rows * max(nIn, nOut) + shift,), np.float32, zero=True)
+    host = np.zeros(mem.shape, np.float32)
+    host[:X.size] = X.ravel()
+    mem.copy_from_host(host)
+    self_amd.call("selfamd_mlp_forward", net._h, _at(mem, 0), _at(mem, shift), rows, None)
+    got = mem.to_host()[shift:shift + want.size].reshape(want.shape)
+    assert (got == want).all()
