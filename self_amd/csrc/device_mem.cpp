@@ -6,6 +6,31 @@
 
 using namespace selfamd;
 
+namespace selfamd {
+
+Source source_of(const void *p, size_t bytes, size_t align, int device) {
+  hipPointerAttribute_t at{};
+  auto known = [&](const void *q) {
+    const hipError_t e = hipPointerGetAttributes(&at, q);
+    if (e != hipSuccess) (void)hipGetLastError();  // memory that the runtime does not know
+    return e == hipSuccess && at.type != hipMemoryTypeUnregistered;
+  };
+  if (!known(p) || at.type != hipMemoryTypeDevice) return Source::kCopy;
+  const int owner = at.device;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, const_cast<void *>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return Source::kCopy;
+  }
+  const size_t before = reinterpret_cast<uintptr_t>(p) - reinterpret_cast<uintptr_t>(base);
+  if (before <= size && bytes <= size - before)
+    return owner == device && reinterpret_cast<uintptr_t>(p) % align == 0 ? Source::kKernel : Source::kCopy;
+  return known(static_cast<const char *>(p) + bytes - 1) ? Source::kCopy : Source::kShort;
+}
+
+}  // namespace selfamd
+
 extern "C" {
 
 int selfamd_device_count(int *count) {

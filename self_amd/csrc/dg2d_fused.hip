@@ -2507,18 +2507,6 @@ int selfamd_model2d_set_field(selfamd_model2d *m, int which, const double *field
   return kOk;
 }
 
-// Whether a kernel on the model's device can read doubles at p in place of a copy call, which also
-// takes another device's memory, host memory and any alignment.
-static bool device_doubles(const selfamd_model2d *m, const void *p) {
-  hipPointerAttribute_t at{};
-  if (reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
-  if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-    (void)hipGetLastError();  // memory that the runtime does not know
-    return false;
-  }
-  return at.type == hipMemoryTypeDevice && at.device == m->device;
-}
-
 namespace {
 // after the model's stream has been waited for
 int resident_status(const selfamd_model2d *m) {
@@ -2531,12 +2519,15 @@ int resident_status(const selfamd_model2d *m) {
 int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   SELFAMD_REQUIRE(m && interior, "model2d_set_solution: null argument");
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
+  const Source from = source_of(interior, sizeof(double) * n, sizeof(double), m->device);
+  SELFAMD_REQUIRE(from != Source::kShort, "model2d_set_solution: the array holds less than the state's %zu bytes",
+                  sizeof(double) * n);
   if (m->kind == SELFAMD_MODEL_EULER && !m->presTrace) {
     // prescribed boundary state := traces of this state (SetPrescribedSolutionFromSolution)
     SELFAMD_HIP(hipMalloc(&m->presTrace, sizeof(double) * (size_t)(m->N + 1) * 9 * 4 * m->nEl));
     m->drop_graphs();  // captured without it
   }
-  const bool direct = device_doubles(m, interior);
+  const bool direct = from == Source::kKernel;
   if (!direct) SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(m->launch_state_in(direct ? interior : m->S));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));

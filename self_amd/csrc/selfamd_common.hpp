@@ -82,6 +82,12 @@ inline bool ranges_overlap(const void *a, size_t na, const void *b, size_t nb) {
   return x < y + nb && y < x + na;
 }
 
+// How a kernel on `device` gets at an array that a caller hands over: it can read all `bytes` at p
+// itself; it needs a copy call, which also takes host memory, another device's memory, ranges of
+// several allocations and any alignment; or the device allocation at p ends before the array does.
+enum class Source { kKernel, kCopy, kShort };
+Source source_of(const void *p, size_t bytes, size_t align, int device);
+
 inline unsigned grid1d(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace selfamd
