@@ -867,6 +867,17 @@ int selfamd_mlp_backward(selfamd_mlp *m, const float *X, const float *dY, int B,
   SELFAMD_REQUIRE(m && X && dY && B >= 1 && B <= m->maxB, "mlp_backward: bad arguments (B=%d, max %d)", B,
                   m ? m->maxB : 0);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (m->rows) {  // the kernels read dY where it is; the layers read a copy
+    const size_t bytes = sizeof(float) * (size_t)B * m->nOut;
+    int device = 0;
+    SELFAMD_HIP(hipGetDevice(&device));
+    const Source from = source_of(dY, bytes, sizeof(float), device);
+    SELFAMD_REQUIRE(from != Source::kShort, "mlp_backward: dY holds less than %d rows of %d", B, m->nOut);
+    if (from == Source::kCopy) {
+      SELFAMD_HIP(hipMemcpyAsync(m->dY, dY, bytes, hipMemcpyDeviceToDevice, st));
+      dY = m->dY;
+    }
+  }
   SELFAMD_HIP(backward_impl(m, X, dY, B, accumulate, dX, st));
   return kOk;
 }
