@@ -3091,6 +3091,7 @@ struct selfamd_batch {
   // one persistent launch per stage for all groups (SW, degrees 3, 5, 7)
   int mode = SELFAMD_BATCH_PER_GROUP;
   int persistentBlocks = 0;
+  int device = 0;  // of the stream and the arrays
 
   FusedArgs group_args(const BatchGroup &g, int stage, int tin) const {
     FusedArgs a{};
@@ -3163,6 +3164,8 @@ struct selfamd_batch {
   }
   // Captures `steps` steps starting from trace buffer `start` (each step flips the buffer).
   hipError_t capture_steps(int start, int steps, hipGraphExec_t *out) {
+    const DeviceScope scope(device);  // the branches' streams
+    if (!scope.ok) return hipErrorInvalidDevice;
     const size_t branches = branches_pay(steps) ? groups.size() : 1;
     struct Branches {  // a stream and the event of its end for each branch but the first
       std::vector<hipStream_t> stream;
@@ -3305,6 +3308,7 @@ int selfamd_batch_create(selfamd_batch **out, int nModels, selfamd_model2d *cons
     selfamd_batch_destroy(b);
     return code;
   };
+  if (hipGetDevice(&b->device) != hipSuccess) return fail("no device");
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return fail("stream creation failed");
   for (int N = 1; N <= 7; N++) {
     BatchGroup g;
@@ -3439,6 +3443,8 @@ int selfamd_batch_scatter(selfamd_batch *b) {
   SELFAMD_REQUIRE(b, "batch_scatter: null batch");
   SELFAMD_HIP(hipStreamSynchronize(b->stream));
   // on the default stream, behind any caller's work on a blocking stream of a model
+  const DeviceScope scope(b->device);
+  SELFAMD_REQUIRE(scope.ok, "batch_scatter: the batch's device cannot be made current");
   CopyList list{};
   auto flush = [&]() -> hipError_t {
     if (list.count == 0) return hipSuccess;
@@ -3457,6 +3463,10 @@ int selfamd_batch_scatter(selfamd_batch *b) {
                                        {m->un[0] ? G.un[b->cur] + off * P * 4 : nullptr, m->un[m->cur], ne * P * 4}};
       for (const auto &it : items) {
         if (!it.src) continue;
+        if (m->device != b->device) {  // a kernel may not reach it
+          SELFAMD_HIP(hipMemcpy(it.dst, it.src, 8 * it.n, hipMemcpyDeviceToDevice));
+          continue;
+        }
         if (list.count == kCopyItems) SELFAMD_HIP(flush());
         list.item[list.count++] = it;
       }

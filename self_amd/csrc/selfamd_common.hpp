@@ -88,6 +88,26 @@ inline bool ranges_overlap(const void *a, size_t na, const void *b, size_t nb) {
 enum class Source { kKernel, kCopy, kShort };
 Source source_of(const void *p, size_t bytes, size_t align, int device);
 
+// Makes `device` the current one for a scope: the null stream and new streams belong to the current
+// device, whatever memory the work on them is given.
+class DeviceScope {
+ public:
+  explicit DeviceScope(int device) {
+    ok = hipGetDevice(&previous) == hipSuccess && (previous == device || hipSetDevice(device) == hipSuccess);
+    changed = ok && previous != device;
+  }
+  ~DeviceScope() {
+    if (changed) (void)hipSetDevice(previous);
+  }
+  DeviceScope(const DeviceScope &) = delete;
+  DeviceScope &operator=(const DeviceScope &) = delete;
+  bool ok = false;
+
+ private:
+  int previous = 0;
+  bool changed = false;
+};
+
 inline unsigned grid1d(size_t n, unsigned block) { return (unsigned)((n + block - 1) / block); }
 
 }  // namespace selfamd

@@ -1,0 +1,62 @@
+"""What the library asks of the HIP runtime, seen by a runtime of two devices without a GPU
+(fake_hip.c) that takes the place of libamdhip64 in a child process: the devices that work is
+launched on, the sizes of grids."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)  # found by its soname when the library is loaded
+fake.fake_log.restype = ctypes.c_char_p
+import numpy as np
+import self_amd
+from self_amd import call
+from tests import cases
+
+def log():
+    lines = fake.fake_log().decode().splitlines()
+    fake.fake_log_clear()
+    return lines
+
+def model(kind, N, nx, ny):
+    return cases.Case(kind, N, nx, ny, periodic=True, metrics="affine").gpu_model()[0]
+
+log()
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("hip") / "libamdhip64.so.7")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-Wall", "-Wl,-soname,libamdhip64.so.7", "-o", lib,
+                    os.path.join(HERE, "fake_hip.c")], check=True)
+
+    def child(code):
+        out = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code), lib], cwd=os.path.dirname(HERE),
+                             capture_output=True, text=True, timeout=100)
+        assert out.returncode == 0, out.stdout + out.stderr
+    return child
+
+
+def test_batch_works_on_its_own_device_whatever_the_current_one(run):
+    run("""
+    models = [model("sw", N, 8, 8) for N in (3, 5, 7)]
+    batch = self_amd.Batch(models, [1e-4] * 3)
+    log()
+    fake.hipSetDevice(1)
+    batch.ForwardStep(64)   # groups as branches: streams of their own
+    batch.scatter()
+    lines = log()
+    assert any(l.startswith("stream") for l in lines) and any("k_copy_list" in l for l in lines)
+    elsewhere = [l for l in lines if not l.endswith("device 0")]
+    assert not elsewhere, elsewhere[:3]
+    current = ctypes.c_int()
+    fake.hipGetDevice(ctypes.byref(current))
+    assert current.value == 1
+    """)
