@@ -924,6 +924,7 @@ namespace {
 // r^2 Pf^2 doubles with its neighbours 64 bytes or whole elements away, took 276 us.  LDS rows of Pf
 // doubles are padded by one: four of five rows would share banks at Pf = 8.
 constexpr int kProjectArgs = 448, kProjectLds = 6144, kProjectChunk = 3072;  // doubles
+constexpr size_t kProjectBlocks = size_t(1) << 24;  // of 256: a grid's work-items stay below 2^32
 struct ProjectArgs {
   const double *fine;
   double *coarse;
@@ -1009,7 +1010,7 @@ __global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
 }
 
 // The same, one work-item per coarse value, for coarsening factors and degrees whose factors or
-// runs are too long for the kernel arguments or LDS of k_project.
+// runs are too long for the kernel arguments or LDS of k_project, and for meshes beyond its grid.
 __global__ void k_project_values(const double *__restrict__ Sf, double *__restrict__ Sc, const double *__restrict__ Px,
                                  int Nf, int Nc, int nxc, int nyc, int r, int nVar) {
   const int Pf = Nf + 1, Pc = Nc + 1;
@@ -1308,7 +1309,8 @@ int selfamd_project_l2_structured_2d(const double *fine, double *coarse, int Nf,
     return wf[p] * lagrange_basis(xc, Nc, i, xi) / (r * wc[i]);
   };
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (nPx <= (size_t)kProjectArgs && run <= (size_t)kProjectLds) {
+  const size_t elements = (size_t)nxc * nyc;
+  if (nPx <= (size_t)kProjectArgs && run <= (size_t)kProjectLds && elements < kProjectBlocks) {
     ProjectArgs g;
     g.fine = fine; g.coarse = coarse; g.Pf = Pf; g.Pc = Pc; g.nxc = nxc; g.r = r; g.nVar = nVar;
     g.rowsB = std::max(1, std::min(r, kProjectChunk / (int)run));
@@ -1319,8 +1321,7 @@ int selfamd_project_l2_structured_2d(const double *fine, double *coarse, int Nf,
         for (int p = 0; p < Pf; p++) g.px[(a * Pc + i) * Pf + p] = entry(a, i, p);
     const size_t lds = nPx + (size_t)g.rowsB * r * nVar * Pf * (Pf + 1) + (size_t)g.rowsB * nVar * Pf * Pc + (size_t)nVar * Pc * Pc;
     if (sizeof(double) * lds <= 64 * 1024) {
-      const unsigned blocks = (unsigned)((size_t)nxc * nyc);
-      auto run_as = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, 256, sizeof(double) * lds, st, g); };
+      auto run_as = [&](auto kernel) { hipLaunchKernelGGL(kernel, (unsigned)elements, 256, sizeof(double) * lds, st, g); };
 #define CASE_F(PC, PF) case PF: run_as(k_project<PC, PF>); break;
 #define CASE(PC)                                                                                        \
   case PC:                                                                                              \

@@ -60,3 +60,13 @@ def test_batch_works_on_its_own_device_whatever_the_current_one(run):
     fake.hipGetDevice(ctypes.byref(current))
     assert current.value == 1
     """)
+
+
+def test_projection_grids_stay_within_the_runtime_limit(run):
+    run("""
+    a = self_amd.DeviceArray((8,))
+    for nyc, kernel in ((4095, "k_project"), (4096, "k_project_values"), (4097, "k_project_values")):
+        call("selfamd_project_l2_structured_2d", a.ptr, a.ptr, 1, 1, 4096, nyc, 1, 1, None)
+        lines = log()
+        assert len(lines) == 1 and f"{len(kernel)}{kernel}" in lines[0], lines  # as mangled
+    """)
