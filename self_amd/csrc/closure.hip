@@ -183,6 +183,7 @@ hipError_t gemm(const float *A, const float *B, float *C, float *Z, const float 
 // Row kernels: 16 rows of the batch through the whole network on the FP32 matrix cores
 // ------------------------------------------------------------------------------
 constexpr int kRowMaxHidden = 256, kRowMaxOut = 256, kRowLds = 56 * 1024;  // 64 KiB with the static arrays
+constexpr int kRowMaxRows = kRowTile * ((1 << 23) - 1);                    // blocks of 512, below 2^32 work-items
 
 // kRowsForward: Y = net(X).  kRowsLoss: forward, dY = 2 (Y - T) / count, backward.
 // kRowsBackward: forward, backward from the cotangent T.  kRowsClosure: features of the state,
@@ -213,7 +214,8 @@ struct RowsArgs {
 inline size_t rows_lds(int nIn, int nH, int nO) {
   return sizeof(float) * kRowTile * ((size_t)rows_ld(nIn) + 2 * rows_ld(nH) + rows_ld(nO));
 }
-inline bool rows_fit(int nIn, int nH, int nO) {
+inline bool rows_fit(int nIn, int nH, int nO, int maxB) {
+  if (maxB > kRowMaxRows) return false;
   return nH <= kRowMaxHidden && nO <= kRowMaxOut && rows_lds(nIn, nH, nO) <= kRowLds;
 }
 
@@ -754,7 +756,7 @@ int selfamd_mlp_create(selfamd_mlp **out, int nIn, int nHidden, int nOut, int ma
   m->nIn = nIn; m->nH = nHidden; m->nOut = nOut; m->maxB = maxBatch;
   m->nParams = (size_t)nIn * nHidden + nHidden + (size_t)nHidden * nHidden + nHidden + (size_t)nHidden * nOut + nOut;
   const size_t B = maxBatch, H = nHidden;
-  m->rows = rows_fit(nIn, nHidden, nOut);
+  m->rows = rows_fit(nIn, nHidden, nOut, maxBatch);
   // One allocation for all arrays (a call each takes longer than the kernels of a training step),
   // each 256-byte aligned; the partial gradients are of at most 64 splits of at least 128 rows.
   const size_t lossBlocks = std::max<size_t>(1024, (B + kRowTile - 1) / kRowTile);

@@ -70,3 +70,16 @@ def test_projection_grids_stay_within_the_runtime_limit(run):
         lines = log()
         assert len(lines) == 1 and f"{len(kernel)}{kernel}" in lines[0], lines  # as mangled
     """)
+
+
+def test_networks_of_very_many_rows_have_grids(run):
+    run("""
+    for rows, kernel in ((1 << 26, "k_mlp_rows"), (1 << 27, "k_gemm")):
+        net = self_amd.MLP(1, 1, 1, rows)
+        a = self_amd.DeviceArray((rows, 1), np.float32)
+        b = self_amd.DeviceArray((rows, 1), np.float32)
+        log()
+        call("selfamd_mlp_forward", net._h, a.ptr, b.ptr, rows, None)
+        lines = log()
+        assert lines and all(f"{len(kernel)}{kernel}" in l for l in lines), lines[:3]
+    """)
