@@ -265,6 +265,9 @@ typedef struct selfamd_model2d selfamd_model2d;
                                           affine meshes), which moves the tendency by up to
                                           ~1e-10 relative (7e-11 at 256^2 on the unit square):
                                           set 1 for the reference's arithmetic to 1e-12 */
+#define SELFAMD_PARAM_POLLS 6  /* how often one wait for another block's traces is repeated in a
+                                  launch of several RK stages before it gives up (default
+                                  2^26, about a minute; 0: at once) */
 /* static per-node fields (selfamd_model2d_set_field), interior(0:N,0:N,1,nEl) device arrays */
 #define SELFAMD_FIELD_TOPOGRAPHY 1  /* SW this%H (SetTopography) */
 #define SELFAMD_FIELD_BATHYMETRY 2  /* LSW this%H (SetBathymetry) */
@@ -320,8 +323,9 @@ int selfamd_model2d_integral_noalloc(selfamd_model2d *model, int var, double *va
 /* nSteps full low-storage RK3 steps of size dt (ForwardStep with tn = t + nSteps*dt). */
 int selfamd_model2d_forward_step(selfamd_model2d *model, int nSteps, double dt);
 /* Blocks until the model's stream has drained.  An error if a step launch gave up waiting for
- * another block's traces (seconds on a device that others hold): the state is then not valid
- * until it is set again. */
+ * another block's traces (about a minute on a device that others hold, SELFAMD_PARAM_POLLS): the
+ * state is then not valid, and every call that waits for it reports it, until it is set again
+ * (selfamd_model2d_set_solution). */
 int selfamd_model2d_synchronize(selfamd_model2d *model);
 /* The HIP stream (hipStream_t, as void*) that the model's kernels and graphs run on, so that
  * a caller can order its own work with the model's.  No reference counterpart (the reference

@@ -1058,15 +1058,18 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // 3.3 us (9.5 us per stage).  A call of one step takes 78 us with set and get, 110 in launches.
 //
 // All blocks must be resident: the launch is cooperative, which the runtime refuses if they
-// cannot be.  Every wait is bounded as well: a lane that has polled kPollBudget times in one wait
-// (seconds) waits no more and raises `timedOut`, which the next synchronising call reports.
+// cannot be.  Every wait is bounded as well: a lane that has polled `polls` times in one wait waits
+// no more and raises `timedOut`, which the next synchronising call reports.  What a wait may last
+// is what others may hold the device for while some blocks are in and some are not: kPolls is about
+// a minute.
 constexpr unsigned long long kEmpty = 0x7FF0DEAD7FF0DEADull;
-constexpr int kPollBudget = 1 << 22;
+constexpr int kPolls = 1 << 26;
 
 struct ResidentArgs {
   unsigned long long *ring;  // 3 buffers (0:N, NX, 4, nEl)
   int stages;                // 3 per step
   double rkA[3], rkGdt[3];   // a_m, g_m dt
+  int polls;                 // per wait; 0: no wait at all
   int *timedOut;             // host memory
 };
 // With a closure attached (NET): the network and where the blocks exchange their mass integrals
@@ -1387,12 +1390,12 @@ k_resident(const FusedArgs a, const ResidentArgs ra, const ResidentNetArgs na) {
   // ---- stages ----
   const unsigned tileAt = blockIdx.x * (unsigned)(EPB * NF * NX);
   const int tileSlots = min(EPB, a.nEl - (int)blockIdx.x * EPB) * NF * NX;
-  int budget = kPollBudget, fill = 0;  // fill: m mod 3
+  int budget = ra.polls - 1, fill = 0;  // fill: m mod 3
 #pragma unroll 1
   for (int m = 0; m < ra.stages; m++) {
     const bool last = m == ra.stages - 1;
     const int before = fill == 0 ? 2 : fill - 1, empty = fill == 2 ? 0 : fill + 1;  // (m - 1), (m - 2) mod 3
-    if (budget >= 0) budget = kPollBudget;
+    if (budget >= 0) budget = ra.polls - 1;
     if (nodeActive) {
       double fx[NV], fy[NV], q[NT];
       Phys::volume(s, auxVal, a.p, fx, fy, q);
@@ -2043,6 +2046,7 @@ struct selfamd_model2d {
   int residentNetBlocks = -1;                   // with a closure
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
   int *timedOut = nullptr;
+  int polls = kPolls;
 
   FusedArgs stage_args(int traceIn) const {
     FusedArgs a{};
@@ -2257,6 +2261,7 @@ hipError_t selfamd_model2d::launch_resident(const ResidentKernel &k, int nSteps,
     ra.rkA[q] = kRk3A[q];
     ra.rkGdt[q] = kRk3G[q] * dt;
   }
+  ra.polls = polls;
   ra.timedOut = timedOut;
   ResidentNetArgs na{};
   if (closure) {
@@ -2482,6 +2487,10 @@ int selfamd_model2d_set_param(selfamd_model2d *m, int which, double value) {
       }
       m->nodal = value != 0.0;
       break;
+    case SELFAMD_PARAM_POLLS:
+      SELFAMD_REQUIRE(value >= 0.0 && value <= 2147483647.0, "model2d_set_param: %g polls", value);
+      m->polls = (int)value;
+      return kOk;
     default: SELFAMD_REQUIRE(false, "model2d_set_param: unknown parameter %d", which);
   }
   m->drop_graphs();
@@ -2514,6 +2523,12 @@ int resident_status(const selfamd_model2d *m) {
                   "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
   return kOk;
 }
+// a valid state has been stored, and the stream waited for
+void state_replaced(selfamd_model2d *m) {
+  if (!m->timedOut || !*m->timedOut) return;
+  *m->timedOut = 0;
+  m->ringValues = 0;  // the exchange ring is emptied before its next use
+}
 }  // namespace
 
 int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
@@ -2531,10 +2546,7 @@ int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   if (!direct) SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(m->launch_state_in(direct ? interior : m->S));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  if (m->timedOut && *m->timedOut) {  // a valid state again; the exchange ring is emptied before its next use
-    *m->timedOut = 0;
-    m->ringValues = 0;
-  }
+  state_replaced(m);
   return kOk;
 }
 
