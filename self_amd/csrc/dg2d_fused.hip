@@ -2860,7 +2860,7 @@ int selfamd_model2d_stage(selfamd_model2d *m, int stage, double dt, double *Ssav
   m->cur ^= 1;
   if (stage == 2) m->t += dt;
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 int selfamd_model2d_tendency_vjp(selfamd_model2d *m, const double *S, const double *un, const double *lambda,
@@ -2980,7 +2980,7 @@ int selfamd_model2d_closure_features(selfamd_model2d *m, float *X) {
   SELFAMD_HIP(closure_features(m->S, m->geom, m->closure->inMean, m->closure->inScale, X, m->N, m->nVar, m->nEl,
                                m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return kOk;
+  return resident_status(m);
 }
 
 int selfamd_tile_count(int kind, int N, int *count) {
@@ -3308,6 +3308,8 @@ int selfamd_batch_create(selfamd_batch **out, int nModels, selfamd_model2d *cons
     SELFAMD_REQUIRE((m->aux != nullptr) == (m0->aux != nullptr) && (m->stat2 != nullptr) == (m0->stat2 != nullptr) &&
                         (m->presTrace != nullptr) == (m0->presTrace != nullptr),
                     "batch_create: run %d: static fields must be set on all runs or on none", r);
+    SELFAMD_HIP(hipStreamSynchronize(m->stream));
+    if (const int status = resident_status(m)) return status;
   }
   selfamd_batch *b = new selfamd_batch();
   b->kind = m0->kind;

@@ -81,8 +81,12 @@ def test_every_reader_reports_it_and_a_new_state_ends_it(kind, N, nx, ny, metric
     want = m.solution
     m.SetSolution(c.sol)
     assert gives_up(m, 4, dt)
-    readers = [lambda: m.solution, m.CalculateTendency, m.flux_registers,
+    readers = [lambda: m.solution, m.CalculateTendency, m.flux_registers, lambda: m.Stage(0, dt),
                lambda: call("selfamd_model2d_synchronize", m._h), lambda: m.time_steps(3, dt)]
+    if hidden:
+        readers.append(m.closure_features)
+    elif metrics == "affine":
+        readers.append(lambda: self_amd.Batch([m], [dt]))
     for read in readers:
         with pytest.raises(SelfAmdError, match="gave up"):
             read()
