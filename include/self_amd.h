@@ -325,7 +325,7 @@ int selfamd_model2d_forward_step(selfamd_model2d *model, int nSteps, double dt);
 /* Blocks until the model's stream has drained.  An error if a step launch gave up waiting for
  * another block's traces (about a minute on a device that others hold, SELFAMD_PARAM_POLLS): the
  * state is then not valid, and every call that waits for it reports it, until it is set again
- * (selfamd_model2d_set_solution). */
+ * (selfamd_model2d_set_solution, selfamd_batch_scatter). */
 int selfamd_model2d_synchronize(selfamd_model2d *model);
 /* The HIP stream (hipStream_t, as void*) that the model's kernels and graphs run on, so that
  * a caller can order its own work with the model's.  No reference counterpart (the reference

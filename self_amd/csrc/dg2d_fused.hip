@@ -3488,6 +3488,10 @@ int selfamd_batch_scatter(selfamd_batch *b) {
   }
   SELFAMD_HIP(flush());
   SELFAMD_HIP(hipStreamSynchronize(nullptr));
+  for (Model *m : b->models) {
+    SELFAMD_HIP(hipStreamSynchronize(m->stream));
+    state_replaced(m);
+  }
   return kOk;
 }
 

@@ -94,3 +94,20 @@ def test_every_reader_reports_it_and_a_new_state_ends_it(kind, N, nx, ny, metric
     m.SetSolution(c.sol)
     m.ForwardStep(4, dt)
     np.testing.assert_array_equal(m.solution, want)
+
+
+def test_scatter_into_a_model_ends_it():
+    c, m = model("sw", 5, 9, 9, "affine")
+    dt = c.dt(0.05)
+    batch = self_amd.Batch([m], [dt])
+    batch.ForwardStep(3)
+    batch.scatter()
+    want = m.solution
+    m.ForwardStep(4, dt)
+    later = m.solution
+    assert gives_up(m, 4, dt)
+    m._param(POLLS, 1 << 26)
+    batch.scatter()
+    np.testing.assert_array_equal(m.solution, want)
+    m.ForwardStep(4, dt)
+    np.testing.assert_array_equal(m.solution, later)
