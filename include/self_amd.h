@@ -265,9 +265,13 @@ typedef struct selfamd_model2d selfamd_model2d;
                                           affine meshes), which moves the tendency by up to
                                           ~1e-10 relative (7e-11 at 256^2 on the unit square):
                                           set 1 for the reference's arithmetic to 1e-12 */
-#define SELFAMD_PARAM_POLLS 6  /* how often one wait for another block's traces is repeated in a
-                                  launch of several RK stages before it gives up (default
-                                  2^26, about a minute; 0: at once) */
+#define SELFAMD_PARAM_POLLS 6  /* how often a launch of several RK stages looks in vain for another
+                                  block's traces before it gives up (default 2^26, about a
+                                  minute; 0: at once) */
+#define SELFAMD_PARAM_GATE_POLLS 7  /* how often a block of such a launch looks whether all
+                                  blocks have found a place on the device before the launch is
+                                  given up and its steps are taken one stage per launch (default
+                                  4096, some milliseconds; 0: always given up) */
 /* static per-node fields (selfamd_model2d_set_field), interior(0:N,0:N,1,nEl) device arrays */
 #define SELFAMD_FIELD_TOPOGRAPHY 1  /* SW this%H (SetTopography) */
 #define SELFAMD_FIELD_BATHYMETRY 2  /* LSW this%H (SetBathymetry) */
@@ -320,12 +324,17 @@ int selfamd_model2d_integral(selfamd_model2d *model, int var, double *value);
  * GPU (other streams, other host threads) race on it.  The current device must be the
  * model's. */
 int selfamd_model2d_integral_noalloc(selfamd_model2d *model, int var, double *value_dev);
-/* nSteps full low-storage RK3 steps of size dt (ForwardStep with tn = t + nSteps*dt). */
+/* nSteps full low-storage RK3 steps of size dt (ForwardStep with tn = t + nSteps*dt), in stream
+ * order and without waiting for them.  On meshes that fit the device all stages are one launch,
+ * whose blocks have to be on the device together; where other work keeps some of them out, the
+ * next call that waits for the model, reads its state or changes what it depends on takes the
+ * steps one stage per launch.  Such a call first waits until pending launches are under way; with
+ * a closure attached forward_step does so itself. */
 int selfamd_model2d_forward_step(selfamd_model2d *model, int nSteps, double dt);
 /* Blocks until the model's stream has drained.  An error if a step launch gave up waiting for
- * another block's traces (about a minute on a device that others hold, SELFAMD_PARAM_POLLS): the
- * state is then not valid, and every call that waits for it reports it, until it is set again
- * (selfamd_model2d_set_solution, selfamd_batch_scatter). */
+ * another block's traces (SELFAMD_PARAM_POLLS): the state is then not valid, and every call that
+ * waits for it reports it, until it is set again (selfamd_model2d_set_solution,
+ * selfamd_batch_scatter). */
 int selfamd_model2d_synchronize(selfamd_model2d *model);
 /* The HIP stream (hipStream_t, as void*) that the model's kernels and graphs run on, so that
  * a caller can order its own work with the model's.  No reference counterpart (the reference

@@ -22,7 +22,7 @@ from ._lib import SelfAmdError, call, load
 GAUSS, GAUSS_LOBATTO, UNIFORM = 1, 2, 5
 BC_PRESCRIBED, BC_RADIATION, BC_NONORMALFLOW = 100, 101, 102
 MODEL_LSW, MODEL_SW, MODEL_EULER = 1, 2, 3
-PARAM_G, PARAM_FCORI, PARAM_GAMMA, PARAM_RGAS, PARAM_NODAL_METRICS, PARAM_POLLS = 1, 2, 3, 4, 5, 6
+PARAM_G, PARAM_FCORI, PARAM_GAMMA, PARAM_RGAS, PARAM_NODAL_METRICS, PARAM_POLLS, PARAM_GATE_POLLS = 1, 2, 3, 4, 5, 6, 7
 FIELD_TOPOGRAPHY, FIELD_BATHYMETRY, FIELD_CORIOLIS, FIELD_POTENTIAL, FIELD_DRAG = 1, 2, 3, 4, 5
 
 __all__ = ["DeviceArray", "device_count", "device_name", "synchronize", "Lagrange", "Mesh2D", "SEMQuad",

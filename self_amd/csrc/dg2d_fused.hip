@@ -22,6 +22,7 @@
 // Geometry: the fast path takes affine elements (metric terms constant per element, true
 // for the structured and block meshes); each element carries one 20-double record.
 #include <algorithm>
+#include <chrono>
 #include <mutex>
 #include <cmath>
 #include <cstdlib>
@@ -49,6 +50,8 @@ constexpr int kResidentSteps = 2, kResidentElements = 1024;
 // Instances whose registers spill pay for it once per call: from this many steps on (SW N = 3,
 // 18,400 elements: 60 against 49 us for one step, 10.2 against 11.3 us per stage).
 constexpr int kResidentSpillSteps = 5;
+// After a launch that found no place for all its blocks, this many calls take step graphs.
+constexpr int kHeldOffCalls = 64;
 // Longer calls are several resident launches (27 ms each at 10^2 elements of degree 7, against some
 // 10 us for a launch), so that other streams get the device in between.
 constexpr int kResidentLaunchSteps = 4096;
@@ -1057,20 +1060,46 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // integrals in one copy that all blocks poll, sent after the face phase, the wait for them alone was
 // 3.3 us (9.5 us per stage).  A call of one step takes 78 us with set and get, 110 in launches.
 //
-// All blocks must be resident: the launch is cooperative, which the runtime refuses if they
-// cannot be.  Every wait is bounded as well: a lane that has polled `polls` times in one wait waits
-// no more and raises `timedOut`, which the next synchronising call reports.  What a wait may last
-// is what others may hold the device for while some blocks are in and some are not: kPolls is about
-// a minute.
+// All blocks must be on the device at once.  The launch is cooperative, which the runtime refuses if
+// they cannot be, but the runtime counts on an empty device: blocks of other streams that are there
+// when the first blocks arrive leave gaps between theirs, and where the launch needs every register
+// (SW N = 7, 4,096 blocks: four wavefronts of 128 of a SIMD's 512 registers) the last ones then never
+// fit, however long the others wait.  So the blocks first meet at a gate, before anything is stored:
+// each counts itself in, the last one opens the gate, and a block that has looked gatePolls times
+// (some ms) closes it for good.  Whichever comes first holds for all blocks: of a launch whose gate
+// is closed every block ends at once, as do those of the launches after it, and the host takes their
+// steps by step graphs.  Past the gate every wait is for a block that is running; they are bounded
+// all the same: a lane that has found slots empty `polls` times in a launch waits no more and raises
+// `timedOut`, which the next synchronising call reports.
 constexpr unsigned long long kEmpty = 0x7FF0DEAD7FF0DEADull;
-constexpr int kPolls = 1 << 26;
+constexpr int kPolls = 1 << 26, kGatePolls = 1 << 12;
 
+// What a model's resident launches tell the host, in host memory.
+struct ResidentReport {
+  int timedOut;      // a wait past the gate gave up
+  unsigned started;  // the last launch whose gate has opened
+  unsigned refused;  // the launch whose gate was closed, or 0
+};
+
+// The gate, in device memory.  Launch L finds the verdict at 2 (L - 1), and it ends at 2 L (open) or
+// odd (closed, for this launch and all that follow).  A launch's blocks count themselves in by groups.
+// What a launch needs only before and after its stages is here too and not in the kernel arguments,
+// where it would be held in registers throughout.
+constexpr int kGateGroups = 64;
+struct ResidentGate {
+  struct alignas(128) Word {
+    unsigned long long value;
+  };
+  Word verdict, groupsIn, in[kGateGroups];
+  ResidentReport *report;
+  int polls;      // per launch and lane
+  int gatePolls;  // 0: the gate never opens
+};
 struct ResidentArgs {
   unsigned long long *ring;  // 3 buffers (0:N, NX, 4, nEl)
   int stages;                // 3 per step
   double rkA[3], rkGdt[3];   // a_m, g_m dt
-  int polls;                 // per wait; 0: no wait at all
-  int *timedOut;             // host memory
+  ResidentGate *gate;
 };
 // With a closure attached (NET): the network and where the blocks exchange their mass integrals
 struct ResidentNetArgs {
@@ -1119,6 +1148,42 @@ __device__ inline unsigned long long ring_load(const unsigned long long *p) {
 }
 __device__ inline void ring_store(unsigned long long *p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ inline unsigned long long gate_count(ResidentGate::Word &word) {
+  return __hip_atomic_fetch_add(&word.value, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Settles the verdict, which this launch found at `found`, unless it is settled.
+__device__ inline void gate_decide(ResidentGate *gate, unsigned long long found, bool open) {
+  if (found & 1) return;
+  const unsigned launch = (unsigned)(found >> 1) + 1;
+  unsigned long long expected = found;
+  if (__hip_atomic_compare_exchange_strong(&gate->verdict.value, &expected, open ? found + 2 : found + 1, __ATOMIC_RELAXED,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+    __hip_atomic_store(open ? &gate->report->started : &gate->report->refused, launch, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);  // the host may be looking
+  }
+}
+// One work-item of every block: counts the block in and waits for the verdict.  The block has not
+// been counted when it reads the verdict first, so that is the one before this launch's, or closed.
+__device__ inline bool gate_opens(ResidentGate *gate) {
+  const unsigned groups = min((unsigned)kGateGroups, gridDim.x), group = blockIdx.x % groups;
+  const unsigned members = gridDim.x / groups + (group < gridDim.x % groups ? 1 : 0);
+  const int polls = gate->gatePolls;
+  const unsigned long long found = ring_load(&gate->verdict.value);
+  if (found & 1) return false;
+  if (gate_count(gate->in[group]) == members - 1) {
+    ring_store(&gate->in[group].value, 0);  // for the next launch
+    if (gate_count(gate->groupsIn) == groups - 1) {
+      ring_store(&gate->groupsIn.value, 0);
+      gate_decide(gate, found, polls > 0);
+    }
+  }
+  for (int k = polls;; k--) {
+    const unsigned long long seen = ring_load(&gate->verdict.value);
+    if (seen != found) return !(seen & 1);
+    if (k <= 0) gate_decide(gate, found, false);
+  }
 }
 
 // The closure's network in a resident block: wavefront w holds the weights of columns 16 w .. 16 w +
@@ -1180,6 +1245,16 @@ struct ResidentNet {
 __global__ void k_ring_fill(unsigned long long *ring, size_t n) {
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
     ring[t] = kEmpty;
+}
+// The gate before launch number launches + 1.
+__global__ void k_gate_reset(ResidentGate *gate, unsigned launches, ResidentReport *report, int polls, int gatePolls) {
+  gate->in[threadIdx.x].value = 0;
+  if (threadIdx.x) return;
+  gate->groupsIn.value = 0;
+  gate->verdict.value = 2ull * launches;
+  gate->report = report;
+  gate->polls = polls;
+  gate->gatePolls = gatePolls;
 }
 
 template <class Phys, int N, bool NODAL, int WPE, bool NET = false>
@@ -1387,15 +1462,28 @@ k_resident(const FusedArgs a, const ResidentArgs ra, const ResidentNetArgs na) {
     }
   }
 
+  // ---- the gate, behind the prologue's loads: uniform ones are scalar loads only before a kernel's
+  // first store (with the gate at the start SW N = 7 takes 132 registers against 126) ----
+  bool open = false;
+  if (tid == 0) open = gate_opens(ra.gate);
+  if constexpr (WAVE) {
+    open = __builtin_amdgcn_readfirstlane((int)open) != 0;
+  } else {
+    __shared__ int sOpen;
+    if (tid == 0) sOpen = open;
+    __syncthreads();
+    open = sOpen != 0;
+  }
+  if (!open) return;
+
   // ---- stages ----
   const unsigned tileAt = blockIdx.x * (unsigned)(EPB * NF * NX);
   const int tileSlots = min(EPB, a.nEl - (int)blockIdx.x * EPB) * NF * NX;
-  int budget = ra.polls - 1, fill = 0;  // fill: m mod 3
+  int budget = ra.gate->polls - 1, fill = 0;  // fill: m mod 3
 #pragma unroll 1
   for (int m = 0; m < ra.stages; m++) {
     const bool last = m == ra.stages - 1;
     const int before = fill == 0 ? 2 : fill - 1, empty = fill == 2 ? 0 : fill + 1;  // (m - 1), (m - 2) mod 3
-    if (budget >= 0) budget = ra.polls - 1;
     if (nodeActive) {
       double fx[NV], fy[NV], q[NT];
       Phys::volume(s, auxVal, a.p, fx, fy, q);
@@ -1623,7 +1711,7 @@ k_resident(const FusedArgs a, const ResidentArgs ra, const ResidentNetArgs na) {
 #pragma unroll
     for (int v = 0; v < NV; v++) a.S[sBase + (size_t)v * NN + node] = s[v];
   }
-  if (budget < 0) *ra.timedOut = 1;
+  if (budget < 0) ra.gate->report->timedOut = 1;
 }
 
 // ------------------------------------------------------------------------------
@@ -2036,8 +2124,7 @@ struct selfamd_model2d {
   std::vector<int32_t> hnbr;      // host copy of the neighbour codes
 
   // resident stepping: the exchange ring (allocated on first use), the blocks that can be
-  // resident at once (-1: not asked yet; 0: not available), the
-  // host flag that a launch raises when a wait ran out
+  // resident at once (-1: not asked yet; 0: not available), the gate and what the launches report
   unsigned long long *ring = nullptr;
   size_t ringLen = 0;
   int ringValues = 0;  // values per face node of the slot layout the ring was emptied for
@@ -2045,8 +2132,23 @@ struct selfamd_model2d {
   bool residentSpills[2][kResidentDense] = {};  // whether those instances' registers spill
   int residentNetBlocks = -1;                   // with a closure
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
-  int *timedOut = nullptr;
-  int polls = kPolls;
+  ResidentGate *gate = nullptr;
+  ResidentReport *report = nullptr;
+  int polls = kPolls, gatePolls = kGatePolls;
+  bool gateReset = false;  // the gate is to be set up before the next launch
+  unsigned launches = 0;  // resident launches so far: the last one's number
+  int heldOff = 0;        // calls still to take step graphs after a refused launch
+  // Launches that may yet be refused: `count` alike from launch `first` on, which starts from trace
+  // buffer `cur`.
+  struct Pending {
+    unsigned first, count;
+    int nSteps, cur;
+    double dt;
+  };
+  std::vector<Pending> pending;
+  unsigned started() const { return __atomic_load_n(&report->started, __ATOMIC_RELAXED); }
+  bool refused() const { return report && __atomic_load_n(&report->refused, __ATOMIC_RELAXED) != 0; }
+  bool timed_out() const { return report && __atomic_load_n(&report->timedOut, __ATOMIC_RELAXED) != 0; }
 
   FusedArgs stage_args(int traceIn) const {
     FusedArgs a{};
@@ -2180,7 +2282,11 @@ struct selfamd_model2d {
 using Model = selfamd_model2d;
 
 bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
-  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || (timedOut && *timedOut)) return false;
+  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || timed_out()) return false;
+  if (heldOff > 0) {
+    heldOff--;
+    return false;
+  }
   int current = -1;  // the ring is allocated on the current device
   if (hipGetDevice(&current) != hipSuccess || current != device) return false;
   // the 64-wide tile of nonlinear SW at N = 5 splits the face sums; the resident kernel does not
@@ -2232,12 +2338,27 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
     if (ring) (void)hipFree(ring);
     ring = nullptr;
     ringLen = 0;
-    if ((!timedOut && hipHostMalloc(&timedOut, sizeof(int), hipHostMallocDefault) != hipSuccess) ||
-        hipMalloc(&ring, sizeof(unsigned long long) * len) != hipSuccess) {
+    if (!report) {
+      if (hipHostMalloc(&report, sizeof(ResidentReport), hipHostMallocDefault) != hipSuccess) {
+        report = nullptr;
+        (void)hipGetLastError();
+        return false;
+      }
+      *report = {0, launches, 0};
+    }
+    if (!gate) {
+      if (hipMalloc(&gate, sizeof(ResidentGate)) != hipSuccess) {
+        gate = nullptr;
+        (void)hipGetLastError();
+        return false;
+      }
+      gateReset = true;
+    }
+    if (hipMalloc(&ring, sizeof(unsigned long long) * len) != hipSuccess) {
+      ring = nullptr;
       (void)hipGetLastError();
       return false;
     }
-    *timedOut = 0;
     ringLen = len;
     ringValues = 0;
   }
@@ -2245,6 +2366,11 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
     hipLaunchKernelGGL(k_ring_fill, (unsigned)std::min<size_t>((ringLen + 255) / 256, 4096), 256, 0, stream, ring, ringLen);
     if (hipGetLastError() != hipSuccess) return false;
     ringValues = k.values;
+  }
+  if (gateReset) {
+    hipLaunchKernelGGL(k_gate_reset, 1, kGateGroups, 0, stream, gate, launches, report, polls, gatePolls);
+    if (hipGetLastError() != hipSuccess) return false;
+    gateReset = false;
   }
   return true;
 }
@@ -2261,8 +2387,7 @@ hipError_t selfamd_model2d::launch_resident(const ResidentKernel &k, int nSteps,
     ra.rkA[q] = kRk3A[q];
     ra.rkGdt[q] = kRk3G[q] * dt;
   }
-  ra.polls = polls;
-  ra.timedOut = timedOut;
+  ra.gate = gate;
   ResidentNetArgs na{};
   if (closure) {
     na.w = mlp_weights(closure->mlp);
@@ -2275,6 +2400,13 @@ hipError_t selfamd_model2d::launch_resident(const ResidentKernel &k, int nSteps,
   void *args[] = {&a, &ra, &na};
   const hipError_t e = hipLaunchCooperativeKernel(k.fn, dim3((nEl + k.elements - 1) / k.elements), dim3(k.threads), args, 0, stream);
   if (e != hipSuccess) return e;
+  launches++;
+  const unsigned in = started();
+  pending.erase(pending.begin(), std::find_if(pending.begin(), pending.end(), [in](const Pending &p) {
+    return (int)(in - (p.first + p.count - 1)) < 0;
+  }));
+  if (!pending.empty() && pending.back().nSteps == nSteps && pending.back().dt == dt) pending.back().count++;
+  else pending.push_back({launches, 1, nSteps, cur, dt});
   cur = end;
   for (int q = 0; q < nSteps; q++) t += dt;
   return hipSuccess;
@@ -2456,7 +2588,8 @@ int selfamd_model2d_destroy(selfamd_model2d *m) {
                     m->aux,  m->stat2, m->presTrace, m->ndsdx, m->nJ,    m->nnHat, m->nnScale};
   if (m->bandElems) (void)hipFree(m->bandElems);
   if (m->ring) (void)hipFree(m->ring);
-  if (m->timedOut) (void)hipHostFree(m->timedOut);
+  if (m->gate) (void)hipFree(m->gate);
+  if (m->report) (void)hipHostFree(m->report);
   if (m->intScratch) (void)hipFree(m->intScratch);
   if (m->adjTrace) (void)hipFree(m->adjTrace);
   if (m->adjChi) (void)hipFree(m->adjChi);
@@ -2468,8 +2601,91 @@ int selfamd_model2d_destroy(selfamd_model2d *m) {
   return kOk;
 }
 
+namespace {
+int step_graphs(selfamd_model2d *m, int nSteps, double dt);
+
+// after the model's stream has been waited for
+int resident_status(const selfamd_model2d *m) {
+  SELFAMD_REQUIRE(!m->timed_out(),
+                  "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
+  return kOk;
+}
+
+// With the model's stream waited for: the steps of a refused launch and of those after it, by step
+// graphs.  Nothing of the model has changed since it was refused.
+int take_refused_steps(selfamd_model2d *m) {
+  std::vector<selfamd_model2d::Pending> todo;
+  todo.swap(m->pending);
+  if (!m->refused()) return kOk;
+  const unsigned first = m->report->refused;
+  m->report->refused = 0;
+  m->gateReset = true;
+  m->heldOff = kHeldOffCalls;
+  const double t = m->t;  // has counted these steps
+  bool taken = false;
+  for (const auto &p : todo) {
+    for (unsigned k = 0; k < p.count; k++) {
+      if ((int)(p.first + k - first) < 0) continue;
+      if (!taken) m->cur = p.cur ^ (p.nSteps & (int)k & 1);
+      taken = true;
+      if (const int status = step_graphs(m, p.nSteps, p.dt)) return status;
+    }
+  }
+  m->t = t;
+  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  return kOk;
+}
+
+// Waits for the model's stream; the steps that were asked for have been taken when it returns.
+int wait_for(selfamd_model2d *m) {
+  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  if (!m->pending.empty())
+    if (const int status = take_refused_steps(m)) return status;
+  return resident_status(m);
+}
+
+// Before other work on the state, and before anything that the steps depend on changes: every
+// resident launch has been let in (which a launch on an idle device is some us after the call), or the
+// steps have been taken.
+int settle(selfamd_model2d *m) {
+  if (m->pending.empty()) return kOk;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  SELFAMD_HIP(hipStreamIsCapturing(m->stream, &capturing));
+  const bool captured = capturing != hipStreamCaptureStatusNone;  // since the launch: not to be waited for
+  const auto until = std::chrono::steady_clock::now() +
+                     (captured ? std::chrono::microseconds(60'000'000) : std::chrono::microseconds(200));
+  while (m->started() != m->launches && !m->refused() && std::chrono::steady_clock::now() < until) {}
+  if (m->started() == m->launches) {
+    m->pending.clear();
+    return kOk;
+  }
+  SELFAMD_REQUIRE(!captured, "model2d: steps before the capture have not been taken; wait for the model before its "
+                             "stream is captured");
+  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  return take_refused_steps(m);
+}
+#define SELFAMD_SETTLE(m)                              \
+  do {                                                 \
+    if (const int status_ = settle(m)) return status_; \
+  } while (0)
+
+// A valid state has been stored, after all pending steps, and the stream waited for.
+void state_replaced(selfamd_model2d *m) {
+  m->pending.clear();
+  if (m->refused()) {
+    m->report->refused = 0;
+    m->gateReset = true;
+  }
+  if (m->timed_out()) {
+    m->report->timedOut = 0;
+    m->ringValues = 0;  // the exchange ring is emptied before its next use
+  }
+}
+}  // namespace
+
 int selfamd_model2d_set_param(selfamd_model2d *m, int which, double value) {
   SELFAMD_REQUIRE(m, "model2d_set_param: null model");
+  SELFAMD_SETTLE(m);
   switch (which) {
     case SELFAMD_PARAM_G: m->p.g = value; break;
     case SELFAMD_PARAM_FCORI: m->p.fCori = value; break;
@@ -2488,8 +2704,10 @@ int selfamd_model2d_set_param(selfamd_model2d *m, int which, double value) {
       m->nodal = value != 0.0;
       break;
     case SELFAMD_PARAM_POLLS:
+    case SELFAMD_PARAM_GATE_POLLS:
       SELFAMD_REQUIRE(value >= 0.0 && value <= 2147483647.0, "model2d_set_param: %g polls", value);
-      m->polls = (int)value;
+      (which == SELFAMD_PARAM_POLLS ? m->polls : m->gatePolls) = (int)value;
+      m->gateReset = m->gate != nullptr;
       return kOk;
     default: SELFAMD_REQUIRE(false, "model2d_set_param: unknown parameter %d", which);
   }
@@ -2509,27 +2727,13 @@ int selfamd_model2d_set_field(selfamd_model2d *m, int which, const double *field
            (which == SELFAMD_FIELD_DRAG && m->kind == SELFAMD_MODEL_EULER))
     slot = &m->stat2;
   SELFAMD_REQUIRE(slot, "model2d_set_field: field %d does not apply to model kind %d", which, m->kind);
+  SELFAMD_SETTLE(m);
   if (!*slot) SELFAMD_HIP(hipMalloc(slot, sizeof(double) * n));
   SELFAMD_HIP(hipMemcpyAsync(*slot, field, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
   m->drop_graphs();
   return kOk;
 }
-
-namespace {
-// after the model's stream has been waited for
-int resident_status(const selfamd_model2d *m) {
-  SELFAMD_REQUIRE(!m->timedOut || !*m->timedOut,
-                  "model2d: a resident launch gave up waiting for a neighbour's traces; the state is not valid");
-  return kOk;
-}
-// a valid state has been stored, and the stream waited for
-void state_replaced(selfamd_model2d *m) {
-  if (!m->timedOut || !*m->timedOut) return;
-  *m->timedOut = 0;
-  m->ringValues = 0;  // the exchange ring is emptied before its next use
-}
-}  // namespace
 
 int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   SELFAMD_REQUIRE(m && interior, "model2d_set_solution: null argument");
@@ -2552,6 +2756,7 @@ int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
 
 int selfamd_model2d_get_solution(selfamd_model2d *m, double *interior) {
   SELFAMD_REQUIRE(m && interior, "model2d_get_solution: null argument");
+  SELFAMD_SETTLE(m);
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
   SELFAMD_HIP(hipMemcpyAsync(interior, m->S, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
@@ -2561,6 +2766,7 @@ int selfamd_model2d_get_solution(selfamd_model2d *m, double *interior) {
 // integral of the current state over the mesh (the integrand kind, and the variable for
 // kIntVariable); synchronises the model's stream
 static int model_integral(selfamd_model2d *m, int what, int var, double *value, const char *who) {
+  SELFAMD_SETTLE(m);
   const size_t PP = (size_t)(m->N + 1) * (m->N + 1), nNodes = PP * m->nEl;
   const int nBlocks = (int)((nNodes + kIntBlock - 1) / kIntBlock);
   if (m->intScratchLen < (size_t)nBlocks + 1) {
@@ -2633,6 +2839,7 @@ int selfamd_model2d_integral_noalloc(selfamd_model2d *m, int var, double *value)
   SELFAMD_REQUIRE(dev == m->device, "model2d_integral_noalloc: the model lives on device %d, the current device is %d",
                   m->device, dev);
   SELFAMD_REQUIRE(dev >= 0 && dev < kMaxDevices, "model2d_integral_noalloc: device %d out of range", dev);
+  SELFAMD_SETTLE(m);
   double *part = nullptr;
   SELFAMD_HIP(scratch_address(dev, &part));
   // every block writes its own partial sum, so nothing in the array needs clearing first
@@ -2660,6 +2867,7 @@ int selfamd_model2d_integral(selfamd_model2d *m, int var, double *value) {
 
 int selfamd_model2d_tendency(selfamd_model2d *m, double *dSdt) {
   SELFAMD_REQUIRE(m && dSdt, "model2d_tendency: null argument");
+  SELFAMD_SETTLE(m);
   SELFAMD_HIP(m->launch_stage(1, 0, 0.0, m->cur, dSdt));
   if (m->un[0]) {
     // the evaluation's velocities become the lag state of the next stage
@@ -2673,6 +2881,7 @@ int selfamd_model2d_tendency(selfamd_model2d *m, double *dSdt) {
 
 int selfamd_model2d_flux_registers(selfamd_model2d *m, double *fluxDivergence, double *flux) {
   SELFAMD_REQUIRE(m && fluxDivergence && flux, "model2d_flux_registers: null argument");
+  SELFAMD_SETTLE(m);
   // a tendency evaluation of the current state that keeps the lag state and writes no dSdt
   // register of the caller's (the model's own buffer takes it)
   double *scratch = nullptr;
@@ -2724,6 +2933,7 @@ hipError_t prepare_graphs(selfamd_model2d *m, int nSteps, double dt) {
 int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   SELFAMD_REQUIRE(m && nSteps >= 0 && dt > 0.0, "model2d_forward_step: bad arguments (nSteps=%d dt=%g)", nSteps, dt);
   if (nSteps == 0) return kOk;
+  if (m->refused()) SELFAMD_SETTLE(m);
   ResidentKernel kernel;
   if (m->resident(nSteps, kernel)) {
     hipError_t e = hipSuccess;
@@ -2732,13 +2942,23 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
       e = m->launch_resident(kernel, n, dt);
       if (e == hipSuccess) nSteps -= n;
     }
-    if (nSteps == 0) return kOk;
+    if (nSteps == 0) {
+      // The network may change next, in stream order: its steps are under way, or taken, first.
+      if (m->closure) SELFAMD_SETTLE(m);
+      return kOk;
+    }
     // not accepted by the runtime: step graphs from here on
     (void)hipGetLastError();
     for (auto &blocks : m->residentBlocks)
       for (int &b : blocks) b = 0;
     m->residentNetBlocks = 0;
   }
+  SELFAMD_SETTLE(m);
+  return step_graphs(m, nSteps, dt);
+}
+
+namespace {
+int step_graphs(selfamd_model2d *m, int nSteps, double dt) {
   if (direct_steps(m, nSteps, dt)) {
     SELFAMD_HIP(m->launch_steps(nSteps, dt));
     return kOk;
@@ -2762,11 +2982,11 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   }
   return kOk;
 }
+}  // namespace
 
 int selfamd_model2d_synchronize(selfamd_model2d *m) {
   SELFAMD_REQUIRE(m, "model2d_synchronize: null model");
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
-  return resident_status(m);
+  return wait_for(m);
 }
 
 int selfamd_model2d_stream(selfamd_model2d *m, void **stream) {
@@ -2779,6 +2999,7 @@ int selfamd_model2d_time_steps(selfamd_model2d *m, int nSteps, double dt, double
   SELFAMD_REQUIRE(m && elapsedMs && nSteps >= 0 && dt > 0.0, "model2d_time_steps: bad arguments");
   // graph capture is host work: done before the first event, so the GPU's idle time during it
   // is not timed
+  SELFAMD_SETTLE(m);
   ResidentKernel kernel;
   if (!m->resident(nSteps, kernel)) SELFAMD_HIP(prepare_graphs(m, nSteps, dt));
   hipEvent_t e0, e1;
@@ -2789,17 +3010,24 @@ int selfamd_model2d_time_steps(selfamd_model2d *m, int nSteps, double dt, double
   if (rc) return rc;
   SELFAMD_HIP(hipEventRecord(e1, m->stream));
   SELFAMD_HIP(hipEventSynchronize(e1));
+  if (m->refused()) {  // the steps are taken now
+    SELFAMD_HIP(hipEventRecord(e0, m->stream));
+    if ((rc = wait_for(m))) return rc;
+    SELFAMD_HIP(hipEventRecord(e1, m->stream));
+    SELFAMD_HIP(hipEventSynchronize(e1));
+  }
   float ms = 0.f;
   SELFAMD_HIP(hipEventElapsedTime(&ms, e0, e1));
   *elapsedMs = ms;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  return resident_status(m);
+  return wait_for(m);
 }
 
 int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const float *inMean, const float *inScale,
                                 const float *outMean, const float *outScale) {
   SELFAMD_REQUIRE(m, "model2d_set_closure: null model");
+  SELFAMD_SETTLE(m);
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
   m->drop_graphs();
   free_closure(m->closure);
@@ -2849,6 +3077,7 @@ int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const floa
 int selfamd_model2d_stage(selfamd_model2d *m, int stage, double dt, double *Ssave, double *unSave) {
   SELFAMD_REQUIRE(m && stage >= 0 && stage < 3 && dt > 0.0, "model2d_stage: bad arguments (stage=%d dt=%g)", stage, dt);
   SELFAMD_REQUIRE(m->nBands == 0, "model2d_stage: banded stepping is on");
+  SELFAMD_SETTLE(m);
   const size_t nS = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
   if (Ssave) SELFAMD_HIP(hipMemcpyAsync(Ssave, m->S, sizeof(double) * nS, hipMemcpyDeviceToDevice, m->stream));
   if (unSave) {
@@ -2900,6 +3129,7 @@ int selfamd_model2d_closure_vjp(selfamd_model2d *m, const double *S, const doubl
 int selfamd_model2d_set_bands(selfamd_model2d *m, int nBands) {
   SELFAMD_REQUIRE(m && nBands >= 0, "model2d_set_bands: bad arguments");
   SELFAMD_REQUIRE(nBands == 0 || !m->closure, "model2d_set_bands: banded stepping does not take a closure");
+  SELFAMD_SETTLE(m);
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
   m->drop_graphs();
   if (m->bandElems) (void)hipFree(m->bandElems);
@@ -2977,6 +3207,7 @@ int selfamd_model2d_set_bands(selfamd_model2d *m, int nBands) {
 int selfamd_model2d_closure_features(selfamd_model2d *m, float *X) {
   SELFAMD_REQUIRE(m && X, "model2d_closure_features: null argument");
   SELFAMD_REQUIRE(m->closure, "model2d_closure_features: no closure attached");
+  SELFAMD_SETTLE(m);
   SELFAMD_HIP(closure_features(m->S, m->geom, m->closure->inMean, m->closure->inScale, X, m->N, m->nVar, m->nEl,
                                m->stream));
   SELFAMD_HIP(hipStreamSynchronize(m->stream));
@@ -3308,8 +3539,7 @@ int selfamd_batch_create(selfamd_batch **out, int nModels, selfamd_model2d *cons
     SELFAMD_REQUIRE((m->aux != nullptr) == (m0->aux != nullptr) && (m->stat2 != nullptr) == (m0->stat2 != nullptr) &&
                         (m->presTrace != nullptr) == (m0->presTrace != nullptr),
                     "batch_create: run %d: static fields must be set on all runs or on none", r);
-    SELFAMD_HIP(hipStreamSynchronize(m->stream));
-    if (const int status = resident_status(m)) return status;
+    if (const int status = wait_for(models[r])) return status;
   }
   selfamd_batch *b = new selfamd_batch();
   b->kind = m0->kind;
@@ -3457,6 +3687,7 @@ int selfamd_batch_scatter(selfamd_batch *b) {
   SELFAMD_REQUIRE(b, "batch_scatter: null batch");
   SELFAMD_HIP(hipStreamSynchronize(b->stream));
   // on the default stream, behind any caller's work on a blocking stream of a model
+  for (Model *m : b->models) SELFAMD_HIP(hipStreamSynchronize(m->stream));
   const DeviceScope scope(b->device);
   SELFAMD_REQUIRE(scope.ok, "batch_scatter: the batch's device cannot be made current");
   CopyList list{};
@@ -3488,10 +3719,7 @@ int selfamd_batch_scatter(selfamd_batch *b) {
   }
   SELFAMD_HIP(flush());
   SELFAMD_HIP(hipStreamSynchronize(nullptr));
-  for (Model *m : b->models) {
-    SELFAMD_HIP(hipStreamSynchronize(m->stream));
-    state_replaced(m);
-  }
+  for (Model *m : b->models) state_replaced(m);
   return kOk;
 }
 
