@@ -329,7 +329,9 @@ int selfamd_model2d_integral_noalloc(selfamd_model2d *model, int var, double *va
  * whose blocks have to be on the device together; where other work keeps some of them out, the
  * next call that waits for the model, reads its state or changes what it depends on takes the
  * steps one stage per launch.  Such a call first waits until pending launches are under way; with
- * a closure attached forward_step does so itself. */
+ * a closure attached forward_step does so itself.  Launches of several models run one after another;
+ * where three or more small models step at the same time (none waited for before the others are
+ * asked), stage launches are taken, which overlap.  The results are the same bits either way. */
 int selfamd_model2d_forward_step(selfamd_model2d *model, int nSteps, double dt);
 /* Blocks until the model's stream has drained.  An error if a step launch gave up waiting for
  * another block's traces (SELFAMD_PARAM_POLLS): the state is then not valid, and every call that

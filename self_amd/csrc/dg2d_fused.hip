@@ -22,6 +22,7 @@
 // Geometry: the fast path takes affine elements (metric terms constant per element, true
 // for the structured and block meshes); each element carries one 20-double record.
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <cmath>
@@ -50,6 +51,16 @@ constexpr int kResidentSteps = 2, kResidentElements = 1024;
 // Instances whose registers spill pay for it once per call: from this many steps on (SW N = 3,
 // 18,400 elements: 60 against 49 us for one step, 10.2 against 11.3 us per stage).
 constexpr int kResidentSpillSteps = 5;
+// Resident launches of one process run one after another, where step graphs of several streams
+// overlap.  So while this many other models step at the same time (company_of), meshes of up to
+// kCompanyWaves wavefronts per CU, a stage of which leaves most of the device idle, take graphs.  Steps
+// of K models, all enqueued from one thread before any is waited for, by graphs and by resident launches:
+//   SW 32^2 N = 3 (1 wavefront per CU), 100 steps   K = 2 1,340 and 1,140 us, K = 3 1,480 and 1,800, K = 8 3,220 and 4,690
+//   Euler 16^2 N = 4 (1), 100 steps                 K = 2 2,130 and 1,540, K = 3 2,270 and 2,360, K = 8 4,740 and 6,200
+//   linear SW 20^2 N = 7 (2), 200 steps             K = 2 2,920 and 2,070, K = 3 3,220 and 3,140, K = 8 7,130 and 8,320
+//   Euler 60^2 N = 4 (7), 24 steps                  K = 2 1,020 and 630, K = 3 1,280 and 930, K = 8 3,750 and 2,500
+//   SW 64^2 N = 7 (16), 24 steps                    K = 2 1,050 and 800, K = 3 1,420 and 1,240, K = 8 3,700 and 3,230
+constexpr int kCompany = 2, kCompanyWaves = 4;
 // After a launch that found no place for all its blocks, this many calls take step graphs.
 constexpr int kHeldOffCalls = 64;
 // Longer calls are several resident launches (27 ms each at 10^2 elements of degree 7, against some
@@ -2131,6 +2142,7 @@ struct selfamd_model2d {
   int residentBlocks[2][kResidentDense] = {{-1, -1, -1, -1}, {-1, -1, -1, -1}};  // [nodal][dense]
   bool residentSpills[2][kResidentDense] = {};  // whether those instances' registers spill
   int residentNetBlocks = -1;                   // with a closure
+  int residentCUs = 0;                          // of the device
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
   ResidentGate *gate = nullptr;
   ResidentReport *report = nullptr;
@@ -2138,6 +2150,10 @@ struct selfamd_model2d {
   bool gateReset = false;  // the gate is to be set up before the next launch
   unsigned launches = 0;  // resident launches so far: the last one's number
   int heldOff = 0;        // calls still to take step graphs after a refused launch
+  // other models stepping at the same time (company_of)
+  std::atomic<bool> unwaited{false};  // steps have been enqueued since the stream was last waited for
+  unsigned long long lastCall = 0;
+  int joined = 0;
   // Launches that may yet be refused: `count` alike from launch `first` on, which starts from trace
   // buffer `cur`.
   struct Pending {
@@ -2167,6 +2183,9 @@ struct selfamd_model2d {
   // at once, and the stages saved pay for a cooperative launch.
   // Sets the kernel to launch.
   bool resident(int nSteps, ResidentKernel &k);
+  bool leaves_room(const ResidentKernel &k) const {
+    return (size_t)((nEl + k.elements - 1) / k.elements) * (k.threads / 64) <= (size_t)kCompanyWaves * residentCUs;
+  }
   int mass_stride(const ResidentKernel &k) const { return ((nEl + k.elements - 1) / k.elements + 511) & ~511; }
   hipError_t launch_resident(const ResidentKernel &k, int nSteps, double dt);
 
@@ -2281,6 +2300,48 @@ struct selfamd_model2d {
 
 using Model = selfamd_model2d;
 
+namespace {
+// The models whose meshes fit the device, and their step calls so far, in one order.
+struct SteppingModels {
+  std::mutex mutex;
+  std::vector<Model *> models;
+  unsigned long long calls = 0;
+};
+SteppingModels &stepping_models() {
+  static SteppingModels *const all = new SteppingModels();  // outlives every model
+  return *all;
+}
+// With a step call on m: how many other models of its device step at the same time.  That is those
+// with steps enqueued since m's last call and not yet waited for, or, where m comes first in a round of
+// calls, those that were enqueued like that beside m's last one.
+int company_of(Model *m) {
+  SteppingModels &all = stepping_models();
+  const std::lock_guard<std::mutex> lock(all.mutex);
+  if (m->lastCall == 0) all.models.push_back(m);
+  auto beside = [m](const Model *o) {
+    return o != m && o->device == m->device && o->unwaited && o->lastCall > m->lastCall;
+  };
+  const int others = (int)std::count_if(all.models.begin(), all.models.end(), beside);
+  for (Model *o : all.models)
+    if (beside(o)) o->joined = std::max(o->joined, others);
+  const int company = std::max(others, m->joined);
+  m->joined = 0;
+  m->unwaited = true;
+  m->lastCall = ++all.calls;
+  return company;
+}
+hipError_t drain(Model *m) {
+  const hipError_t e = hipStreamSynchronize(m->stream);
+  if (e == hipSuccess) m->unwaited = false;
+  return e;
+}
+void leave_company(Model *m) {
+  SteppingModels &all = stepping_models();
+  const std::lock_guard<std::mutex> lock(all.mutex);
+  all.models.erase(std::remove(all.models.begin(), all.models.end(), m), all.models.end());
+}
+}  // namespace
+
 bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
   if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || timed_out()) return false;
   if (heldOff > 0) {
@@ -2306,6 +2367,7 @@ bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
         (void)hipGetLastError();
         perCU = 0;
       }
+      residentCUs = cus;
       spills = at.localSizeBytes > 0;
       blocks = coop ? cus * perCU : 0;
       // Euler at N = 2 on a full device: 3,060 blocks 17.1 us per stage, in launches 15.9; 2,600 blocks
@@ -2588,6 +2650,7 @@ int selfamd_model2d_destroy(selfamd_model2d *m) {
                     m->aux,  m->stat2, m->presTrace, m->ndsdx, m->nJ,    m->nnHat, m->nnScale};
   if (m->bandElems) (void)hipFree(m->bandElems);
   if (m->ring) (void)hipFree(m->ring);
+  leave_company(m);
   if (m->gate) (void)hipFree(m->gate);
   if (m->report) (void)hipHostFree(m->report);
   if (m->intScratch) (void)hipFree(m->intScratch);
@@ -2632,13 +2695,13 @@ int take_refused_steps(selfamd_model2d *m) {
     }
   }
   m->t = t;
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return kOk;
 }
 
 // Waits for the model's stream; the steps that were asked for have been taken when it returns.
 int wait_for(selfamd_model2d *m) {
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   if (!m->pending.empty())
     if (const int status = take_refused_steps(m)) return status;
   return resident_status(m);
@@ -2661,7 +2724,7 @@ int settle(selfamd_model2d *m) {
   }
   SELFAMD_REQUIRE(!captured, "model2d: steps before the capture have not been taken; wait for the model before its "
                              "stream is captured");
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return take_refused_steps(m);
 }
 #define SELFAMD_SETTLE(m)                              \
@@ -2699,7 +2762,7 @@ int selfamd_model2d_set_param(selfamd_model2d *m, int which, double value) {
         m->nodal = value != 0.0;
         SELFAMD_HIP(launch_un_init(m->N, m->trace[m->cur], m->un[m->cur], m->geom, m->nodal ? m->nnHat : nullptr,
                                    m->nEl, m->stream));
-        SELFAMD_HIP(hipStreamSynchronize(m->stream));
+        SELFAMD_HIP(drain(m));
       }
       m->nodal = value != 0.0;
       break;
@@ -2730,7 +2793,7 @@ int selfamd_model2d_set_field(selfamd_model2d *m, int which, const double *field
   SELFAMD_SETTLE(m);
   if (!*slot) SELFAMD_HIP(hipMalloc(slot, sizeof(double) * n));
   SELFAMD_HIP(hipMemcpyAsync(*slot, field, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   m->drop_graphs();
   return kOk;
 }
@@ -2749,7 +2812,7 @@ int selfamd_model2d_set_solution(selfamd_model2d *m, const double *interior) {
   const bool direct = from == Source::kKernel;
   if (!direct) SELFAMD_HIP(hipMemcpyAsync(m->S, interior, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
   SELFAMD_HIP(m->launch_state_in(direct ? interior : m->S));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   state_replaced(m);
   return kOk;
 }
@@ -2759,7 +2822,7 @@ int selfamd_model2d_get_solution(selfamd_model2d *m, double *interior) {
   SELFAMD_SETTLE(m);
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
   SELFAMD_HIP(hipMemcpyAsync(interior, m->S, sizeof(double) * n, hipMemcpyDeviceToDevice, m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return resident_status(m);
 }
 
@@ -2795,7 +2858,7 @@ static int model_integral(selfamd_model2d *m, int what, int var, double *value, 
                      m->intScratch + nBlocks);
   SELFAMD_CHECK_LAUNCH();
   SELFAMD_HIP(hipMemcpyAsync(value, m->intScratch + nBlocks, sizeof(double), hipMemcpyDeviceToHost, m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return resident_status(m);
 }
 
@@ -2875,7 +2938,7 @@ int selfamd_model2d_tendency(selfamd_model2d *m, double *dSdt) {
                                sizeof(double) * (m->nodal ? 2 : 1) * (m->N + 1) * 4 * (size_t)m->nEl,
                                hipMemcpyDeviceToDevice, m->stream));
   }
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return resident_status(m);
 }
 
@@ -2888,7 +2951,7 @@ int selfamd_model2d_flux_registers(selfamd_model2d *m, double *fluxDivergence, d
   const size_t n = (size_t)(m->N + 1) * (m->N + 1) * m->nVar * m->nEl;
   SELFAMD_HIP(hipMalloc(&scratch, sizeof(double) * n));
   hipError_t e = m->launch_stage(1, 0, 0.0, m->cur, scratch, -1, flux, fluxDivergence);
-  if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+  if (e == hipSuccess) e = drain(m);
   (void)hipFree(scratch);
   SELFAMD_HIP(e);
   return resident_status(m);
@@ -2935,7 +2998,7 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   if (nSteps == 0) return kOk;
   if (m->refused()) SELFAMD_SETTLE(m);
   ResidentKernel kernel;
-  if (m->resident(nSteps, kernel)) {
+  if (m->resident(nSteps, kernel) && (company_of(m) < kCompany || !m->leaves_room(kernel))) {
     hipError_t e = hipSuccess;
     while (e == hipSuccess && nSteps > 0) {
       const int n = std::min(nSteps, kResidentLaunchSteps);
@@ -3028,7 +3091,7 @@ int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const floa
                                 const float *outMean, const float *outScale) {
   SELFAMD_REQUIRE(m, "model2d_set_closure: null model");
   SELFAMD_SETTLE(m);
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   m->drop_graphs();
   free_closure(m->closure);
   m->closure = nullptr;
@@ -3088,7 +3151,7 @@ int selfamd_model2d_stage(selfamd_model2d *m, int stage, double dt, double *Ssav
   SELFAMD_HIP(m->launch_stage(0, stage, dt, m->cur, nullptr));
   m->cur ^= 1;
   if (stage == 2) m->t += dt;
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return resident_status(m);
 }
 
@@ -3112,7 +3175,7 @@ int selfamd_model2d_tendency_vjp(selfamd_model2d *m, const double *S, const doub
   SELFAMD_HIP(sw_tendency_vjp(m->N, m->nEl, S, m->adjTrace, un, m->aux, m->geom, m->nbr, m->mats, m->p.g, m->p.fCori,
                               m->p.auxConst, lambda, mu, m->adjChi, m->adjTrace + nTr, muPrev, m->adjChi + nTr,
                               m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return kOk;
 }
 
@@ -3122,7 +3185,7 @@ int selfamd_model2d_closure_vjp(selfamd_model2d *m, const double *S, const doubl
   const int P = m->N + 1;
   SELFAMD_HIP(closure_vjp(*m->closure, S, m->geom, m->mats + 2 * P * P + 2 * P, lambda, mu, m->N, m->nVar, 2, m->nEl,
                           m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return kOk;
 }
 
@@ -3130,7 +3193,7 @@ int selfamd_model2d_set_bands(selfamd_model2d *m, int nBands) {
   SELFAMD_REQUIRE(m && nBands >= 0, "model2d_set_bands: bad arguments");
   SELFAMD_REQUIRE(nBands == 0 || !m->closure, "model2d_set_bands: banded stepping does not take a closure");
   SELFAMD_SETTLE(m);
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   m->drop_graphs();
   if (m->bandElems) (void)hipFree(m->bandElems);
   m->bandElems = nullptr;
@@ -3210,7 +3273,7 @@ int selfamd_model2d_closure_features(selfamd_model2d *m, float *X) {
   SELFAMD_SETTLE(m);
   SELFAMD_HIP(closure_features(m->S, m->geom, m->closure->inMean, m->closure->inScale, X, m->N, m->nVar, m->nEl,
                                m->stream));
-  SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  SELFAMD_HIP(drain(m));
   return resident_status(m);
 }
 
@@ -3687,7 +3750,7 @@ int selfamd_batch_scatter(selfamd_batch *b) {
   SELFAMD_REQUIRE(b, "batch_scatter: null batch");
   SELFAMD_HIP(hipStreamSynchronize(b->stream));
   // on the default stream, behind any caller's work on a blocking stream of a model
-  for (Model *m : b->models) SELFAMD_HIP(hipStreamSynchronize(m->stream));
+  for (Model *m : b->models) SELFAMD_HIP(drain(m));
   const DeviceScope scope(b->device);
   SELFAMD_REQUIRE(scope.ok, "batch_scatter: the batch's device cannot be made current");
   CopyList list{};

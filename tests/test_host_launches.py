@@ -83,3 +83,33 @@ def test_networks_of_very_many_rows_have_grids(run):
         lines = log()
         assert lines and all(f"{len(kernel)}{kernel}" in l for l in lines), lines[:3]
     """)
+
+
+def test_small_models_that_step_together_keep_to_graphs(run):
+    run("""
+    def routes(models, wait):
+        \"\"\"How each model's call of a round is launched.\"\"\"
+        out = []
+        for m in models:
+            log()
+            call("selfamd_model2d_forward_step", m._h, 4, 1e-4)
+            lines = [l.split()[0] for l in log()]
+            out.append("R" if "cooperative" in lines else "G" if "graph" in lines else "?")
+            if wait:
+                call("selfamd_model2d_synchronize", m._h)
+        for m in models:
+            call("selfamd_model2d_synchronize", m._h)
+        return "".join(out)
+
+    a, b, c = (model("lsw", 3, 9, 9) for _ in range(3))
+    assert routes([a, b], False) == "RR" and routes([a, b], False) == "RR"  # two: one after the other
+    assert routes([a, b, c], False) == "RRG"                                # a third joins
+    assert routes([a, b, c], False) == "GGG" and routes([a, b, c], False) == "GGG"
+    assert routes([a, b, c], True) == "GGR"                                 # waited for each time from here on
+    assert routes([a, b, c], True) == "RRR"
+    assert routes([a], False) == "R"
+    big = [model("lsw", 3, 66, 66) for _ in range(3)]                       # 1,089 blocks of a wavefront
+    assert routes(big, False) == "RRR" and routes(big, False) == "RRR"
+    del b, c
+    assert routes([a], False) == "R"
+    """)
