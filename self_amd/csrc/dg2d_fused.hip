@@ -60,12 +60,15 @@ constexpr int kResidentSpillSteps = 5;
 //   linear SW 20^2 N = 7 (2), 200 steps             K = 2 2,920 and 2,070, K = 3 3,220 and 3,140, K = 8 7,130 and 8,320
 //   Euler 60^2 N = 4 (7), 24 steps                  K = 2 1,020 and 630, K = 3 1,280 and 930, K = 8 3,750 and 2,500
 //   SW 64^2 N = 7 (16), 24 steps                    K = 2 1,050 and 800, K = 3 1,420 and 1,240, K = 8 3,700 and 3,230
-constexpr int kCompany = 2, kCompanyWaves = 4;
+constexpr int kCompany = 2, kCompanyWaves = 4;  // the latter: leaves_room
 // After a launch that found no place for all its blocks, this many calls take step graphs.
 constexpr int kHeldOffCalls = 64;
-// Longer calls are several resident launches (27 ms each at 10^2 elements of degree 7, against some
-// 10 us for a launch), so that other streams get the device in between.
-constexpr int kResidentLaunchSteps = 4096;
+// Longer calls are several resident launches, so that other streams get the device in between.  A mesh
+// that leaves room for others' wavefronts beside its own does not keep them waiting (a step of a 256^2
+// mesh takes 0.33 ms beside 10^2 elements), and its launches are long ones; a step beside SW 64^2
+// N = 7, which holds every register, waits for the launch to end: 62 ms with 4,096 steps, 6.7 with 512,
+// which cost 0.6 % of the call.
+constexpr int kResidentLaunchSteps = 4096, kResidentFullSteps = 512;
 
 // Williamson low-storage RK3 (src/SELF_Model.f90:25-27)
 constexpr double kRk3A[3] = {0.0, -5.0 / 9.0, -153.0 / 128.0};
@@ -3001,7 +3004,7 @@ int selfamd_model2d_forward_step(selfamd_model2d *m, int nSteps, double dt) {
   if (m->resident(nSteps, kernel) && (company_of(m) < kCompany || !m->leaves_room(kernel))) {
     hipError_t e = hipSuccess;
     while (e == hipSuccess && nSteps > 0) {
-      const int n = std::min(nSteps, kResidentLaunchSteps);
+      const int n = std::min(nSteps, m->leaves_room(kernel) ? kResidentLaunchSteps : kResidentFullSteps);
       e = m->launch_resident(kernel, n, dt);
       if (e == hipSuccess) nSteps -= n;
     }

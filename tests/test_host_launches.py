@@ -113,3 +113,14 @@ def test_small_models_that_step_together_keep_to_graphs(run):
     del b, c
     assert routes([a], False) == "R"
     """)
+
+
+def test_launches_that_fill_the_device_are_short(run):
+    run("""
+    for n, steps, launches in ((9, 4096, 1), (9, 4097, 2), (66, 512, 1), (66, 1025, 3)):
+        m = model("lsw", 3, n, n)
+        log()
+        call("selfamd_model2d_forward_step", m._h, steps, 1e-4)
+        assert sum(l.startswith("cooperative") for l in log()) == launches, (n, steps)
+        call("selfamd_model2d_synchronize", m._h)
+    """)
