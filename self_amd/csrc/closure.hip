@@ -927,6 +927,7 @@ namespace {
 // doubles are padded by one: four of five rows would share banks at Pf = 8.
 constexpr int kProjectArgs = 448, kProjectLds = 6144, kProjectChunk = 3072;  // doubles
 constexpr size_t kProjectBlocks = size_t(1) << 24;  // of 256: a grid's work-items stay below 2^32
+constexpr size_t kProjectFew = 4000, kProjectProducts = 1300;
 struct ProjectArgs {
   const double *fine;
   double *coarse;
@@ -1012,7 +1013,8 @@ __global__ void __launch_bounds__(256) k_project(const ProjectArgs a) {
 }
 
 // The same, one work-item per coarse value, for coarsening factors and degrees whose factors or
-// runs are too long for the kernel arguments or LDS of k_project, and for meshes beyond its grid.
+// runs are too long for the kernel arguments or LDS of k_project, for meshes beyond its grid, and for
+// large meshes of small elements.
 __global__ void k_project_values(const double *__restrict__ Sf, double *__restrict__ Sc, const double *__restrict__ Px,
                                  int Nf, int Nc, int nxc, int nyc, int r, int nVar) {
   const int Pf = Nf + 1, Pc = Nc + 1;
@@ -1312,7 +1314,14 @@ int selfamd_project_l2_structured_2d(const double *fine, double *coarse, int Nf,
   };
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const size_t elements = (size_t)nxc * nyc;
-  if (nPx <= (size_t)kProjectArgs && run <= (size_t)kProjectLds && elements < kProjectBlocks) {
+  // A block per coarse element takes 1.45 ns from some thousand elements on, whatever is in it, and a
+  // product of a coarse value and a fine one 1.1e-3 ns by the value-by-value kernel, half of that at
+  // Pf = 2.  By values and by blocks: 547^2 elements, r = 2, Pf = Pc = 3, one variable (324 products
+  // each) 116 and 417 us; 252^2, r = 2, Pf = Pc = 4, three variables (3,072) 197 and 125 us.
+  const size_t products = (size_t)Pc * Pc * nVar * r * r * Pf * Pf;
+  const size_t cheap = Pf == 2 ? 2 : 1;
+  const bool blocksPay = elements <= kProjectFew / cheap || products >= kProjectProducts * cheap;
+  if (nPx <= (size_t)kProjectArgs && run <= (size_t)kProjectLds && elements < kProjectBlocks && blocksPay) {
     ProjectArgs g;
     g.fine = fine; g.coarse = coarse; g.Pf = Pf; g.Pc = Pc; g.nxc = nxc; g.r = r; g.nVar = nVar;
     g.rowsB = std::max(1, std::min(r, kProjectChunk / (int)run));

@@ -66,9 +66,21 @@ def test_projection_grids_stay_within_the_runtime_limit(run):
     run("""
     a = self_amd.DeviceArray((8,))
     for nyc, kernel in ((4095, "k_project"), (4096, "k_project_values"), (4097, "k_project_values")):
-        call("selfamd_project_l2_structured_2d", a.ptr, a.ptr, 1, 1, 4096, nyc, 1, 1, None)
+        call("selfamd_project_l2_structured_2d", a.ptr, a.ptr, 7, 3, 4096, nyc, 1, 3, None)
         lines = log()
         assert len(lines) == 1 and f"{len(kernel)}{kernel}" in lines[0], lines  # as mangled
+    """)
+
+
+def test_projection_of_many_small_elements_goes_by_values(run):
+    run("""
+    a = self_amd.DeviceArray((8,))
+    for Nf, Nc, r, nv, n, kernel in ((1, 1, 1, 3, 512, "k_project_values"), (2, 2, 2, 1, 512, "k_project_values"),
+                                     (2, 2, 2, 1, 60, "k_project"), (3, 3, 2, 3, 512, "k_project"),
+                                     (1, 1, 4, 3, 512, "k_project_values"), (7, 3, 4, 3, 64, "k_project")):
+        call("selfamd_project_l2_structured_2d", a.ptr, a.ptr, Nf, Nc, n, n, r, nv, None)
+        lines = log()
+        assert len(lines) == 1 and f"{len(kernel)}{kernel}" in lines[0], (Nf, Nc, r, nv, n, lines)
     """)
 
 
