@@ -3354,8 +3354,10 @@ struct BatchGroup {
 namespace {
 // Device-to-device copies of many arrays in one launch, the list in the kernel arguments: a copy
 // call each costs 3 us whatever its size (48 runs of 8^2 to 64^2 elements, four arrays each: 567 us
-// in 192 calls, 70 us in two launches).  blockIdx.y is the array, kCopyBlocks blocks stride through it.
+// in 192 calls, 70 us in two launches).  blockIdx.y is the item, kCopyBlocks blocks stride through it;
+// long arrays are several items of kCopyDoubles, so that the blocks grow with the data.
 constexpr int kCopyItems = 160, kCopyBlocks = 48;
+constexpr size_t kCopyDoubles = size_t(1) << 18;
 struct CopyList {
   struct Item {
     const double *src;
@@ -3778,8 +3780,10 @@ int selfamd_batch_scatter(selfamd_batch *b) {
           SELFAMD_HIP(hipMemcpy(it.dst, it.src, 8 * it.n, hipMemcpyDeviceToDevice));
           continue;
         }
-        if (list.count == kCopyItems) SELFAMD_HIP(flush());
-        list.item[list.count++] = it;
+        for (size_t at = 0; at < it.n; at += kCopyDoubles) {
+          if (list.count == kCopyItems) SELFAMD_HIP(flush());
+          list.item[list.count++] = {it.src + at, it.dst + at, std::min(kCopyDoubles, it.n - at)};
+        }
       }
     }
   }
