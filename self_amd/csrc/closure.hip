@@ -665,10 +665,19 @@ hipError_t weight_grads_rows(selfamd_mlp *m, const float *X, const float *dY, in
   return hipGetLastError();
 }
 
+// Whether the forward pass of a row network goes layer by layer.  A block of the row kernel has 512
+// work-items and 64 reduction indices a piece for its 16 rows, however narrow the network, and pays by
+// the launches it saves; on many rows a narrow network's layers are the cheaper ones.  Layers and the row
+// kernel, us (in, hidden, out): 1, 1, 1 on 16,384 rows 15 and 10, on 32,768 14 and 18, on 131,072 22 and
+// 62; 16, 16, 16 on 32,768 24 and 19, on 65,536 30 and 35, on 400,000 128 and 189; 40, 48, 40 on 400,000
+// 259 and 224.  The line follows where they cross over hidden widths 1 to 48 and inputs 1 to 120.
+inline bool narrow_by_layers(int nIn, int nH, int B) {
+  return nH <= 40 && B >= 24576 + 1280 * nH + 256 * std::min(nIn, 1024);
+}
 // Y = net(X); Y may lie over X.
 hipError_t forward_impl(selfamd_mlp *m, const float *X, float *Y, int B, hipStream_t st) {
   hipError_t e;
-  if (m->rows) {
+  if (m->rows && !narrow_by_layers(m->nIn, m->nH, B)) {
     // a block writes its rows of Y while others still read theirs of X
     const size_t nY = sizeof(float) * (size_t)B * m->nOut;
     const bool over = ranges_overlap(Y, nY, X, sizeof(float) * (size_t)B * m->nIn);
@@ -677,8 +686,9 @@ hipError_t forward_impl(selfamd_mlp *m, const float *X, float *Y, int B, hipStre
     if ((e = launch_rows<kRowsForward>(a, st)) || !over) return e;
     return hipMemcpyAsync(Y, m->Y, nY, hipMemcpyDeviceToDevice, st);
   }
-  if ((e = gemm<false, false, 2>(X, m->W1(), m->H1, m->Z1, m->b1(), B, m->nH, m->nIn, m->nIn, m->nH, 1, st))) return e;
-  if ((e = gemm<false, false, 2>(m->H1, m->W2(), m->H2, m->Z2, m->b2(), B, m->nH, m->nH, m->nH, m->nH, 1, st))) return e;
+  float *Z1 = m->rows ? m->D1 : m->Z1, *Z2 = m->rows ? m->D2 : m->Z2;  // no backward pass reads a row network's
+  if ((e = gemm<false, false, 2>(X, m->W1(), m->H1, Z1, m->b1(), B, m->nH, m->nIn, m->nIn, m->nH, 1, st))) return e;
+  if ((e = gemm<false, false, 2>(m->H1, m->W2(), m->H2, Z2, m->b2(), B, m->nH, m->nH, m->nH, m->nH, 1, st))) return e;
   return gemm<false, false, 1>(m->H2, m->W3(), Y, nullptr, m->b3(), B, m->nOut, m->nH, m->nH, m->nOut, 1, st);
 }
 

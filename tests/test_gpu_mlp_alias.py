@@ -69,3 +69,28 @@ def test_forward_over_its_input(nIn, nH, nOut, rows, shift):
     self_amd.call("selfamd_mlp_forward", net._h, _at(mem, 0), _at(mem, shift), rows, None)
     got = mem.to_host()[shift:shift + want.size].reshape(want.shape)
     assert (got == want).all()
+
+
+# narrow networks on both sides of the line from which the forward pass goes layer by layer
+@pytest.mark.parametrize("nIn,nH,nOut,rows", [(3, 2, 4, 27903), (3, 2, 4, 27904), (17, 40, 5, 80128), (17, 40, 5, 80127)])
+def test_narrow_networks_on_many_rows(nIn, nH, nOut, rows):
+    import self_amd
+    net = _net(nIn, nH, nOut, rows)
+    rng = np.random.default_rng(rows)
+    X = rng.standard_normal((rows, nIn)).astype(np.float32)
+    p = {k: v.astype(np.float32).astype(np.float64) for k, v in om.init_params(nIn, nH, nOut, seed=3).items()}
+    want, _ = om.forward(p, X.astype(np.float64))
+    Xd = self_amd.DeviceArray.from_host(X)
+    before = net.backward(Xd, want.astype(np.float32), want_dX=False), net.get_grads()
+    got = net.forward(Xd)
+    assert np.max(np.abs(got - want)) <= 4 * U * (nIn + 2 * nH + 16) * np.max(np.abs(want))
+    # in place, and a backward pass after it
+    mem = self_amd.DeviceArray((rows * max(nIn, nOut),), np.float32, zero=True)
+    host = np.zeros(mem.shape, np.float32)
+    host[:X.size] = X.ravel()
+    mem.copy_from_host(host)
+    self_amd.call("selfamd_mlp_forward", net._h, _at(mem, 0), _at(mem, 0), rows, None)
+    assert (mem.to_host()[:want.size].reshape(want.shape) == got).all()
+    net.backward(Xd, want.astype(np.float32), want_dX=False)
+    after = net.get_grads()
+    assert all((after[k] == before[1][k]).all() for k in after)
