@@ -3119,12 +3119,13 @@ int selfamd_model2d_set_closure(selfamd_model2d *m, selfamd_mlp *mlp, const floa
   ClosureBuffers *c = new ClosureBuffers();
   c->mlp = mlp; c->nIn = nIn; c->nOut = nOut; c->invArea = 1.0 / area;
   const size_t nEl = m->nEl;
-  bool ok = hipMalloc(&c->X, 4 * nEl * nIn) == hipSuccess && hipMalloc(&c->Y, 4 * nEl * nOut) == hipSuccess &&
+  const bool layers = !mlp_weights(mlp).rows;  // the row kernels keep outputs and input cotangents to themselves
+  bool ok = hipMalloc(&c->X, 4 * nEl * nIn) == hipSuccess && (!layers || hipMalloc(&c->Y, 4 * nEl * nOut) == hipSuccess) &&
             hipMalloc(&c->inMean, 4 * nIn) == hipSuccess && hipMalloc(&c->inScale, 4 * nIn) == hipSuccess &&
             hipMalloc(&c->outMean, 4 * nOut) == hipSuccess && hipMalloc(&c->outScale, 4 * nOut) == hipSuccess &&
             hipMalloc(&c->corr, 8 * nEl * nOut) == hipSuccess && hipMalloc(&c->elemMass, 8 * nEl) == hipSuccess &&
             hipMalloc(&c->shift, 8) == hipSuccess && hipMalloc(&c->dY, 4 * nEl * nOut) == hipSuccess &&
-            hipMalloc(&c->dX, 4 * nEl * nIn) == hipSuccess &&
+            (!layers || hipMalloc(&c->dX, 4 * nEl * nIn) == hipSuccess) &&
             hipMalloc(&c->vjpPartial, 8 * closure_vjp_partials(m->N, m->nEl)) == hipSuccess;
   ok = ok && hipMemcpy(c->inMean, inMean, 4 * nIn, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(c->inScale, inScale, 4 * nIn, hipMemcpyHostToDevice) == hipSuccess &&
