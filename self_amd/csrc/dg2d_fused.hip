@@ -2040,11 +2040,14 @@ template <class Phys, int N, bool NODAL>
 ResidentKernel resident_instance(int dense) {
   using L = ResidentTile<Phys, N, NODAL>;
   constexpr bool FIVE = Phys::NV == 3 && (N >= 3 || (N == 2 && !Phys::kLag));
+  constexpr bool FOUR = Phys::NV == 3 || !(N == 2 || N == 3 || N == 5);  // LDS of these Euler tiles: 3 at most
   const void *fn = nullptr;
   switch (dense) {
     case 0: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 1>); break;
     case 1: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 3>); break;
-    case 2: fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 4>); break;
+    case 2:
+      if constexpr (FOUR) fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 4>);
+      break;
     case 3:
       if constexpr (FIVE) fn = reinterpret_cast<const void *>(&k_resident<Phys, N, NODAL, 5>);
   }
