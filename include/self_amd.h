@@ -316,7 +316,7 @@ int selfamd_model2d_entropy(selfamd_model2d *model, double *entropy);
 int selfamd_model2d_integral(selfamd_model2d *model, int var, double *value);
 /* selfamd_model2d_integral without any allocation: the same kernels and the same result, bit
  * for bit, written to *value_dev (device memory) on the model's stream, without
- * synchronising.  No counterpart in the reference: for callers that cannot allocate device
+ * synchronising (right after selfamd_model2d_forward_step: once its launch is under way).  No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  The partial sums live in a 512 KiB device array of the library, one per GPU,
  * kept until the process ends; meshes of more than 16,777,216 nodes ((N+1)^2 nEl) are

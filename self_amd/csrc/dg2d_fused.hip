@@ -46,7 +46,9 @@ constexpr int kNbrOrphan = -0x40000000;
 constexpr int kDirectSteps = 2;
 // Calls of at least kResidentSteps steps take a resident launch where the mesh allows it, single
 // steps from kResidentElements elements on: below, a cooperative launch of three stages costs what
-// it saves (N = 7: 28.8 against 28.3 us per call at 10^2 elements, 31.9 against 34.1 at 40^2).
+// it saves (N = 7: 28.8 against 28.3 us per call at 10^2 elements before the gate, which adds 2 to 3;
+// 34.6 against 36.2 at 40^2.  On 17 meshes of all physics from 1,024 to 14,400 elements no call of 1 to
+// 8 steps is slower than by graphs).
 constexpr int kResidentSteps = 2, kResidentElements = 1024;
 // Instances whose registers spill pay for it once per call: from this many steps on (SW N = 3,
 // 18,400 elements: 60 against 49 us for one step, 10.2 against 11.3 us per stage).
@@ -1049,8 +1051,8 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 //              conditions, Riemann flux -> LDS; node lanes: divergence, update; face lanes: traces
 //              of the new state -> registers and the exchange ring.
 // The arithmetic and its order are the stage kernel's, so the results are the same bits.
-// Measured per stage (200-step and 24-step calls): linear SW 10^2 N = 7 4.1 -> 2.2 us, 45 x 37 N = 6
-// 8.6 -> 3.0 us, Euler 93 x 61 N = 4 19 -> 7 us.  Instances: WPE = 1 leaves the registers to the
+// Measured per stage (200-, 40- and 20-step calls): linear SW 10^2 N = 7 4.0 -> 1.7 us, 45 x 37 N = 6
+// 8.0 -> 2.8 us, Euler 93 x 61 N = 4 15.3 -> 7.3 us.  Instances: WPE = 1 leaves the registers to the
 // compiler and unrolls the divergence; where the mesh needs more blocks than fit that way, 3, 4 or 5
 // wavefronts per SIMD (twice the elements and more).
 //
@@ -1070,7 +1072,7 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const PersistentArgs b
 // units 80 of them; 1 block per CU), so a stage reads nothing from memory but traces and the other
 // blocks' mass integrals, which every block sends to all others right after the network and needs
 // only at the update.  64 x 64 elements, N = 3, 51 -> 128 -> 128 -> 48, per stage: 16.2 us in two
-// launches (network 8.1 us of them), 6.7 us here: network 3.9, face and volume work 2.5.  With the
+// launches (network 8.1 us of them), 6.6 us here: network 3.9, face and volume work 2.5.  With the
 // integrals in one copy that all blocks poll, sent after the face phase, the wait for them alone was
 // 3.3 us (9.5 us per stage).  A call of one step takes 78 us with set and get, 110 in launches.
 //
