@@ -91,9 +91,9 @@ def test_networks_of_very_many_rows_have_grids(run):
         a = self_amd.DeviceArray((rows, 1), np.float32)
         b = self_amd.DeviceArray((rows, 1), np.float32)
         log()
-        call("selfamd_mlp_forward", net._h, a.ptr, b.ptr, rows, None)
+        call("selfamd_mlp_loss_grad", net._h, a.ptr, b.ptr, rows, None, None)
         lines = log()
-        assert lines and all(f"{len(kernel)}{kernel}" in l for l in lines), lines[:3]
+        assert lines and f"{len(kernel)}{kernel}" in lines[0], lines[:3]
     """)
 
 
