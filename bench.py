@@ -312,6 +312,8 @@ def run_single(a, root):
         cpu = cpu_single(oracle, a.workload, w, steps_all, steps_one)
     phys, kind = {"sw256": ("PhysSW", 2), "euler512": ("PhysEuler", 3), "lsw10": ("PhysLSW", 1)}[a.workload]
     kernel = tile_name(self_amd, N, phys, kind)
+    if a.workload == "lsw10":
+        kernel = "k_resident: all stages of a call in one launch (times per launch are per stage)"
     if a.nodal_metrics:
         t = {7: 64, 6: 64, 5: 128, 4: 128}.get(N, 256)
         kernel = f"k_fused<{phys}, {N}, 0, true, {t}, 1, false>"

@@ -272,6 +272,9 @@ typedef struct selfamd_model2d selfamd_model2d;
                                   blocks have found a place on the device before the launch is
                                   given up and its steps are taken one stage per launch (default
                                   4096, some milliseconds; 0: always given up) */
+#define SELFAMD_PARAM_STAGE_LAUNCHES 8  /* 1: forward_step always takes one stage per launch
+                                  (default 0: all stages of a call in one launch where the mesh
+                                  allows it; the same bits) */
 /* static per-node fields (selfamd_model2d_set_field), interior(0:N,0:N,1,nEl) device arrays */
 #define SELFAMD_FIELD_TOPOGRAPHY 1  /* SW this%H (SetTopography) */
 #define SELFAMD_FIELD_BATHYMETRY 2  /* LSW this%H (SetBathymetry) */

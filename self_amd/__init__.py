@@ -22,7 +22,8 @@ from ._lib import SelfAmdError, call, load
 GAUSS, GAUSS_LOBATTO, UNIFORM = 1, 2, 5
 BC_PRESCRIBED, BC_RADIATION, BC_NONORMALFLOW = 100, 101, 102
 MODEL_LSW, MODEL_SW, MODEL_EULER = 1, 2, 3
-PARAM_G, PARAM_FCORI, PARAM_GAMMA, PARAM_RGAS, PARAM_NODAL_METRICS, PARAM_POLLS, PARAM_GATE_POLLS = 1, 2, 3, 4, 5, 6, 7
+PARAM_G, PARAM_FCORI, PARAM_GAMMA, PARAM_RGAS, PARAM_NODAL_METRICS = 1, 2, 3, 4, 5
+PARAM_POLLS, PARAM_GATE_POLLS, PARAM_STAGE_LAUNCHES = 6, 7, 8
 FIELD_TOPOGRAPHY, FIELD_BATHYMETRY, FIELD_CORIOLIS, FIELD_POTENTIAL, FIELD_DRAG = 1, 2, 3, 4, 5
 
 __all__ = ["DeviceArray", "device_count", "device_name", "synchronize", "Lagrange", "Mesh2D", "SEMQuad",
@@ -323,6 +324,11 @@ class Model2D:
         """Use per-node metric terms (the reference's representation; required on curved
         meshes) instead of one affine record per element."""
         self._param(PARAM_NODAL_METRICS, 1.0 if on else 0.0)
+
+    def SetStageLaunches(self, on=True):
+        """Take one RK stage per launch (step graphs) also where the mesh allows all stages of a
+        call in one launch.  The results are the same bits."""
+        self._param(PARAM_STAGE_LAUNCHES, 1.0 if on else 0.0)
 
     def SetSolution(self, interior):
         """SetSolution (src/SELF_Model2D.f90:313-332) from interior[e, v, j, i] (numpy or DeviceArray)."""

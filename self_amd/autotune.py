@@ -91,7 +91,12 @@ def _model(kind, N, nx):
 def tune(N, nx, kind=MODEL_SW, steps=10, warmup=3, repeats=3, log=None):
     """Time every variant (and the default tile, -1) of the stage kernel of `kind` on an
     nx x nx mesh at degree N; returns {"best": v, "timings": {v: us per launch}}."""
-    make, dt = _model(kind, N, nx)
+    factory, dt = _model(kind, N, nx)
+
+    def make():
+        m = factory()
+        m.SetStageLaunches()  # the tiles are the stage kernel's: small meshes would not launch it
+        return m
     before = get_tile(N, kind)
     timings, ref = {}, None
     # bring the GPU to its steady clock first (the first ~100 steps run slower), so that the

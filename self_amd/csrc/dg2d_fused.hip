@@ -2152,6 +2152,7 @@ struct selfamd_model2d {
   int residentNetBlocks = -1;                   // with a closure
   int residentCUs = 0;                          // of the device
   bool paired = false;  // every interior side's neighbour names that side as its own neighbour
+  bool stageLaunches = false;  // asked for by the caller
   ResidentGate *gate = nullptr;
   ResidentReport *report = nullptr;
   int polls = kPolls, gatePolls = kGatePolls;
@@ -2351,7 +2352,7 @@ void leave_company(Model *m) {
 }  // namespace
 
 bool selfamd_model2d::resident(int nSteps, ResidentKernel &k) {
-  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || timed_out()) return false;
+  if (nSteps < (nEl < kResidentElements ? kResidentSteps : 1) || nBands > 0 || !paired || stageLaunches || timed_out()) return false;
   if (heldOff > 0) {
     heldOff--;
     return false;
@@ -2780,6 +2781,7 @@ int selfamd_model2d_set_param(selfamd_model2d *m, int which, double value) {
       (which == SELFAMD_PARAM_POLLS ? m->polls : m->gatePolls) = (int)value;
       m->gateReset = m->gate != nullptr;
       return kOk;
+    case SELFAMD_PARAM_STAGE_LAUNCHES: m->stageLaunches = value != 0.0; return kOk;
     default: SELFAMD_REQUIRE(false, "model2d_set_param: unknown parameter %d", which);
   }
   m->drop_graphs();

@@ -136,3 +136,22 @@ def test_launches_that_fill_the_device_are_short(run):
         assert sum(l.startswith("cooperative") for l in log()) == launches, (n, steps)
         call("selfamd_model2d_synchronize", m._h)
     """)
+
+
+def test_tiles_of_small_meshes_are_tuned_on_stage_launches(run):
+    run("""
+    from self_amd import autotune
+    m = model("sw", 7, 8, 8)
+    type(m).solution = property(lambda self: np.ones(self.shape))  # no kernel has stored one
+    autotune._model = lambda kind, N, nx: ((lambda: model("sw", 7, 8, 8)), 1e-4)
+    m.ForwardStep(4, 1e-4)
+    assert any(l.startswith("cooperative") for l in log())
+    autotune.tune(7, 8, steps=4, warmup=3, repeats=2)
+    assert not any(l.startswith("cooperative") for l in log())
+    m.SetStageLaunches()
+    m.ForwardStep(4, 1e-4)
+    assert not any(l.startswith("cooperative") for l in log())
+    m.SetStageLaunches(False)
+    m.ForwardStep(4, 1e-4)
+    assert any(l.startswith("cooperative") for l in log())
+    """)
