@@ -90,6 +90,7 @@ def traffic_probe(self_amd, model, dt):
     self_amd.synchronize()
     del a, b
     print("probe: 2 RK3 steps", flush=True)
+    model.SetStageLaunches()
     model.ForwardStep(2, dt)
     self_amd.synchronize()
     print("probe: done", flush=True)
